@@ -30,31 +30,11 @@ namespace splat {
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-constexpr int kAcc = 16;       // per-splat accumulator stride of the exact path (floats)
 constexpr int kPairRecMax = 10;   // per-pair sums record, at most (floats): Q, Qu, Qv, Quu, Qvv, Quv, colour[C]
 template <int C>
 __host__ __device__ constexpr int pair_rec() { return 6 + C; }   // record stride of C channels
-constexpr int kSums = 10;      // sums carried through the reduction
 
 __host__ __device__ constexpr int tile_threads(int tile) { return tile * tile > 64 ? tile * tile : 64; }
-
-// One pixel-pair of the forward: accumulates the colour weight and its colour sums, returns 1 - a for the
-// caller's transmittance product. op * falloff = exp2(log2(op) - m) with m = u^2 + v^2.
-template <int C, bool ODDS>
-__device__ __forceinline__ float fwd_pair(const float* __restrict__ r, float py, float px, float& s_a, float* sc) {
-  const float dy = py - r[R_GY], dx = px - r[R_GX];
-  const float u = fmaf(r[R_A], dy, r[R_B] * dx);
-  const float v = fmaf(r[R_CC], dy, r[R_D] * dx);
-  const float fo = hw_exp2(-fmaf(u, u, fmaf(v, v, -r[R_LOP])));
-  const float a = fminf(fo, kClamp);
-  float oma = 1.f - a;
-  if (ODDS) oma = one_minus_alpha(oma, fo, fmaf(u, u, v * v), r[R_OP], 1.f - r[R_OP]);
-  const float w = ODDS ? a * hw_rcp(oma) : a;
-  s_a += w;
-#pragma unroll
-  for (int c = 0; c < C; ++c) sc[c] = fmaf(w, r[R_COL + c], sc[c]);
-  return oma;
-}
 
 // Opacity bound (as float bits; opacities are non-negative, and any other bit pattern compares above it) at or
 // below which op * falloff = exp2(log2(op) - m), m >= 0, stays below 0.99988 plus a few ulps, under the alpha
@@ -474,23 +454,6 @@ __global__ __launch_bounds__(tile_threads(TILE)) void k_fields_combine(LevelTabl
   for (int c = 0; c < C; ++c) sac[pp * C + c] = sc[c];
 }
 
-// Exact path forward (render_triton.py:58-125): 64 pixels per workgroup in flat pixel order, pixel centres
-// supplied by the caller (render.py:61-65 linspace), every splat in splat order.
-template <int C>
-__global__ __launch_bounds__(64) void k_fwd_exact(const float* __restrict__ rec, int N, const float* __restrict__ pyv,
-                                                  const float* __restrict__ pxv, int P, const float* __restrict__ bg,
-                                                  float* __restrict__ out, float* __restrict__ Tout,
-                                                  float* __restrict__ asum_out, float* __restrict__ fg_out) {
-  const int p = blockIdx.x * 64 + threadIdx.x;
-  const bool valid = p < P;
-  const float py = valid ? pyv[p] : 0.f, px = valid ? pxv[p] : 0.f;
-  float sl = 0.f, s_a = 0.f, sc[C];
-#pragma unroll
-  for (int c = 0; c < C; ++c) sc[c] = 0.f;
-  for (int g = 0; g < N; ++g) sl += hw_log2(fwd_pair<C, false>(rec + (size_t)g * kRec, py, px, s_a, sc));
-  if (valid) store_composite<C>(p, sl, s_a, sc, bg, out, Tout, asum_out, fg_out);
-}
-
 // Per-pixel upstream terms of the backward (render_triton.py:640-654). Masked pixels give zeros.
 // FIELDS: loaded from the packed fields at slot pp. Composite: derived from T, asum, fg, gout and bg; with
 // UPS, `asum` holds the unclamped S_a and dS_a follows torch's clamp_min gradient (0 below 1e-8,
@@ -625,19 +588,6 @@ __device__ __forceinline__ void bwd_px_near(float u, float v, float m, float f, 
     }
   }
   bwd_acc<C, ODDS>(u, v, f, oma, col, pa, pb, s);
-}
-
-// One pixel-pair of the backward, given whitened offsets u, v, with its own wave-uniform choice between the
-// one-fma 1 - a and bwd_px_near (every lane of the wave must be executing).
-template <int C, bool ODDS>
-__device__ __forceinline__ void bwd_px(float u, float v, const PairOp& po, const float4& col, const float4& pa,
-                                       const float2& pb, PairSums<C>& s) {
-  const float m = fmaf(u, u, v * v);
-  const float f = hw_exp2(-m);
-  if (__any(f > po.thr))
-    bwd_px_near<C, ODDS>(u, v, m, f, po, col, pa, pb, s);
-  else
-    bwd_acc<C, ODDS>(u, v, f, fmaf(-po.op, f, 1.f), col, pa, pb, s);
 }
 
 template <int C>
@@ -1397,107 +1347,568 @@ __global__ __launch_bounds__(256) void k_zero_grads(int N, float* __restrict__ g
   if (g < N) zero_grads<C>(g, g_mu, g_scale, g_theta, g_op, g_col);
 }
 
-// Exact path backward (render_triton.py:161-266): lane = splat over every pixel; the per-pixel upstream
-// terms of each 64-pixel chunk are staged in LDS. Each splat is owned by one lane: plain stores.
-template <int C>
-__global__ __launch_bounds__(64) void k_bwd_exact(const float* __restrict__ rec, int N, const float* __restrict__ pyv,
-                                                  const float* __restrict__ pxv, int P, const float* __restrict__ bg,
-                                                  const float* __restrict__ Tin, const float* __restrict__ asum_in,
-                                                  const float* __restrict__ fg_in, const float* __restrict__ gout,
-                                                  float* __restrict__ acc) {
-  __shared__ float4 s_pa[64];
-  __shared__ float2 s_pb[64], s_pyx[64];
-  const int lane = threadIdx.x;
-  const int g = blockIdx.x * 64 + lane;
-  const int gs = g < N ? g : N - 1;
-  const float4* r4 = reinterpret_cast<const float4*>(rec) + (size_t)gs * 4;
-  const float4 r0 = r4[0], r1 = r4[1], col = r4[2];
-  const float gy = r0.x, gx = r0.y, A = r0.z, B = r0.w, Cc = r1.x, D = r1.y;
-  const PairOp po = pair_op(r1.z);
-  PairSums<C> s;
-  float bgp[kMaxC] = {0.f, 0.f, 0.f, 0.f};
-  for (int p0 = 0; p0 < P; p0 += 64) {
-    const int p = p0 + lane;
-    float4 pa = make_float4(0.f, 0.f, 0.f, 0.f);
-    float2 pb = make_float2(0.f, 0.f), pyx = pb;
-    if (p < P) {
-      pixel_upstream<C, false, false>(p, 0, bg, Tin, asum_in, fg_in, gout, nullptr, nullptr, nullptr, pa, pb, bgp);
-      pyx = make_float2(pyv[p], pxv[p]);
-    }
-    __syncthreads();
-    s_pa[lane] = pa;
-    s_pb[lane] = pb;
-    s_pyx[lane] = pyx;
-    __syncthreads();
-    const int np = P - p0 < 64 ? P - p0 : 64;
-    for (int j = 0; j < np; ++j) {
-      const float2 q = s_pyx[j];
-      const float dy = q.x - gy, dx = q.y - gx;
-      bwd_px<C, false>(fmaf(A, dy, B * dx), fmaf(Cc, dy, D * dx), po, col, s_pa[j],
-                               C > 2 ? s_pb[j] : make_float2(0.f, 0.f), s);
-    }
+// ------------------------------------------------------------------------------------------------ exact path
+// Every splat at every pixel (render_triton.py:58-266), O(P + N) memory: nothing of size P x N is stored.
+//
+// Pixels come in groups of 64 (the 8 x 8 tiles of a grid of at least 8 x 8 pixels, else 64 consecutive pixels of the
+// list) or, in the forward of larger problems, of 256 (16 x 16 tiles); splats in batches of 64 consecutive ones. The
+// falloff of a splat is exactly zero in float32 past u^2 + v^2 = 126 (v_exp_f32 flushes results below 2^-126), about
+// 13.2 sigma: there a = 0, 1 - a = 1 and every term of the forward and the backward is an exact zero. The decode pass
+// stores each splat's reach, the box outside which this holds (splat_reach; everything for a splat whose own values are
+// not finite, so that they still spread), and the union of every batch's; the kernels leave out the batches and the
+// splats whose box misses a pixel group's, then the splats that splat_meets rules out. Without `reach` nothing is left
+// out. A list in no order would leave every group as large as the canvas: splat_exact_order sorts it by cells first.
+//
+// Work split: P / 64 pixel groups in the forward and N / 64 splat batches in the backward are far too few waves for the
+// card at most sizes (64 waves for a 64 x 64 forward, 256 for 16,384 splats' backward, against 1,024 SIMDs that want
+// several each), so the other dimension is split as well, into interleaved shares whose partial sums are added in a
+// fixed order (deterministic); exact_fwd_plan and exact_bwd_split have the rules.
+// Measured (MI355X) against one wave per 64 pixels (64 splats) over all splats (pixels): 512 x 512 with 16,384 splats of
+// 4 pixels forward 4,563 -> 141 us, backward 39,994 -> 425 us; 64 x 64 with 1,024 splats forward 266 -> 15 us, backward
+// 628 -> 27 us (all launches); 10,000 random pixels of 768 x 768 with 92,160 splats 22,960 -> 129 and 1,744 -> 149 us. The
+// VALU is busy 61% of the backward's cycles and 46% of the forward's; the rest is the latency of lists and gathers.
+struct ExactPixels {
+  int P, W, H;      // W > 0: a grid of H rows of W pixels, centre (py[y], px[x]); W = 0: a list of P centres
+  int ntx, groups;  // ntx > 0: the groups are the grid's tiles, ntx per row
+  const int* perm;  // a list's order (slot -> pixel), or null
+};
+
+// Pixel of slot (row, column) of tile `group`, or of slot `i` of list group `group` of `size`: its index (-1: no pixel).
+template <int TW>
+__device__ __forceinline__ int exact_tile_pixel(const ExactPixels& G, int group, int row, int column) {
+  const int ty = group / G.ntx, tx = group - ty * G.ntx;
+  const int y = ty * TW + row, x = tx * TW + column;
+  return y < G.H && x < G.W ? y * G.W + x : -1;
+}
+__device__ __forceinline__ int exact_list_pixel(const ExactPixels& G, int slot) {
+  return slot < G.P ? (G.perm ? G.perm[slot] : slot) : -1;
+}
+// Centre of pixel p (p < 0: of pixel `first` instead).
+__device__ __forceinline__ void exact_centre(const ExactPixels& G, int p, int first, const float* __restrict__ pyv,
+                                             const float* __restrict__ pxv, float& py, float& px) {
+  const int q = p < 0 ? first : p;
+  if (G.W) {
+    const int y = q / G.W;
+    py = pyv[y];
+    px = pxv[q - y * G.W];
+  } else {
+    py = pyv[q];
+    px = pxv[q];
   }
-  if (g >= N) return;
-  float* dst = acc + (size_t)g * kAcc;
-  dst[0] = s.q; dst[1] = s.qu; dst[2] = s.qv; dst[3] = s.quu; dst[4] = s.qvv; dst[5] = s.quv;
-#pragma unroll
-  for (int c = 0; c < C; ++c) dst[6 + c] = po.op * s.gc[c];
 }
 
-// sum_p gout[p, c] * T[p] partials over 256-pixel chunks (the exact path's g_bg, render_triton.py:301).
+// Boxes (y0, y1, x0, x1): whether two of them meet. An empty box is (inf, -inf, inf, -inf).
+__device__ __forceinline__ bool boxes_meet(const float4& a, const float4& b) {
+  return (a.x <= b.y) & (b.x <= a.y) & (a.z <= b.w) & (b.z <= a.w);   // no branches: one load per box
+}
+__device__ __forceinline__ float4 empty_box() { return make_float4(INFINITY, -INFINITY, INFINITY, -INFINITY); }
+__device__ __forceinline__ float4 every_box() { return make_float4(-INFINITY, INFINITY, -INFINITY, INFINITY); }
+__device__ __forceinline__ bool is_every(const float4& box) { return box.x == -INFINITY; }
+
+// Union of the lanes' boxes (every lane calls it; everything when a lane's is not finite or not `ok`).
+__device__ __forceinline__ float4 wave_box(float4 b, bool ok) {
+  ok = ok & (fabsf(b.x) < INFINITY) & (fabsf(b.y) < INFINITY) & (fabsf(b.z) < INFINITY) & (fabsf(b.w) < INFINITY);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    b.x = fminf(b.x, __shfl_xor(b.x, m, 64));
+    b.y = fmaxf(b.y, __shfl_xor(b.y, m, 64));
+    b.z = fminf(b.z, __shfl_xor(b.z, m, 64));
+    b.w = fmaxf(b.w, __shfl_xor(b.w, m, 64));
+  }
+  return __all(ok) ? b : every_box();
+}
+
+// Whether a splat's falloff can be nonzero at a pixel centre in the box with middle (ym, xm) and half extents (hy, hx):
+// box_min_m's lower bound of u^2 + v^2 against splat_reach's limit, by a rounding margin of 1.5. True where the terms
+// of u or v are so large that the margin would not cover their rounding, and for values that are not finite.
+__device__ __forceinline__ bool splat_meets(const float4& r0, const float4& r1, float ym, float xm, float hy, float hx) {
+  const float dy = ym - r0.x, dx = xm - r0.y;
+  const float a = r0.z * dy, b = r0.w * dx, c = r1.x * dy, d = r1.y * dx;
+  const float m = box_min_m(a + b, c + d, fmaf(fabsf(r0.z), hy, fabsf(r0.w) * hx), fmaf(fabsf(r1.x), hy, fabsf(r1.y) * hx));
+  const bool out = (m > 127.5f + fmaxf(r1.w, 0.f)) & (fmaxf(fabsf(a) + fabsf(b), fabsf(c) + fabsf(d)) < 1e5f);
+  return !out;
+}
+
+// Running forward sums of one pixel: the transmittance product as t 2^e with t in [0.5, 1) after each norm() (exact, so
+// the product's rounding is the factors' own), the colour weight and the weighted colours.
 template <int C>
-__global__ __launch_bounds__(256) void k_bg_partial(const float* __restrict__ gout, const float* __restrict__ Tin, int P,
-                                                    float* __restrict__ part) {
-  __shared__ float s_w[4][kMaxC];
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+struct ExactSums {
+  float t = 1.f, s_a = 0.f, sc[C];
+  int e = 0;
+  __device__ ExactSums() {
+#pragma unroll
+    for (int c = 0; c < C; ++c) sc[c] = 0.f;
+  }
+  // at most four factors, each at least 1e-4, between two calls: t stays a normal float
+  __device__ __forceinline__ void norm() {
+    e += __builtin_amdgcn_frexp_expf(t);
+    t = __builtin_amdgcn_frexp_mantf(t);
+  }
+  // a pixel-pair with whitened offsets u, v of a splat with log2(opacity) lop and colour col
+  __device__ __forceinline__ void add(float u, float v, float lop, const float* col) {
+    const float a = fminf(hw_exp2(-fmaf(u, u, fmaf(v, v, -lop))), kClamp);
+    t = fmaf(-a, t, t);   // t (1 - a), one rounding
+    s_a += a;
+#pragma unroll
+    for (int c = 0; c < C; ++c) sc[c] = fmaf(a, col[c], sc[c]);
+  }
+  __device__ __forceinline__ void put(float* d, int stride) const {   // exact_part() floats, `stride` apart
+    d[0] = t;
+    d[stride] = __int_as_float(e);
+    d[2 * stride] = s_a;
+#pragma unroll
+    for (int c = 0; c < C; ++c) d[(3 + c) * stride] = sc[c];
+  }
+  __device__ __forceinline__ void take(const float* d, size_t stride) {
+    t *= d[0];
+    e += __float_as_int(d[stride]);
+    norm();
+    s_a += d[2 * stride];
+#pragma unroll
+    for (int c = 0; c < C; ++c) sc[c] += d[(3 + c) * stride];
+  }
+};
+
+template <int C>
+__host__ __device__ constexpr int exact_part() { return 3 + C; }   // floats of a pixel's partial sums: t, e, S_a, S_ac
+
+template <int C>
+__device__ __forceinline__ void store_exact(int p, const ExactSums<C>& s, const float* __restrict__ bg,
+                                            float* __restrict__ out, float* __restrict__ Tout,
+                                            float* __restrict__ asum_out, float* __restrict__ fg_out) {
+  const float T = ldexpf(s.t, s.e);
+  const float as = fmaxf(s.s_a, kAsumMin);
+  Tout[p] = T;
+  asum_out[p] = as;
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    float v = p < P ? gout[(size_t)p * C + c] * Tin[p] : 0.f;
-    v = wave_sum(v);
+    const float f = s.sc[c] / as;
+    fg_out[(size_t)p * C + c] = f;
+    out[(size_t)p * C + c] = (1.f - T) * f + T * bg[c];
+  }
+}
+
+// Pixel k < PX of `lane` in a forward group of 64 PX pixels: tiles of 8 x 8 (PX = 1) or 16 x 16 (PX = 4, a lane's four
+// pixels side by side in a row, so that they share the row's terms of u and v).
+template <int PX>
+__device__ __forceinline__ int exact_fwd_pixel(const ExactPixels& G, int group, int lane, int k) {
+  if (!G.ntx) return exact_list_pixel(G, (group * PX + k) * 64 + lane);
+  return PX == 1 ? exact_tile_pixel<8>(G, group, lane >> 3, lane & 7)
+                 : exact_tile_pixel<16>(G, group, lane >> 2, (lane & 3) * 4 + k);
+}
+
+// Forward. Workgroup = S shares (one per wave) of the splat batches for pixel group blockIdx.x / nsplit; lane = PX
+// pixels. Each wave lists the splats that meet its group and takes them 64 at a time: lane = splat loads their records
+// into LDS (one round trip for 64), lane = pixel reads them by broadcast. Bound by the VALU with PX = 4: a record's LDS
+// reads serve 256 pixels. (Records by scalar loads, one pixel per lane, each four records waiting for their own round trip: 245 us at 512 x 512
+// with 16,384 splats, 770 us for 10,000 unordered pixels and 92,160 splats.)
+// nsplit > 1: partial sums at part[split][k][slot], k < exact_part, slot = (group PX + pixel) 64 + lane.
+constexpr int kExactFwdWaves = 8;
+template <int C, int PX, bool GRID>
+__global__ __launch_bounds__(64 * kExactFwdWaves) void k_fwd_exact(
+    const float* __restrict__ rec, const float4* __restrict__ reach, int N, ExactPixels G,
+    const float* __restrict__ pyv, const float* __restrict__ pxv, int qi, int qo, const float* __restrict__ bg,
+    float* __restrict__ out, float* __restrict__ Tout, float* __restrict__ asum_out, float* __restrict__ fg_out,
+    float* __restrict__ part) {
+  constexpr int S = kExactFwdWaves, K = exact_part<C>();
+  constexpr int RS = C > 1 ? 12 : 8;   // floats of a staged record: gy, gx, A, B, Cc, D, lop, colour
+  __shared__ float4 s_rec4[S][64 * RS / 4];
+  __shared__ int s_cand[S][192], s_list[S][128];
+  static_assert(K <= RS, "the waves' partial sums take the staged records' place");
+  float (*s_part)[K][64] = reinterpret_cast<float (*)[K][64]>(&s_rec4[0][0]);
+  const int nsplit = qi / S * qo;
+  const int wg = xcd_swizzle(blockIdx.x, G.groups * nsplit);
+  const int group = wg / nsplit, split = wg - group * nsplit;
+  const int lane = (int)threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int so = split / (qi / S), q = (split - so * (qi / S)) * S + wv;
+  float py[PX], px[PX];
+  const int first = exact_fwd_pixel<PX>(G, group, 0, 0);
+  float4 gb;
+#pragma unroll
+  for (int k = 0; k < PX; ++k) {
+    exact_centre(G, exact_fwd_pixel<PX>(G, group, lane, k), first, pyv, pxv, py[k], px[k]);
+    gb = k ? make_float4(fminf(gb.x, py[k]), fmaxf(gb.y, py[k]), fminf(gb.z, px[k]), fmaxf(gb.w, px[k]))
+           : make_float4(py[k], py[k], px[k], px[k]);
+    if (GRID && k) py[k] = py[0];   // one row (a lane past the canvas: whatever, its pixels are not stored)
+  }
+  gb = wave_box(gb, true);
+  const float ym = 0.5f * (gb.x + gb.y), xm = 0.5f * (gb.z + gb.w), hy = 0.5f * (gb.y - gb.x), hx = 0.5f * (gb.w - gb.z);
+  const int nb = (N + 63) >> 6;
+  const float4* boxes = reach + N;
+  int* cand = s_cand[wv];   // splats whose box meets the group's
+  int* list = s_list[wv];   // those of them that splat_meets keeps
+  float4* st4 = s_rec4[wv];
+  const float* st = reinterpret_cast<const float*>(st4);
+  ExactSums<C> s[PX];
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int nc = 0, n = 0;
+  auto add = [&](int j) {
+    const float4 a = *reinterpret_cast<const float4*>(st + j * RS), b = *reinterpret_cast<const float4*>(st + j * RS + 4);
+    float col[kMaxC] = {b.w, 0.f, 0.f, 0.f};
+    if constexpr (C > 1) {
+      const float4 d = *reinterpret_cast<const float4*>(st + j * RS + 8);
+      col[1] = d.x;
+      col[2] = d.y;
+      col[3] = d.z;
+    }
+    float uy = 0.f, vy = 0.f;
+    if (GRID) {
+      const float dy = py[0] - a.x;
+      uy = a.z * dy;
+      vy = b.x * dy;
+    }
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+      const float dx = px[k] - a.y;
+      if (!GRID) {
+        const float dy = py[k] - a.x;
+        uy = a.z * dy;
+        vy = b.x * dy;
+      }
+      s[k].add(fmaf(a.w, dx, uy), fmaf(b.y, dx, vy), b.z, col);
+    }
+  };
+  // the first `cnt` <= 64 listed splats
+  auto run = [&](int cnt) {
+    wave_lds_sync();
+    const float4* r4 = reinterpret_cast<const float4*>(rec) + (size_t)list[lane < cnt ? lane : 0] * 4;
+    const float4 r0 = r4[0], r1 = r4[1], col = r4[2];
+    st4[lane * (RS / 4)] = r0;
+    st4[lane * (RS / 4) + 1] = make_float4(r1.x, r1.y, r1.w, col.x);
+    if constexpr (C > 1) st4[lane * (RS / 4) + 2] = make_float4(col.y, col.z, col.w, 0.f);
+    wave_lds_sync();
+    int j = 0;
+    for (; j + 4 <= cnt; j += 4) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add(j + i);
+#pragma unroll
+      for (int k = 0; k < PX; ++k) s[k].norm();
+    }
+    if (j < cnt) {
+      for (; j < cnt; ++j) add(j);
+#pragma unroll
+      for (int k = 0; k < PX; ++k) s[k].norm();
+    }
+  };
+  // the first `cnt` <= 64 candidates: the kept ones go to the list, 64 listed ones run
+  auto keep = [&](int cnt) {
+    wave_lds_sync();
+    const int id = cand[lane < cnt ? lane : 0];
+    bool in = lane < cnt;
+    if (reach) {
+      const float4* r4 = reinterpret_cast<const float4*>(rec) + (size_t)id * 4;
+      in = in & (splat_meets(r4[0], r4[1], ym, xm, hy, hx) | is_every(reach[id]));
+    }
+    const unsigned long long sm = __ballot(in);
+    if (in) list[n + __popcll(sm & below)] = id;
+    n += __popcll(sm);
+    if (n >= 64) {
+      run(64);
+      const int rest = list[64 + lane];   // past n: not used
+      wave_lds_sync();
+      list[lane] = rest;
+      n -= 64;
+    }
+  };
+  auto candidates = [&](bool in, int g) {
+    const unsigned long long sm = __ballot(in);
+    if (in) cand[nc + __popcll(sm & below)] = g;
+    nc += __popcll(sm);
+  };
+  int turn = 0;   // of the batches that meet the group, the wave takes those of its turn (turn = q modulo qi)
+  for (int sb = so * 64; sb < nb; sb += qo * 64) {
+    const float4 bb = reach ? boxes[min(sb + lane, nb - 1)] : every_box();
+    unsigned long long bm = __ballot((sb + lane < nb) & boxes_meet(bb, gb));
+    auto next = [&]() {   // the wave's next batch (its splat of this lane), or N
+      for (; bm; bm &= bm - 1, ++turn)
+        if ((turn & (qi - 1)) == q) {
+          const int g = (sb + __builtin_ctzll(bm)) * 64 + lane;
+          bm &= bm - 1;
+          ++turn;
+          return g;
+        }
+      return N;
+    };
+    while (bm) {   // two batches at once: their boxes' loads in flight together
+      const int ga = next(), gz = next();
+      const float4 oa = reach ? reach[min(ga, N - 1)] : every_box(), oz = reach ? reach[min(gz, N - 1)] : every_box();
+      candidates((ga < N) & boxes_meet(oa, gb), ga);
+      candidates((gz < N) & boxes_meet(oz, gb), gz);
+      while (nc >= 64) {   // at most 63 + 128 wait
+        keep(64);
+        const int r0 = cand[64 + lane], r1 = cand[128 + lane];   // past nc: not used
+        wave_lds_sync();
+        cand[lane] = r0;
+        cand[64 + lane] = r1;
+        nc -= 64;
+      }
+    }
+  }
+  if (nc) keep(nc);
+  if (n) run(n);
+  // pixel k of every lane: the waves' sums in wave order, by wave k
+#pragma unroll
+  for (int k = 0; k < PX; ++k) {
+    __syncthreads();   // the records, and pixel k - 1's sums, have been read
+    s[k].put(&s_part[wv][0][lane], 64);
+    __syncthreads();
+    if (wv == k) {
+      ExactSums<C> o;
+      for (int w = 0; w < S; ++w) o.take(&s_part[w][0][lane], 64);
+      if (nsplit > 1) {
+        const size_t plane = (size_t)G.groups * 64 * PX;
+        float* d = part + (size_t)split * K * plane + (size_t)(group * PX + k) * 64 + lane;
+        d[0] = o.t;
+        d[plane] = __int_as_float(o.e);
+        d[2 * plane] = o.s_a;
+#pragma unroll
+        for (int c = 0; c < C; ++c) d[(3 + c) * plane] = o.sc[c];
+      } else {
+        const int p = exact_fwd_pixel<PX>(G, group, lane, k);
+        if (p >= 0) store_exact<C>(p, o, bg, out, Tout, asum_out, fg_out);
+      }
+    }
+  }
+}
+
+// The workgroups' partial sums of every pixel, added in split order, then the composite. Wave = 64 slots.
+template <int C, int PX>
+__global__ __launch_bounds__(256) void k_exact_combine(ExactPixels G, int nsplit, const float* __restrict__ part,
+                                                       const float* __restrict__ bg, float* __restrict__ out,
+                                                       float* __restrict__ Tout, float* __restrict__ asum_out,
+                                                       float* __restrict__ fg_out) {
+  const int w = blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  if (w >= G.groups * PX) return;
+  const int p = exact_fwd_pixel<PX>(G, w / PX, lane, w % PX);
+  const size_t plane = (size_t)G.groups * 64 * PX;
+  const float* d = part + (size_t)w * 64 + lane;
+  ExactSums<C> s;
+  for (int k = 0; k < nsplit; ++k, d += exact_part<C>() * plane) s.take(d, plane);
+  if (p >= 0) store_exact<C>(p, s, bg, out, Tout, asum_out, fg_out);
+}
+
+// The backward's pixels, one wave per group: pix[slot] = (py, px, dS_log, dS_a, dS_ac[0..3]) of pixel slot
+// group * 64 + lane (zero terms for a lane without a pixel), the group's box (everything when a term is not finite: it
+// then reaches every splat, as 0 * inf does), and per workgroup of four groups the partial sums of g_bg =
+// sum_p gout T (render_triton.py:301), bg_part[c * gridDim.x + blockIdx.x].
+template <int C>
+__global__ __launch_bounds__(256) void k_exact_upstream(ExactPixels G, const float* __restrict__ pyv,
+                                                        const float* __restrict__ pxv, const float* __restrict__ bg,
+                                                        const float* __restrict__ Tin,
+                                                        const float* __restrict__ asum_in,
+                                                        const float* __restrict__ fg_in,
+                                                        const float* __restrict__ gout, float4* __restrict__ pix,
+                                                        float4* __restrict__ gboxes, float* __restrict__ bg_part) {
+  __shared__ float s_w[4][kMaxC];
+  const int wv = (int)(threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+  const int group = blockIdx.x * 4 + wv;
+  float bgp[kMaxC] = {0.f, 0.f, 0.f, 0.f};
+  if (group < G.groups) {
+    float4 pa = make_float4(0.f, 0.f, 0.f, 0.f);
+    float2 pb = make_float2(0.f, 0.f);
+    float py, px;
+    const int p = exact_fwd_pixel<1>(G, group, lane, 0);
+    exact_centre(G, p, __shfl(p, 0, 64), pyv, pxv, py, px);
+    if (p >= 0)
+      pixel_upstream<C, false, false>(p, 0, bg, Tin, asum_in, fg_in, gout, nullptr, nullptr, nullptr, pa, pb, bgp);
+    const float big = fmaxf(fmaxf(fmaxf(fabsf(pa.x), fabsf(pa.y)), fmaxf(fabsf(pa.z), fabsf(pa.w))),
+                            fmaxf(fabsf(pb.x), fabsf(pb.y)));
+    const bool nan = !(pa.x == pa.x && pa.y == pa.y && pa.z == pa.z && pa.w == pa.w && pb.x == pb.x && pb.y == pb.y);
+    const float4 gb = wave_box(make_float4(py, py, px, px), !nan && big < INFINITY);
+    float4* d = pix + ((size_t)group * 64 + lane) * 2;
+    d[0] = make_float4(py, px, pa.x, pa.y);
+    d[1] = make_float4(pa.z, pa.w, pb.x, pb.y);
+    if (lane == 0) gboxes[group] = gb;
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const float v = wave_sum(bgp[c]);
     if (lane == 0) s_w[wv][c] = v;
   }
   __syncthreads();
-  if (threadIdx.x < C) part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s_w[0][threadIdx.x] + s_w[1][threadIdx.x] +
-                                                                             s_w[2][threadIdx.x] + s_w[3][threadIdx.x];
+  if (threadIdx.x < C)
+    bg_part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
+        (s_w[0][threadIdx.x] + s_w[1][threadIdx.x]) + (s_w[2][threadIdx.x] + s_w[3][threadIdx.x]);
 }
 
-// g_bg[c] = sum of the nparts channel-major partials part[c * nparts + i], one 1024-thread workgroup.
-template <int C>
-__global__ __launch_bounds__(1024) void k_bg_sum(const float* __restrict__ part, int nparts, float* __restrict__ g_bg) {
-  __shared__ float s_w[16][kMaxC];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// Backward. Workgroup = kExactBwdWaves splat batches (512 splats) and one share of the blocks of GB pixel groups. For
+// each block its pixels are staged in LDS (the groups' records kExactStride floats apart, so that lanes on different
+// groups read different banks), every thread finds the groups that its own splat meets, and the (splat, group) pairs,
+// listed splat by splat, are taken 512 at a time by all waves, lane = pair over the group's 64 pixels; fewer pairs get a
+// power of two of lanes each. Then every thread adds its own splat's sums in list order. So only pairs that meet take
+// lanes, and the waves share them evenly (lane = splat over every group that any splat of its batch meets: 1,776
+// against 425 us at 512 x 512 with 16,384 splats).
+// The workgroup's sums go to part[split][k][splat slot], k < 6 + C.
+constexpr int kExactBwdWaves = 8;
+constexpr int kExactBwdThreads = 64 * kExactBwdWaves;
+constexpr int kExactStride = 64 * 8 + 4;
+template <int C, int GB>
+__global__ __launch_bounds__(kExactBwdThreads) void k_bwd_exact(
+    const float* __restrict__ rec, const float4* __restrict__ reach, int N, int groups,
+    const float4* __restrict__ pix, const float4* __restrict__ gboxes, int nsplit, float* __restrict__ part) {
+  constexpr int S = kExactBwdWaves, NT = kExactBwdThreads, R = pair_rec<C>();
+  static_assert(GB <= 16, "one bit of the pair code's low byte, one of 64 lanes, per group");
+  __shared__ float4 s_pix4[GB * kExactStride / 4];
+  __shared__ unsigned short s_pair[NT];   // of one pass: splat of the workgroup << 4 | group of the block
+  __shared__ float s_sum[R][NT];
+  __shared__ int s_tot[2][S];   // a block without pairs has one barrier only: the next block takes the other row
+  const float* s_pix = reinterpret_cast<const float*>(s_pix4);
+  const int nb = (N + 63) >> 6, nrow = (nb + S - 1) / S;
+  const int wg = xcd_swizzle(blockIdx.x, nrow * nsplit);
+  const int row = wg / nsplit, split = wg - row * nsplit;
+  const int t = (int)threadIdx.x, lane = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = row * NT + t, gs = min(g, N - 1);
+  const float4* recs = reinterpret_cast<const float4*>(rec);
+  float4 own = reach ? reach[gs] : every_box();
+  if (g >= N) own = empty_box();
+  const bool every = is_every(own);
+  const float4 r0 = recs[(size_t)gs * 4], r1 = recs[(size_t)gs * 4 + 1];
+  float4 wb = empty_box();   // the union of the workgroup's batches
+  for (int w = 0; w < S && row * S + w < nb; ++w) {
+    const float4 b = reach ? reach[N + row * S + w] : every_box();
+    wb = make_float4(fminf(wb.x, b.x), fmaxf(wb.y, b.y), fminf(wb.z, b.z), fmaxf(wb.w, b.w));
+  }
+  float acc[R];
 #pragma unroll
-  for (int c = 0; c < C; ++c) {
-    const float* row = part + (size_t)c * nparts;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
-    int i = threadIdx.x;
-    for (; i + 3 * 1024 < nparts; i += 4 * 1024) {
-      a0 += row[i]; a1 += row[i + 1024]; a2 += row[i + 2048]; a3 += row[i + 3072];
+  for (int k = 0; k < R; ++k) acc[k] = 0.f;
+  const int nblocks = (groups + GB - 1) / GB;
+  int turn = 0;
+  for (int blk = split; blk < nblocks; blk += nsplit) {
+    const int gr0 = blk * GB, ng = min(GB, groups - gr0);
+    const float4 gbl = gboxes[gr0 + min(lane, ng - 1)];   // lane k: group k of the block
+    if (!__any(boxes_meet(gbl, wb))) continue;            // the same for every wave
+    auto group_at = [&](int k) {
+      auto f = [&](float x) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), k)); };
+      return make_float4(f(gbl.x), f(gbl.y), f(gbl.z), f(gbl.w));
+    };
+    unsigned mk = 0;   // the groups that the thread's splat meets
+    for (int k = 0; k < ng; ++k) {
+      const float4 gb = group_at(k);
+      bool in = boxes_meet(gb, own);
+      if (in && !every)
+        in = splat_meets(r0, r1, 0.5f * (gb.x + gb.y), 0.5f * (gb.z + gb.w), 0.5f * (gb.y - gb.x), 0.5f * (gb.w - gb.z));
+      mk |= in ? 1u << k : 0u;
     }
-    for (; i < nparts; i += 1024) a0 += row[i];
-    const float x = wave_sum((a0 + a1) + (a2 + a3));
-    if (lane == 0) s_w[wv][c] = x;
+    const int cnt = __popc(mk);
+    const int inc = wave_incl_scan<int>(cnt, lane);
+    int* tot = s_tot[turn ^= 1];
+    if (lane == 63) tot[wv] = inc;
+    __syncthreads();   // also: the previous block's pixels and sums have been read
+    int start = inc - cnt, total = 0;
+#pragma unroll
+    for (int w = 0; w < S; ++w) {
+      const int x = tot[w];
+      if (w < wv) start += x;
+      total += x;
+    }
+    const int end = start + cnt;
+    if (total)
+      for (int i = t; i < ng * 128; i += NT)
+        s_pix4[(i >> 7) * (kExactStride / 4) + (i & 127)] = pix[(size_t)gr0 * 128 + i];
+    unsigned left = mk;   // the lane's pairs not yet listed
+    for (int p0 = 0, o = start; p0 < total; p0 += NT) {
+      const int np = min(NT, total - p0);
+      for (; left && o < p0 + NT; left &= left - 1, ++o) s_pair[o - p0] = (unsigned short)(t << 4 | __builtin_ctz(left));
+      __syncthreads();   // the pairs, and the block's pixels
+      int lg = 0;   // 2^lg <= 64 lanes per pair
+      while (lg < 6 && (np << (lg + 1)) <= NT) ++lg;
+      const int pr = t >> lg;
+      const bool act = pr < np;
+      const int code = act ? s_pair[pr] : 0;
+      const int grp = code & 15;
+      const float4* rr = recs + (size_t)min(row * NT + (code >> 4), N - 1) * 4;
+      const float4 q0 = rr[0], q1 = rr[1], col = rr[2];
+      const float2 sc = *reinterpret_cast<const float2*>(rr + 3);
+      PairGeo pg = pair_geo(q0, q1);
+      mute_pair(!act, pg);
+      const PairOp po = pair_op(q1.z);
+      const float4 gb = make_float4(__shfl(gbl.x, grp, 64), __shfl(gbl.y, grp, 64), __shfl(gbl.z, grp, 64),
+                                    __shfl(gbl.w, grp, 64));
+      const bool near = act && near_possible(po.op, q1.w, q0.x, q0.y, fmaxf(sc.x, sc.y), gb.x, gb.y, gb.z, gb.w);
+      const int npx = 64 >> lg, step = 8 << lg;   // a pair's lanes take its pixels in turn
+      const float* px = s_pix + grp * kExactStride + (t & ((1 << lg) - 1)) * 8;
+      PairSums<C> s;
+      auto pixels = [&](auto careful) {
+#pragma unroll 2
+        for (int j = 0; j < npx; ++j, px += step) {
+          const float4 a = *reinterpret_cast<const float4*>(px), b = *reinterpret_cast<const float4*>(px + 4);
+          const float dy = a.x - pg.gy, dx = a.y - pg.gx;
+          const float u = fmaf(pg.A, dy, pg.B * dx), v = fmaf(pg.Cc, dy, pg.D * dx);
+          const float m = fmaf(u, u, v * v);
+          const float f = hw_exp2(-m);
+          const float4 pa = make_float4(a.z, a.w, b.x, b.y);
+          const float2 pb = make_float2(b.z, b.w);
+          if constexpr (decltype(careful)::value != 0)
+            bwd_px_near<C, false>(u, v, m, f, po, col, pa, pb, s);
+          else
+            bwd_acc<C, false>(u, v, f, fmaf(-po.op, f, 1.f), col, pa, pb, s);
+        }
+      };
+      if (__any(near))
+        pixels(IC<1>{});
+      else
+        pixels(IC<0>{});
+      s_sum[0][t] = s.q; s_sum[1][t] = s.qu; s_sum[2][t] = s.qv;
+      s_sum[3][t] = s.quu; s_sum[4][t] = s.qvv; s_sum[5][t] = s.quv;
+#pragma unroll
+      for (int c = 0; c < C; ++c) s_sum[6 + c][t] = s.gc[c];
+      __syncthreads();
+      const int e0 = max(start - p0, 0) << lg, e1 = min(end - p0, np) << lg;
+      for (int e = e0; e < e1; ++e) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) acc[k] += s_sum[k][e];
+      }
+    }
+  }
+  if (g >= nb * 64) return;
+  float* d = part + (size_t)split * R * nb * 64 + g;
+#pragma unroll
+  for (int k = 0; k < R; ++k) d[(size_t)k * nb * 64] = acc[k];
+}
+
+// The workgroups' sums of every splat, then its parameter gradients (w.r.t. the raw log-scales with lsc, chained
+// through the activation). Workgroup = 64 splats, wave w adds splits w, w + 4, ... in order and wave 0 the four waves'
+// sums; the first workgroup sums g_bg when asked for.
+template <int C>
+__global__ __launch_bounds__(256) void k_exact_finalize(const float* __restrict__ rec, int N, int nsplit,
+                                                        const float* __restrict__ part,
+                                                        const float* __restrict__ bg_part, int nparts,
+                                                        float* __restrict__ g_mu, float* __restrict__ g_scale,
+                                                        float* __restrict__ g_theta, float* __restrict__ g_op,
+                                                        float* __restrict__ g_col, float* __restrict__ g_bg,
+                                                        const float* __restrict__ lsc) {
+  constexpr int R = pair_rec<C>();
+  __shared__ float s_w[3][R][64];
+  if (g_bg && blockIdx.x == 0) {
+    block_bg_sum<C>(bg_part, nparts, g_bg);
+    return;
+  }
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
+  const int g = (blockIdx.x - (g_bg ? 1 : 0)) * 64 + lane;   // a slot of the partial sums, also past N
+  const size_t plane = (size_t)((N + 63) & ~63);
+  const float* d = part + g + (size_t)wv * R * plane;
+  float v[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) v[k] = 0.f;
+  for (int i = wv; i < nsplit; i += 4, d += 4 * R * plane) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) v[k] += d[k * plane];
+  }
+  if (wv > 0) {
+#pragma unroll
+    for (int k = 0; k < R; ++k) s_w[wv - 1][k][lane] = v[k];
   }
   __syncthreads();
-  if (threadIdx.x < C) {
-    float x = 0.f;
-    for (int w = 0; w < 16; ++w) x += s_w[w][threadIdx.x];
-    g_bg[threadIdx.x] = x;
+  if (wv > 0 || g >= N) return;
+  const float op = rec[(size_t)g * kRec + R_OP];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    v[k] += s_w[0][k][lane] + s_w[1][k][lane] + s_w[2][k][lane];
+    if (k >= 6) v[k] *= op;
   }
-}
-
-// Exact path: per-splat sums (stride kAcc) -> parameter gradients.
-template <int C>
-__global__ __launch_bounds__(256) void k_acc_finalize(const float* __restrict__ rec, const float* __restrict__ acc, int N,
-                                                      float* __restrict__ g_mu, float* __restrict__ g_scale,
-                                                      float* __restrict__ g_theta, float* __restrict__ g_op,
-                                                      float* __restrict__ g_col) {
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  if (g >= N) return;
-  float v[kSums];
-  for (int k = 0; k < kSums; ++k) v[k] = acc[(size_t)g * kAcc + k];
-  splat_grads<C>(g, rec, v, g_mu, g_scale, g_theta, g_op, g_col, nullptr);
+  splat_grads<C>(g, rec, v, g_mu, g_scale, g_theta, g_op, g_col, lsc);
 }
 
 // ------------------------------------------------------------------------------------ upsample adjoint
@@ -2097,44 +2508,180 @@ int splat_reduce_pairs(const float* rec, const int* offsets, const int* pair_spl
   });
 }
 
-int splat_exact_fwd(const float* rec, int N, int C, const float* py, const float* px, int P, const float* bg, float* out,
-                    float* T, float* asum, float* fg, void* stream) {
-  if (N < 0 || P < 1 || !rec || !py || !px || !bg || !out || !T || !asum || !fg)
-    return set_error(kInvalid, "splat_exact_fwd: bad arguments N=%d P=%d", N, P);
+namespace {
+
+// Groups of 64 `px` pixels (1 or 4) of P pixels (grid_w = 0), or of a grid of P / grid_w rows of grid_w pixels.
+ExactPixels exact_pixels(int P, int grid_w, int px, const int* perm) {
+  ExactPixels G{P, grid_w, grid_w > 0 ? P / grid_w : 0, 0, (int)((P + 64LL * px - 1) / (64 * px)), grid_w > 0 ? nullptr : perm};
+  const int tw = px == 4 ? 16 : 8;
+  if (G.W >= 8 && G.H >= 8) {   // narrower grids would leave lanes of a tile without a pixel
+    G.ntx = (G.W + tw - 1) / tw;
+    G.groups = G.ntx * ((G.H + tw - 1) / tw);
+  }
+  return G;
+}
+
+constexpr int kExactWaves = 8192;   // 8 per SIMD
+
+// Forward: four pixels per lane where groups of 256 pixels times batches make enough waves; shares of the splat
+// batches for about kExactWaves waves in all: qi shares (a power of two from one workgroup's to 64, no more than there
+// are batches) that take the batches meeting a group in turn, so that a group's waves have the same number of them
+// wherever it lies (shares by the batch's number instead, splats in cell order: 229 against 141 us at 512 x 512), and
+// qo shares of the blocks of 64 batches.
+struct ExactFwdPlan {
+  int px, qi, qo, nsplit;
+  ExactPixels G;
+};
+ExactFwdPlan exact_fwd_plan(int N, int P, int grid_w, const int* perm) {
+  const long long nb = (N + 63) / 64, blocks = (nb + 63) / 64;
+  ExactFwdPlan p{};
+  p.px = (P + 255LL) / 256 * nb >= kExactWaves / 2 ? 4 : 1;
+  p.G = exact_pixels(P, grid_w, p.px, perm);
+  const long long groups = p.G.groups;
+  p.qi = kExactFwdWaves;
+  p.qo = 1;
+  while (p.qi < 64 && p.qi < nb && groups * p.qi < kExactWaves) p.qi *= 2;
+  while (p.qi == 64 && p.qo < 16 && p.qo < blocks && groups * p.qi * p.qo < kExactWaves) ++p.qo;
+  p.nsplit = p.qi / kExactFwdWaves * p.qo;
+  return p;
+}
+
+// Backward: blocks of 16 pixel groups while they fill the card twice over, else of one (a 64 x 64 grid with 1,024 splats
+// is 8 workgroups of 16 groups or 128 of one); shares of the blocks for about twice kExactWaves waves.
+struct ExactBwdSplit {
+  int gb, nsplit;
+};
+ExactBwdSplit exact_bwd_split(const ExactPixels& G, int N) {
+  const long long rows = N > 0 ? (N + kExactBwdThreads - 1) / kExactBwdThreads : 1;
+  ExactBwdSplit s{16, 1};
+  if (rows * ((G.groups + 15) / 16) < 512) s.gb = 1;
+  const long long blocks = (G.groups + s.gb - 1) / s.gb, want = (2 * kExactWaves / kExactBwdWaves + rows - 1) / rows;
+  s.nsplit = (int)max(1LL, min(min(want, blocks), 256LL));
+  return s;
+}
+
+bool exact_sizes_ok(int N, int C, int P, int grid_w) {
+  return N >= 0 && C >= 1 && C <= kMaxC && P >= 1 && grid_w >= 0 && (grid_w == 0 || P % grid_w == 0);
+}
+
+struct ExactBwdPlan {
+  int gb, nsplit, nup;
+  size_t off_gbox, off_bg, off_part, total;
+};
+ExactBwdPlan exact_bwd_plan(const ExactPixels& G, int N, int C) {
+  ExactBwdPlan p{};
+  const ExactBwdSplit sp = exact_bwd_split(G, N);
+  p.gb = sp.gb;
+  p.nsplit = sp.nsplit;
+  p.nup = (G.groups + 3) / 4;
+  size_t o = align256(sizeof(float) * 8 * 64 * (size_t)G.groups);
+  p.off_gbox = o; o += align256(sizeof(float4) * (size_t)G.groups);
+  p.off_bg = o;   o += align256(sizeof(float) * (size_t)p.nup * C);
+  p.off_part = o; o += align256(sizeof(float) * (6 + C) * (size_t)((N + 63) & ~63) * p.nsplit);
+  p.total = o;
+  return p;
+}
+
+}  // namespace
+
+size_t splat_exact_fwd_workspace_bytes(int N, int C, int P, int grid_w) {
+  if (!exact_sizes_ok(N, C, P, grid_w)) return 0;
+  const ExactFwdPlan p = exact_fwd_plan(N, P, grid_w, nullptr);
+  return p.nsplit > 1 ? align256(sizeof(float) * (3 + C) * 64 * (size_t)(p.G.groups * p.px) * p.nsplit) : 0;
+}
+
+int splat_exact_render(const float* rec, const float* reach, int N, int C, const float* py, const float* px, int P,
+                       int grid_w, const int* order, const float* bg, float* out, float* T, float* asum, float* fg,
+                       void* ws, size_t ws_bytes, void* stream) {
+  if (!exact_sizes_ok(N, C, P, grid_w) || (N > 0 && !rec) || !py || !px || !bg || !out || !T || !asum || !fg)
+    return set_error(kInvalid, "splat_exact_render: bad arguments N=%d C=%d P=%d grid_w=%d", N, C, P, grid_w);
+  ExactFwdPlan p = exact_fwd_plan(N, P, grid_w, order);
+  if (!ws) {   // without a workspace the shares stay within one workgroup
+    p.qi = kExactFwdWaves;
+    p.qo = p.nsplit = 1;
+  } else if (ws_bytes < splat_exact_fwd_workspace_bytes(N, C, P, grid_w)) {
+    return set_error(kWorkspace, "splat_exact_render: workspace of %zu bytes, %zu needed", ws_bytes,
+                     splat_exact_fwd_workspace_bytes(N, C, P, grid_w));
+  }
   hipStream_t st = (hipStream_t)stream;
   return with_c(C, [&](auto cc) {
-    k_fwd_exact<decltype(cc)::value><<<(P + 63) / 64, 64, 0, st>>>(rec, N, py, px, P, bg, out, T, asum, fg);
+    constexpr int CC = decltype(cc)::value;
+    auto launch = [&](auto npx, auto grid) {
+      constexpr int PX = decltype(npx)::value;
+      k_fwd_exact<CC, PX, decltype(grid)::value != 0><<<p.G.groups * p.nsplit, 64 * kExactFwdWaves, 0, st>>>(
+          rec, reinterpret_cast<const float4*>(reach), N, p.G, py, px, p.qi, p.qo, bg, out, T, asum, fg, (float*)ws);
+      if (p.nsplit > 1)
+        k_exact_combine<CC, PX><<<(p.G.groups * PX + 3) / 4, 256, 0, st>>>(p.G, p.nsplit, (const float*)ws, bg, out, T,
+                                                                          asum, fg);
+    };
+    if (p.px == 1)
+      launch(IC<1>{}, IC<0>{});   // a pixel has its row's terms to itself
+    else if (p.G.ntx)
+      launch(IC<4>{}, IC<1>{});
+    else
+      launch(IC<4>{}, IC<0>{});
     return check_launch("k_fwd_exact");
   });
 }
 
+size_t splat_exact_render_bwd_workspace_bytes(int N, int C, int P, int grid_w) {
+  if (!exact_sizes_ok(N, C, P, grid_w)) return 0;
+  return exact_bwd_plan(exact_pixels(P, grid_w, 1, nullptr), N, C).total;
+}
+
+int splat_exact_render_bwd(const float* rec, const float* reach, int N, int C, const float* py, const float* px, int P,
+                           int grid_w, const int* order, const float* bg, const float* T, const float* asum,
+                           const float* fg, const float* gout, const float* log_scale, float* g_mu, float* g_scale, float* g_theta,
+                           float* g_op, float* g_color, float* g_bg, void* ws, size_t ws_bytes, void* stream) {
+  if (!exact_sizes_ok(N, C, P, grid_w) || !py || !px || !bg || !T || !asum || !fg || !gout ||
+      (N > 0 && (!rec || !g_mu || !g_scale || !g_op || !g_color)))
+    return set_error(kInvalid, "splat_exact_render_bwd: bad arguments N=%d C=%d P=%d grid_w=%d", N, C, P, grid_w);
+  const ExactPixels G = exact_pixels(P, grid_w, 1, order);
+  const ExactBwdPlan pl = exact_bwd_plan(G, N, C);
+  if (!ws || ws_bytes < pl.total) return set_error(kWorkspace, "splat_exact_render_bwd: workspace too small");
+  if (N == 0 && !g_bg) return kOk;
+  hipStream_t st = (hipStream_t)stream;
+  char* base = (char*)ws;
+  float4* pix = (float4*)base;
+  float4* gboxes = (float4*)(base + pl.off_gbox);
+  float* bg_part = (float*)(base + pl.off_bg);
+  float* part = (float*)(base + pl.off_part);
+  return with_c(C, [&](auto cc) {
+    constexpr int CC = decltype(cc)::value;
+    k_exact_upstream<CC><<<pl.nup, 256, 0, st>>>(G, py, px, bg, T, asum, fg, gout, pix, gboxes, bg_part);
+    if (N > 0) {
+      const int grid = (N + kExactBwdThreads - 1) / kExactBwdThreads * pl.nsplit;
+      const float4* rc = reinterpret_cast<const float4*>(reach);
+      auto launch = [&](auto gb) {
+        k_bwd_exact<CC, decltype(gb)::value><<<grid, kExactBwdThreads, 0, st>>>(rec, rc, N, G.groups, pix, gboxes,
+                                                                                pl.nsplit, part);
+      };
+      if (pl.gb == 16)
+        launch(IC<16>{});
+      else
+        launch(IC<1>{});
+    }
+    k_exact_finalize<CC><<<(N + 63) / 64 + (g_bg ? 1 : 0), 256, 0, st>>>(
+        rec, N, pl.nsplit, part, bg_part, pl.nup, g_mu, g_scale, g_theta, g_op, g_color, g_bg, log_scale);
+    return check_launch("splat_exact_render_bwd");
+  });
+}
+
+int splat_exact_fwd(const float* rec, int N, int C, const float* py, const float* px, int P, const float* bg, float* out,
+                    float* T, float* asum, float* fg, void* stream) {
+  if (!rec) return set_error(kInvalid, "splat_exact_fwd: bad arguments N=%d P=%d", N, P);
+  return splat_exact_render(rec, nullptr, N, C, py, px, P, 0, nullptr, bg, out, T, asum, fg, nullptr, 0, stream);
+}
+
 size_t splat_exact_bwd_workspace_bytes(int N, int C, int P) {
-  return align256(sizeof(float) * kAcc * (size_t)(N > 0 ? N : 1)) +
-         align256(sizeof(float) * (size_t)((P + 255) / 256 + 1) * (C > 0 ? C : 1));
+  return splat_exact_render_bwd_workspace_bytes(N, C, P, 0);
 }
 
 int splat_exact_bwd(const float* rec, int N, int C, const float* py, const float* px, int P, const float* bg,
                     const float* T, const float* asum, const float* fg, const float* gout, float* g_mu, float* g_scale,
                     float* g_theta, float* g_op, float* g_color, float* g_bg, void* ws, size_t ws_bytes, void* stream) {
-  if (N < 0 || P < 1 || !py || !px || !bg || !T || !asum || !fg || !gout ||
-      (N > 0 && (!rec || !g_mu || !g_scale || !g_op || !g_color)))
-    return set_error(kInvalid, "splat_exact_bwd: bad arguments N=%d P=%d", N, P);
-  if (ws_bytes < splat_exact_bwd_workspace_bytes(N, C, P)) return set_error(kWorkspace, "splat_exact_bwd: workspace too small");
-  hipStream_t st = (hipStream_t)stream;
-  float* acc = (float*)ws;
-  float* part = (float*)((char*)ws + align256(sizeof(float) * kAcc * (size_t)(N > 0 ? N : 1)));
-  const int nchunk = (P + 255) / 256;
-  return with_c(C, [&](auto cc) {
-    constexpr int CC = decltype(cc)::value;
-    if (N > 0) k_bwd_exact<CC><<<(N + 63) / 64, 64, 0, st>>>(rec, N, py, px, P, bg, T, asum, fg, gout, acc);
-    if (g_bg) {
-      k_bg_partial<CC><<<nchunk, 256, 0, st>>>(gout, T, P, part);
-      k_bg_sum<CC><<<1, 1024, 0, st>>>(part, nchunk, g_bg);
-    }
-    if (N > 0)
-      k_acc_finalize<CC><<<(N + 255) / 256, 256, 0, st>>>(rec, acc, N, g_mu, g_scale, g_theta, g_op, g_color);
-    return check_launch("splat_exact_bwd");
-  });
+  return splat_exact_render_bwd(rec, nullptr, N, C, py, px, P, 0, nullptr, bg, T, asum, fg, gout, nullptr, g_mu, g_scale,
+                                g_theta, g_op, g_color, g_bg, ws, ws_bytes, stream);
 }
 
 }  // extern "C"

@@ -65,6 +65,15 @@ _SIGS = {
     "splat_exact_bwd_workspace_bytes": (_SZ, [_I, _I, _I]),
     "splat_exact_bwd": (_I, [_VP, _I, _I, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,
                              _VP, _SZ, _VP]),
+    "splat_exact_reach_bytes": (_SZ, [_I]),
+    "splat_decode_exact": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I, _I, _VP, _VP, _VP]),
+    "splat_exact_fwd_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
+    "splat_exact_order_bytes": (_SZ, [_I, _I]),
+    "splat_exact_order": (_I, [_VP, _VP, _I, _I, _VP, _SZ, _VP]),
+    "splat_exact_render": (_I, [_VP, _VP, _I, _I, _VP, _VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
+    "splat_exact_render_bwd_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
+    "splat_exact_render_bwd": (_I, [_VP, _VP, _I, _I, _VP, _VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,
+                                    _VP, _VP, _VP, _VP, _SZ, _VP]),
 }
 
 EXPORTED = tuple(_SIGS)

@@ -11,10 +11,15 @@ from __future__ import annotations
 import torch
 
 
+def _pixel_axes(H, W, device, dtype):
+    """render.py:61-65: the row centres [H] and column centres [W] from linspace."""
+    return (torch.linspace(0.5 / H, 1 - 0.5 / H, H, device=device, dtype=dtype),
+            torch.linspace(0.5 / W, 1 - 0.5 / W, W, device=device, dtype=dtype))
+
+
 def _pixels(H, W, device, dtype):
     """render.py:61-65: [H*W, 2] (y, x) pixel centres from linspace."""
-    ys = torch.linspace(0.5 / H, 1 - 0.5 / H, H, device=device, dtype=dtype)
-    xs = torch.linspace(0.5 / W, 1 - 0.5 / W, W, device=device, dtype=dtype)
+    ys, xs = _pixel_axes(H, W, device, dtype)
     gy, gx = torch.meshgrid(ys, xs, indexing="ij")
     return torch.stack([gy, gx], dim=-1).reshape(H * W, 2)
 

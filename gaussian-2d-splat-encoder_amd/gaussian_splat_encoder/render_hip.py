@@ -26,7 +26,7 @@ import torch.nn.functional as F
 from . import _lib
 from ._lib import FLAG_DEFER, FLAG_FIELDS, FLAG_LOG_SCALE, FLAG_ODDS, FLAG_UPS, FLAG_WIDE, SplatLevels, check, ptr
 from .params import activate_scale
-from .render import _pixels
+from .render import _pixel_axes
 
 
 class PairBudgetExceeded(RuntimeError):
@@ -1126,68 +1126,83 @@ class _AlphaRenderLevels(torch.autograd.Function):
 
 
 # ----------------------------------------------------------------------------------------------- exact path
-def _forward(mu, scale, color, opacity, bg, py, px, theta):
-    """render_triton.py:128-157: every pixel sums every splat. Returns out [B,P,C], T, asum, fg."""
+def _forward(mu, scale, color, opacity, bg, py, px, theta, grid_w=0, scale_is_log=False):
+    """render_triton.py:128-157: every pixel sums every splat. Returns out [B,P,C], T, asum, fg and what the backward
+    reads again: the pixels' order (or None), then each image's decoded splats (records, then the boxes outside which
+    their falloff is zero). grid_w = 0: P pixels with centres
+    (py[p], px[p]); else a grid of len(py) rows and grid_w columns with centres (py[y], px[x]). scale_is_log: `scale`
+    holds fp32 raw log-scales, activated in the decode pass."""
     _dev_check(mu, scale, color, opacity, bg, theta)
     B, N, C = color.shape
-    P = py.shape[0]
+    P = py.shape[0] * (grid_w or 1)
     dev = mu.device
     lib, stream = _lib.load(), _lib.stream_ptr(dev)
     mu_, sc_, col_, op_, th_, bgf = _f32(mu), _f32(scale), _f32(color), _f32(opacity), _f32(theta), _f32(bg)
     pyf, pxf = _f32(py), _f32(px)
     out, T, asum, fg = _empty((B, P, C), dev), _empty((B, P), dev), _empty((B, P), dev), _empty((B, P, C), dev)
-    recs = []
+    flags = FLAG_LOG_SCALE if scale_is_log else 0
+    nr = 64 * N
+    nws = lib.splat_exact_fwd_workspace_bytes(N, C, P, grid_w)
+    ws = _ws(nws, dev) if nws else None   # reused across the batch (stream order)
+    nord = 0 if grid_w else lib.splat_exact_order_bytes(N, P)
+    order = _ws(nord, dev) if nord else None
+    if nord:
+        check(lib.splat_exact_order(ptr(pyf), ptr(pxf), N, P, ptr(order), nord, stream), "splat_exact_order")
+    recs = [order]
     for b in range(B):
-        rec = _empty((max(N, 1), 16), dev)
-        if N:
-            check(lib.splat_decode(ptr(mu_[b]), ptr(sc_[b]), None if th_ is None else ptr(th_[b]), ptr(op_[b]),
-                                   ptr(col_[b]), C, N, ptr(rec), stream), "splat_decode")
-        check(lib.splat_exact_fwd(ptr(rec), N, C, ptr(pyf), ptr(pxf), P, ptr(bgf[b]), ptr(out[b]), ptr(T[b]),
-                                  ptr(asum[b]), ptr(fg[b]), stream), "splat_exact_fwd")
+        rec = _ws(nr + lib.splat_exact_reach_bytes(N), dev)
+        r0 = rec.data_ptr()
+        check(lib.splat_decode_exact(_bptr(mu_, b), _bptr(sc_, b), _bptr(th_, b), _bptr(op_, b), _bptr(col_, b), C, N,
+                                     flags, r0, r0 + nr, stream), "splat_decode_exact")
+        check(lib.splat_exact_render(r0, r0 + nr, N, C, ptr(pyf), ptr(pxf), P, grid_w, ptr(order), _bptr(bgf, b),
+                                     _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b), ptr(ws), nws, stream),
+              "splat_exact_render")
         recs.append(rec)
     return out, T, asum, fg, recs
 
 
-def _backward(grad_out, mu, scale, color, opacity, bg, py, px, theta, T, asum, fg, recs=None):
-    """render_triton.py:269-303: grads for mu, scale, color, opacity, bg, theta."""
+def _backward(grad_out, mu, scale, color, opacity, bg, py, px, theta, T, asum, fg, recs=None, grid_w=0,
+              scale_is_log=False):
+    """render_triton.py:269-303: grads for mu, scale (the raw log-scale with scale_is_log), color, opacity, bg, theta."""
     B, N, C = color.shape
-    P = py.shape[0]
+    P = py.shape[0] * (grid_w or 1)
     dev = mu.device
-    has_th = theta is not None
     lib, stream = _lib.load(), _lib.stream_ptr(dev)
-    g_mu, g_scale, g_col, g_op, g_th = _grads_out(B, N, C, dev, has_th)
-    g_bg = _empty((B, C), dev)
+    g_mu, g_scale, g_col, g_op, g_th, g_bg = _grads_bg_out(B, N, C, dev, theta is not None)
     if recs is None:
-        recs = _forward(mu, scale, color, opacity, bg, py, px, theta)[4]
+        recs = _forward(mu, scale, color, opacity, bg, py, px, theta, grid_w, scale_is_log)[4]
     go, bgf, pyf, pxf = _f32(grad_out), _f32(bg), _f32(py), _f32(px)
-    ws = _ws(lib.splat_exact_bwd_workspace_bytes(N, C, P), dev)
+    lsc = _f32(scale) if scale_is_log else None
+    ws = _ws(lib.splat_exact_render_bwd_workspace_bytes(N, C, P, grid_w), dev)
     for b in range(B):
-        check(lib.splat_exact_bwd(ptr(recs[b]), N, C, ptr(pyf), ptr(pxf), P, ptr(bgf[b]), ptr(T[b]), ptr(asum[b]),
-                                  ptr(fg[b]), ptr(go[b]), ptr(g_mu[b]), ptr(g_scale[b]),
-                                  None if g_th is None else ptr(g_th[b]), ptr(g_op[b]), ptr(g_col[b]), ptr(g_bg[b]),
-                                  ptr(ws), ws.numel(), stream), "splat_exact_bwd")
+        r0 = recs[1 + b].data_ptr()
+        check(lib.splat_exact_render_bwd(r0, r0 + 64 * N, N, C, ptr(pyf), ptr(pxf), P, grid_w, ptr(recs[0]),
+                                         _bptr(bgf, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b), _bptr(go, b), _bptr(lsc, b),
+                                         _bptr(g_mu, b), _bptr(g_scale, b), _bptr(g_th, b), _bptr(g_op, b),
+                                         _bptr(g_col, b), _bptr(g_bg, b), ptr(ws), ws.numel(), stream),
+              "splat_exact_render_bwd")
     return g_mu, g_scale, g_col, g_op, g_bg, g_th
 
 
 class _AlphaRender(torch.autograd.Function):
-    """render_triton.py:307-323 (exact path)."""
+    """render_triton.py:307-323 (exact path). grid_w, scale_is_log as in _forward; with scale_is_log the gradient of
+    `scale` is w.r.t. the raw log-scale."""
 
     @staticmethod
-    def forward(ctx, mu, scale, color, opacity, bg, theta, py, px):
-        out, T, asum, fg, recs = _forward(mu, scale, color, opacity, bg, py, px, theta)
+    def forward(ctx, mu, scale, color, opacity, bg, theta, py, px, grid_w=0, scale_is_log=False):
+        out, T, asum, fg, recs = _forward(mu, scale, color, opacity, bg, py, px, theta, grid_w, scale_is_log)
         ctx.has_theta = theta is not None
         ctx.recs = recs
-        ctx.save_for_backward(mu, scale, color, opacity, bg, theta if theta is not None else mu.new_zeros(1),
-                              py, px, T, asum, fg)
+        ctx.opts = (grid_w, scale_is_log)
+        ctx.save_for_backward(mu, scale, color, opacity, bg, theta, py, px, T, asum, fg)
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
         mu, scale, color, opacity, bg, theta, py, px, T, asum, fg = ctx.saved_tensors
-        th = theta if ctx.has_theta else None
-        g_mu, g_scale, g_col, g_op, g_bg, g_th = _backward(grad_out, mu, scale, color, opacity, bg, py, px, th, T,
-                                                           asum, fg, ctx.recs)
-        return g_mu, g_scale, g_col, g_op, g_bg, g_th, None, None
+        g_mu, g_scale, g_col, g_op, g_bg, g_th = _backward(grad_out, mu, scale, color, opacity, bg, py, px, theta, T,
+                                                           asum, fg, ctx.recs, *ctx.opts)
+        return g_mu, g_scale, g_col, g_op, g_bg, g_th, None, None, None, None
 
 
 # ----------------------------------------------------------------------------------------------- public API
@@ -1239,14 +1254,12 @@ def render_alpha_full_triton(mu, log_scale, color, opacity, bg, H, W, theta=None
     if cull:
         scale, is_log = _scale_arg(log_scale)
         return _AlphaRenderCull.apply(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, odds, is_log)
-    else:
-        scale = activate_scale(log_scale)
-        if odds:
-            raise NotImplementedError("odds compositing is only wired through the cull/octave path; "
-                                      "use cull=True or render_alpha_octave")
-        pyx = _pixels(H, W, mu.device, torch.float32)
-        out = _AlphaRender.apply(mu, scale, color, opacity, bg, theta, pyx[:, 0].contiguous(),
-                                 pyx[:, 1].contiguous())
+    if odds:
+        raise NotImplementedError("odds compositing is only wired through the cull/octave path; "
+                                  "use cull=True or render_alpha_octave")
+    scale, is_log = _scale_arg(log_scale)
+    ys, xs = _pixel_axes(H, W, mu.device, torch.float32)
+    out = _AlphaRender.apply(mu, scale, color, opacity, bg, theta, ys, xs, W, is_log)
     return out.reshape(B, H, W, C).permute(0, 3, 1, 2)
 
 

@@ -251,6 +251,30 @@ int splat_exact_bwd(const float *rec, int N, int C, const float *py, const float
                     float *g_scale, float *g_theta, float *g_op, float *g_color, float *g_bg, void *ws,
                     size_t ws_bytes, void *stream);
 
+/* The exact path over a pixel list (grid_w = 0: py[P], px[P]) or a grid of P / grid_w rows of grid_w pixels
+ * (py[P / grid_w] row centres, px[grid_w] column centres). splat_decode_exact also writes `reach`
+ * (splat_exact_reach_bytes: per splat the box outside which its falloff is zero in float32, then the unions of every
+ * 64 splats); with it the kernels leave out the pixel-pairs whose every term is an exact zero. `reach` may be NULL, and
+ * the forward's workspace too (the splats are then split over one workgroup per 64 pixels only). With
+ * SPLAT_FLAG_LOG_SCALE `scale` holds raw log-scales, and log_scale[N,2] (or NULL) makes g_scale w.r.t. them. */
+size_t splat_exact_reach_bytes(int N);
+int splat_decode_exact(const float *mu, const float *scale, const float *theta, const float *opacity,
+                       const float *color, int C, int N, int flags, float *rec, float *reach, void *stream);
+/* Order of a pixel list for the kernels below (order[P], the rest of the buffer is scratch): pixels that are close
+ * together come together. splat_exact_order_bytes is 0 where the list is better taken as it is (order = NULL). */
+size_t splat_exact_order_bytes(int N, int P);
+int splat_exact_order(const float *py, const float *px, int N, int P, int *order, size_t order_bytes, void *stream);
+size_t splat_exact_fwd_workspace_bytes(int N, int C, int P, int grid_w);
+int splat_exact_render(const float *rec, const float *reach, int N, int C, const float *py, const float *px, int P,
+                       int grid_w, const int *order, const float *bg, float *out, float *T, float *asum, float *fg,
+                       void *ws, size_t ws_bytes, void *stream);
+size_t splat_exact_render_bwd_workspace_bytes(int N, int C, int P, int grid_w);
+int splat_exact_render_bwd(const float *rec, const float *reach, int N, int C, const float *py, const float *px,
+                           int P, int grid_w, const int *order, const float *bg, const float *T, const float *asum,
+                           const float *fg, const float *gout, const float *log_scale, float *g_mu, float *g_scale,
+                           float *g_theta, float *g_op, float *g_color, float *g_bg, void *ws, size_t ws_bytes,
+                           void *stream);
+
 #ifdef __cplusplus
 }
 #endif
