@@ -93,11 +93,12 @@ __device__ __forceinline__ float4 splat_reach(float2 m, float2 s, float cs, floa
             : make_float4(-INFINITY, INFINITY, -INFINITY, INFINITY);
 }
 
-template <int C>
+// BIN: the binning's count pass; else the records and, with `reach`, the reach boxes (exact path).
+template <int C, bool BIN>
 __global__ __launch_bounds__(kBlock) void k_decode_count(
     const float* __restrict__ mu, const float* __restrict__ scale, const float* __restrict__ theta,
     const float* __restrict__ opacity, const float* __restrict__ color, int N, LevelTable L, Routing R, float fT,
-    float cutoff, int do_bin, int act, float4* __restrict__ rec, int4* __restrict__ rect, int* __restrict__ counts,
+    float cutoff, int act, float4* __restrict__ rec, int4* __restrict__ rect, int* __restrict__ counts,
     long long* __restrict__ block_sums, int2* __restrict__ rowhist, int nb, float4* __restrict__ reach) {
   __shared__ long long s_part[kWaves];
   __shared__ int s_lev[kMaxLevels];
@@ -108,7 +109,7 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
   // float4 k of splat t of the block sits at s_rec[4 t + (k ^ ((t >> 2) & 3))]: 16 consecutive lanes then write
   // 16 different 16-byte bank groups (slot mod 16) and read back 16 consecutive slots
   auto rec_slot = [](int t, int k) { return 4 * t + (k ^ ((t >> 2) & 3)); };
-  if (do_bin) {
+  if (BIN) {
     for (int i = threadIdx.x; i < kMaxLevels; i += kBlock) s_lev[i] = 0;
     if (rowhist)
       for (int i = threadIdx.x; i <= nrows; i += kBlock) {
@@ -143,11 +144,11 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
     s_rec[rec_slot(t, 1)] = make_float4(-sn * kx, cs * kx, op, log2f(op));
     s_rec[rec_slot(t, 2)] = col;
     s_rec[rec_slot(t, 3)] = make_float4(s.x, s.y, cs, sn);
-    if (reach) {
+    if (!BIN && reach) {
       box = splat_reach(m, s, cs, sn, op, col);
       reach[g] = box;
     }
-    if (do_bin) {
+    if (BIN) {
       // level: render_triton.py:925-932 + 950-952 (octave), :904-913 (coarse/fine split)
       if (R.mode == 1) {
         const float px = fmaxf(s.x, s.y) * R.rep;
@@ -155,6 +156,8 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
         lev = (int)fminf(fmaxf(o, 0.f), (float)R.max_oct);
       } else if (R.mode == 2) {
         lev = g < R.n_coarse ? 1 : 0;
+      } else if (R.mode == 3) {
+        lev = min(g / R.n_coarse, L.n - 1);
       }
       const float fH = (float)L.H[lev], fW = (float)L.W[lev];
       const float xmax = (float)(L.ntx[lev] - 1);
@@ -185,7 +188,7 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
       }
     }
   }
-  if (do_bin) {   // per-level pair sums: one LDS atomic per level present in the wave (lanes of a level summed)
+  if (BIN) {   // per-level pair sums: one LDS atomic per level present in the wave (lanes of a level summed)
     const int lane = threadIdx.x & 63;
     for (unsigned long long rem = __ballot(cnt != 0); rem;) {
       const int l0 = __shfl(lev, __ffsll((long long)rem) - 1, 64);
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
     float4* dst = rec + (size_t)blockIdx.x * kBlock * 4;
     for (int i = threadIdx.x; i < nrec; i += kBlock) dst[i] = s_rec[rec_slot(i >> 2, i & 3)];
   }
-  if (!do_bin) {
+  if (!BIN) {
     if (reach) {   // the union of every 64 splats' boxes, behind the splats' own
 #pragma unroll
       for (int msk = 32; msk >= 1; msk >>= 1) {
@@ -1572,7 +1575,7 @@ int splat_decode_exact(const float* mu, const float* scale, const float* theta, 
   LevelTable L{};
   Routing R{};
 #define SPLAT_DECODE(CC)                                                                                      \
-  k_decode_count<CC><<<nb, kBlock, 0, st>>>(mu, scale, theta, opacity, color, N, L, R, 1.f, 0.f, 0,          \
+  k_decode_count<CC, false><<<nb, kBlock, 0, st>>>(mu, scale, theta, opacity, color, N, L, R, 1.f, 0.f,     \
                                             (flags & kFlagLogScale) ? 1 : 0, reinterpret_cast<float4*>(rec), \
                                             nullptr, nullptr, nullptr, nullptr, 0,                           \
                                             reinterpret_cast<float4*>(reach))
@@ -1630,7 +1633,7 @@ int bin_count_launch(const float* mu, const float* scale, const float* theta, co
   int2* rowhist = cp.rows ? (int2*)((char*)ws + cp.off_rowhist) : nullptr;
   int2* rtot = cp.rows ? (int2*)((char*)ws + cp.off_rtot) : nullptr;
 #define SPLAT_DC(CC)                                                                                         \
-  k_decode_count<CC><<<nb, kBlock, 0, st>>>(mu, scale, theta, opacity, color, N, L, R, (float)TILE, cutoff, 1, \
+  k_decode_count<CC, true><<<nb, kBlock, 0, st>>>(mu, scale, theta, opacity, color, N, L, R, (float)TILE, cutoff, \
                                             (flags & kFlagLogScale) ? 1 : 0,                                \
                                             reinterpret_cast<float4*>(rec), reinterpret_cast<int4*>(rect), \
                                             offsets, sums, rowhist, nb, nullptr)

@@ -216,17 +216,18 @@ __device__ __forceinline__ void add_coarse(const LevelTable& L, int yp, int xp, 
   }
 }
 
-// A global tile, its level and coordinates.
+// A global tile, its level and coordinates, its number within the level and the level's first pixel slot.
 struct TileAt {
-  int t, l, tx, ty, H, W;
+  int t, l, tx, ty, H, W, lt, pb;
 };
 __device__ __forceinline__ TileAt tile_of(const LevelTable& L, int t, int l) {
   TileAt a;
   a.t = t;
   a.l = l;
-  const int lt = a.t - L.tbase[a.l];
-  a.ty = lt / L.ntx[a.l];
-  a.tx = lt - a.ty * L.ntx[a.l];
+  a.lt = a.t - L.tbase[a.l];
+  a.pb = L.pbase[a.l];
+  a.ty = a.lt / L.ntx[a.l];
+  a.tx = a.lt - a.ty * L.ntx[a.l];
   a.H = L.H[a.l];
   a.W = L.W[a.l];
   return a;
@@ -296,12 +297,18 @@ __host__ __device__ constexpr int fwd_split() { return TILE == 8 ? (WIDE ? 16 : 
 template <int TILE, int S>
 __host__ __device__ constexpr int fwd_threads() { return tile_threads(TILE) * S; }
 
-template <int C, bool FIELDS, bool ODDS, bool UPS, int TILE, int S>
+// What a composite launch renders: level 0 alone, level 0 with the coarse levels' upsampled fields added, or the images
+// of a batch (one level each). The batch is a variant of its own: the image's number and offset, kept over the pair loop
+// next to the records' scalar registers, cost a single image 56.5 against 53.8 us at 768 x 768.
+enum Composite : int { kPlain = 0, kUps = 1, kBatch = 2 };
+
+template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S>
 __global__ __launch_bounds__((fwd_threads<TILE, S>())) void k_fwd_cull(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L, int tb0,
     int ntiles, const float* __restrict__ bg, float* __restrict__ out, float* __restrict__ Tout,
     float* __restrict__ asum_out, float* __restrict__ fg_out, float* __restrict__ slog, float* __restrict__ sa,
     float* __restrict__ sac) {
+  constexpr bool UPS = MODE == kUps, BATCH = MODE == kBatch;
   constexpr int NW = fwd_threads<TILE, S>() / 64;   // waves per workgroup
   __shared__ float2 s_uv[NW][64];
   const TileAt ta = tile_at(L, tb0, ntiles);
@@ -343,9 +350,10 @@ __global__ __launch_bounds__((fwd_threads<TILE, S>())) void k_fwd_cull(
     }
   }
   if (!valid) return;
-  const int p = yp * ta.W + xp;
+  const int p = (BATCH ? ta.pb : 0) + yp * ta.W + xp;
+  if (BATCH) bg += ta.l * C;
   if (FIELDS) {
-    const size_t pp = (size_t)L.pbase[ta.l] + p;
+    const size_t pp = (size_t)ta.pb + p;
     slog[pp] = sl * kLn2;
     sa[pp] = s_a;
 #pragma unroll
@@ -982,9 +990,13 @@ __device__ __forceinline__ PairSums<C> careful_pair(const float* __restrict__ re
   return s;
 }
 
+// Floats between two images' background partials: each starts 16-byte aligned, as a single image's do (block_bg_sum then
+// adds them in the same order).
+__host__ __device__ constexpr int bg_stride(int C, int ntiles) { return (C * ntiles + 3) & ~3; }
+
 // Backward over the tiles [tb0, tb0 + ntiles) of the level table (levels without pairs are skipped).
-// Composite (level 0): upstream from T/asum/fg/gout (see pixel_upstream for UPS); per-tile partials of
-// sum_p gout * T go to bg_part[c * ntiles + (t - tb0)]. FIELDS: upstream from the packed fields.
+// Composite (level 0, or the images of a batch): upstream from T/asum/fg/gout (see pixel_upstream for UPS); per-tile
+// partials of sum_p gout * T go to bg_part[l bg_stride + c * ntiles + t] for tile t of level l. FIELDS: upstream from the packed fields.
 // S waves per tile (S = 1, or 16 with kFlagWide for few tiles with long pair lists: the dense coarse levels of
 // an octave render): the per-pixel upstream terms are staged in LDS once for the tile, then each wave takes a
 // contiguous share of the tile's pair list (every pair's sums are independent) 64 at a time (lane = pair) in
@@ -994,7 +1006,7 @@ __device__ __forceinline__ PairSums<C> careful_pair(const float* __restrict__ re
 // sums are combined with xor shuffles. At 5 waves per SIMD (at most 96 VGPRs, no spills) there are enough waves
 // to cover the latency of the VALU, LDS and transcendental pipes.
 // SPLIT (FIELDS only, S = 1): workgroup = a work item of the SplitTable, the item's chunk of its tile's pairs.
-template <int C, bool FIELDS, bool ODDS, bool UPS, int TILE, int S, bool SPLIT = false>
+template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S, bool SPLIT = false>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_cull(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L, int tb0,
     int ntiles, const float* __restrict__ bg, const float* __restrict__ Tin, const float* __restrict__ asum_in,
@@ -1002,6 +1014,7 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
     float* __restrict__ dsa, float* __restrict__ dsac, const int* __restrict__ pair_q, float* __restrict__ psum,
     float* __restrict__ bg_part, SplitTable P) {
   static_assert(!SPLIT || (FIELDS && S == 1), "split items: FIELDS backward, one wave per item");
+  constexpr bool UPS = MODE == kUps, BATCH = MODE == kBatch;
   constexpr int NP = TILE * TILE;
   __shared__ float4 s_up4[TILE * UpRows<TILE>::RF / 4];
   const UpRows<TILE> ups{reinterpret_cast<float*>(s_up4)};
@@ -1021,8 +1034,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
     float4 pa = make_float4(0.f, 0.f, 0.f, 0.f);
     float2 pb = make_float2(0.f, 0.f);
     if (yp < ta.H && xp < ta.W) {
-      const int p = yp * ta.W + xp;
-      pixel_upstream<C, FIELDS, UPS>(p, (size_t)L.pbase[ta.l] + p, bg, Tin, asum_in, fg_in, gout, dslog, dsa, dsac,
+      const int p = (BATCH ? ta.pb : 0) + yp * ta.W + xp;
+      pixel_upstream<C, FIELDS, UPS>(p, (size_t)ta.pb + p, BATCH ? bg + ta.l * C : bg, Tin, asum_in, fg_in, gout, dslog, dsa, dsac,
                                      pa, pb, bgp);
     }
     ups.put(l / TILE, l % TILE, pa, pb);
@@ -1038,7 +1051,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
     if (threadIdx.x < C) {
       float v = 0.f;
       for (int w = 0; w < S; ++w) v += s_bgw[w][threadIdx.x];
-      bg_part[(size_t)threadIdx.x * ntiles + (t - tb0)] = v;
+      const int nt = BATCH ? L.tbase[1] : ntiles;
+      bg_part[(BATCH ? (size_t)ta.l * bg_stride(C, nt) : 0) + (size_t)threadIdx.x * nt + ta.lt] = v;
     }
   }
   // the tile's pixel centres (render_triton.py:455-456): rows and columns in LDS, columns also wave-uniform
@@ -1252,8 +1266,8 @@ __device__ __forceinline__ void zero_grads(int g, float* __restrict__ g_mu, floa
 // the group's partial sums are combined by a fixed xor tree. A splat with more than kLightPairs pairs is
 // left out of that loop and summed afterwards by its whole wave (lane-strided partial sums, then a fixed
 // xor tree), so one heavy splat does not serialise its wave. The order of every addition is fixed:
-// deterministic. Splats with no pair (none for valid rects) get zeros. With g_bg set, the grid's first
-// workgroup sums the per-tile background partials instead.
+// deterministic. Splats with no pair (none for valid rects) get zeros. The grid's first `images` workgroups (0: none)
+// sum the images' per-tile background partials instead.
 // Measured at C2 (about 20 records per splat) and C4: 8 lanes per splat 17.2 us and 261 us per launch, against 18.1
 // and 265 with 4 lanes, 20.9 and 278 with 2, 19.9 and 270 with 16; with 8 lanes, 2 loads in flight instead of 4
 // 18.1 and 284 us. Splats of more than 128 pairs go to the whole-wave path: 16.3 us at C2 against 17.2 with 64
@@ -1288,17 +1302,17 @@ __global__ __launch_bounds__(256) void k_splat_sum(const float* __restrict__ rec
                                                    const int* __restrict__ offsets, int N, float* __restrict__ g_mu,
                                                    float* __restrict__ g_scale, float* __restrict__ g_theta,
                                                    float* __restrict__ g_op, float* __restrict__ g_col,
-                                                   const float* __restrict__ bg_part, int nparts,
+                                                   const float* __restrict__ bg_part, int nparts, int images,
                                                    float* __restrict__ g_bg, const float* __restrict__ lsc) {
   constexpr int R = pair_rec<C>();
   constexpr int kPerBlock = 256 / kSumLanes;
-  if (g_bg && blockIdx.x == 0) {   // first, so it overlaps the splat waves
-    block_bg_sum<C>(bg_part, nparts, g_bg);
+  if ((int)blockIdx.x < images) {   // first, so they overlap the splat waves
+    block_bg_sum<C>(bg_part + (size_t)blockIdx.x * bg_stride(C, nparts), nparts, g_bg + blockIdx.x * C);
     return;
   }
   const int lane = threadIdx.x & 63;
   const int r = lane % kSumLanes;
-  const int g = (blockIdx.x - (g_bg ? 1 : 0)) * kPerBlock + (int)threadIdx.x / kSumLanes;
+  const int g = ((int)blockIdx.x - images) * kPerBlock + (int)threadIdx.x / kSumLanes;
   int q0 = 0, q1 = 0;
   if (g < N) {
     q0 = offsets[g];
@@ -1333,17 +1347,17 @@ __global__ __launch_bounds__(256) void k_splat_sum(const float* __restrict__ rec
     zero_grads<C>(g, g_mu, g_scale, g_theta, g_op, g_col);
 }
 
-// Zero gradients for every splat (a render with no pairs), plus g_bg from the partials in the first block.
+// Zero gradients for every splat (a render with no pairs), plus g_bg from the partials in the first blocks.
 template <int C>
 __global__ __launch_bounds__(256) void k_zero_grads(int N, float* __restrict__ g_mu, float* __restrict__ g_scale,
                                                     float* __restrict__ g_theta, float* __restrict__ g_op,
                                                     float* __restrict__ g_col, const float* __restrict__ bg_part,
-                                                    int nparts, float* __restrict__ g_bg) {
-  if (g_bg && blockIdx.x == 0) {
-    block_bg_sum<C>(bg_part, nparts, g_bg);
+                                                    int nparts, int images, float* __restrict__ g_bg) {
+  if ((int)blockIdx.x < images) {
+    block_bg_sum<C>(bg_part + (size_t)blockIdx.x * bg_stride(C, nparts), nparts, g_bg + blockIdx.x * C);
     return;
   }
-  const int g = (blockIdx.x - (g_bg ? 1 : 0)) * 256 + threadIdx.x;
+  const int g = ((int)blockIdx.x - images) * 256 + threadIdx.x;
   if (g < N) zero_grads<C>(g, g_mu, g_scale, g_theta, g_op, g_col);
 }
 
@@ -2177,9 +2191,10 @@ int with_tile(int TILE, F&& f) {
   return set_error(kUnsupported, "TILE=%d not supported (4, 8 or 16)", TILE);
 }
 
-// FIELDS, ODDS, UPS (UPS only with the composite: the caller rejects FIELDS | UPS).
+// FIELDS, ODDS and the composite's mode (kPlain with FIELDS: launch_levels rejects FIELDS | UPS and both with a batch).
 template <typename F>
-int with_flags(int flags, F&& f) {
+int with_flags(int flags, const splat_levels* lv, F&& f) {
+  if (lv && lv->mode == 3) return flags & kFlagOdds ? f(IC<0>{}, IC<1>{}, IC<kBatch>{}) : f(IC<0>{}, IC<0>{}, IC<kBatch>{});
   switch (flags & 7) {
     case 0: return f(IC<0>{}, IC<0>{}, IC<0>{});
     case 1: return f(IC<1>{}, IC<0>{}, IC<0>{});
@@ -2198,7 +2213,9 @@ static int launch_levels(const char* who, int H, int W, int TILE, const splat_le
   if (make_levels(H, W, TILE, lv, L, nullptr)) return set_error(kInvalid, "%s: bad levels for H=%d W=%d", who, H, W);
   if (lev_begin < 0 || lev_end > L->n || lev_begin >= lev_end)
     return set_error(kInvalid, "%s: levels [%d, %d) outside [0, %d)", who, lev_begin, lev_end, L->n);
-  if (!(flags & kFlagFields) && (lev_begin != 0 || lev_end != 1))
+  const bool batch = lv && lv->mode == 3;
+  if (batch && (flags & (kFlagFields | kFlagUps))) return set_error(kInvalid, "%s: a batch renders its composites", who);
+  if (!(flags & kFlagFields) && !batch && (lev_begin != 0 || lev_end != 1))
     return set_error(kInvalid, "%s: the composite renders level 0 only", who);
   L->mask = levmask & L->mask;
   *tb0 = L->tbase[lev_begin];
@@ -2262,9 +2279,10 @@ int splat_render_fwd(const float* rec, const int* gid_sorted, const int* tile_st
   hipStream_t st = (hipStream_t)stream;
   return with_c(C, [&](auto cc) {
     return with_tile(TILE, [&](auto tt) {
-      return with_flags(flags, [&](auto fl, auto od, auto up) {
+      return with_flags(flags, lv, [&](auto fl, auto od, auto up) {
         constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
-        constexpr bool FL = decltype(fl)::value != 0, OD = decltype(od)::value != 0, UP = decltype(up)::value != 0;
+        constexpr bool FL = decltype(fl)::value != 0, OD = decltype(od)::value != 0;
+        constexpr int UP = decltype(up)::value;
         if (TT == 8 && (flags & kFlagWide)) {
           constexpr int S = fwd_split<TT, true>();
           launch_tile_kernel(k_fwd_cull<CC, FL, OD, UP, TT, S>, ntiles, fwd_threads<TT, S>(), st, rec, gid_sorted,
@@ -2304,9 +2322,10 @@ int splat_render_bwd(const float* rec, const int* gid_sorted, const int* tile_st
   hipStream_t st = (hipStream_t)stream;
   return with_c(C, [&](auto cc) {
     return with_tile(TILE, [&](auto tt) {
-      return with_flags(flags, [&](auto fl, auto od, auto up) {
+      return with_flags(flags, lv, [&](auto fl, auto od, auto up) {
         constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
-        constexpr bool FL = decltype(fl)::value != 0, OD = decltype(od)::value != 0, UP = decltype(up)::value != 0;
+        constexpr bool FL = decltype(fl)::value != 0, OD = decltype(od)::value != 0;
+        constexpr int UP = decltype(up)::value;
         if (TT == 8 && (flags & kFlagWide))
           launch_tile_kernel(k_bwd_cull<CC, FL, OD, UP, TT, 16>, ntiles, 64 * 16, st, rec, gid_sorted, tile_starts, L,
                              tb0, ntiles, bg, T, asum, fg, gout, dslog, dsa, dsac, pair_q, pair_sums, bg_part,
@@ -2432,11 +2451,11 @@ int splat_render_fields_split_bwd(const float* rec, const int* gid_sorted, const
     return with_tile(TILE, [&](auto tt) {
       constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
       if (flags & kFlagOdds)
-        launch_tile_kernel(k_bwd_cull<CC, true, true, false, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
+        launch_tile_kernel(k_bwd_cull<CC, true, true, kPlain, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
                            tile_starts, L, 0, nitems, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
                            pair_q, pair_sums, nullptr, P);
       else
-        launch_tile_kernel(k_bwd_cull<CC, true, false, false, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
+        launch_tile_kernel(k_bwd_cull<CC, true, false, kPlain, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
                            tile_starts, L, 0, nitems, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
                            pair_q, pair_sums, nullptr, P);
       return check_launch("k_bwd_cull(split)");
@@ -2459,7 +2478,7 @@ size_t splat_upsample_adjoint_workspace_bytes(int C, int H, int W, int TILE, con
 int splat_upsample_adjoint(int C, int H, int W, int TILE, const splat_levels* lv, unsigned levmask, float* dslog,
                            float* dsa, float* dsac, void* ws, size_t ws_bytes, void* stream) {
   LevelTable L;
-  if (C < 1 || C > kMaxC || H < 1 || W < 1 || make_levels(H, W, TILE, lv, &L, nullptr))
+  if (C < 1 || C > kMaxC || H < 1 || W < 1 || (lv && lv->mode == 3) || make_levels(H, W, TILE, lv, &L, nullptr))
     return set_error(kInvalid, "splat_upsample_adjoint: C=%d H=%d W=%d or bad levels", C, H, W);
   if (!dslog || !dsa || !dsac) return set_error(kInvalid, "splat_upsample_adjoint: null fields");
   L.mask = levmask & L.mask & ~1u;
@@ -2486,26 +2505,33 @@ int splat_upsample_adjoint(int C, int H, int W, int TILE, const splat_levels* lv
   });
 }
 
-int splat_reduce_pairs(const float* rec, const int* offsets, const int* pair_splat, long long tot,
-                       int N, int C, const float* pair_sums, const float* bg_part, int nparts, const float* log_scale,
-                       float* g_mu, float* g_scale, float* g_theta, float* g_op, float* g_color, float* g_bg, void* stream) {
-  if (N < 0 || tot < 0 || tot > 0x7fffffffLL - 64 || (N == 0 && tot > 0))
-    return set_error(kInvalid, "splat_reduce_pairs: N=%d tot=%lld", N, tot);
+int splat_reduce_images(const float* rec, const int* offsets, long long tot, int N, int C, const float* pair_sums,
+                        const float* bg_part, int nparts, int images, const float* log_scale, float* g_mu,
+                        float* g_scale, float* g_theta, float* g_op, float* g_color, float* g_bg, void* stream) {
+  if (N < 0 || tot < 0 || tot > 0x7fffffffLL - 64 || (N == 0 && tot > 0) || images < 1)
+    return set_error(kInvalid, "splat_reduce_pairs: N=%d tot=%lld images=%d", N, tot, images);
   if ((N > 0 && (!rec || !offsets || !g_mu || !g_scale || !g_op || !g_color)) ||
       (tot > 0 && !pair_sums) || (g_bg && (!bg_part || nparts < 1)))
     return set_error(kInvalid, "splat_reduce_pairs: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  const unsigned extra = g_bg ? 1u : 0u;
+  const int extra = g_bg ? images : 0;
   return with_c(C, [&](auto cc) {
     constexpr int CC = decltype(cc)::value;
     if (tot > 0)
-      k_splat_sum<CC><<<(unsigned)((N + 256 / kSumLanes - 1) / (256 / kSumLanes)) + extra, 256, 0, st>>>(
-          rec, pair_sums, offsets, N, g_mu, g_scale, g_theta, g_op, g_color, bg_part, nparts, g_bg, log_scale);
+      k_splat_sum<CC><<<(unsigned)((N + 256 / kSumLanes - 1) / (256 / kSumLanes) + extra), 256, 0, st>>>(
+          rec, pair_sums, offsets, N, g_mu, g_scale, g_theta, g_op, g_color, bg_part, nparts, extra, g_bg, log_scale);
     else if (N > 0 || g_bg)
-      k_zero_grads<CC><<<(unsigned)((N + 255) / 256) + extra, 256, 0, st>>>(N, g_mu, g_scale, g_theta, g_op,
-                                                                            g_color, bg_part, nparts, g_bg);
+      k_zero_grads<CC><<<(unsigned)((N + 255) / 256 + extra), 256, 0, st>>>(N, g_mu, g_scale, g_theta, g_op, g_color,
+                                                                            bg_part, nparts, extra, g_bg);
     return check_launch("splat_reduce_pairs");
   });
+}
+
+int splat_reduce_pairs(const float* rec, const int* offsets, const int* pair_splat, long long tot,
+                       int N, int C, const float* pair_sums, const float* bg_part, int nparts, const float* log_scale,
+                       float* g_mu, float* g_scale, float* g_theta, float* g_op, float* g_color, float* g_bg, void* stream) {
+  return splat_reduce_images(rec, offsets, tot, N, C, pair_sums, bg_part, nparts, 1, log_scale, g_mu, g_scale, g_theta,
+                             g_op, g_color, g_bg, stream);
 }
 
 namespace {

@@ -141,11 +141,11 @@ struct LevelTable {
 
 // Splat -> level routing, evaluated in the decode pass.
 struct Routing {
-  int mode;         // 0 single level, 1 octave by scale, 2 split by index
+  int mode;         // 0 single level, 1 octave by scale, 2 split by index, 3 one level per image
   int max_oct;      // mode 1
   float rep;        // mode 1: float(min(H, W))
   float inv_base;   // mode 1: fp32 1 / base_texels (a tensor divided by a CPU scalar is a multiply by its reciprocal)
-  int n_coarse;     // mode 2: splats [0, n_coarse) are level 1
+  int n_coarse;     // mode 2: splats [0, n_coarse) are level 1; mode 3: splats per image
 };
 
 // Level of global tile row r.
@@ -185,10 +185,11 @@ __device__ __forceinline__ int bilinear_src(int d, int in, float scale, int* p1,
 extern "C" {
 // C-ABI description of the levels of a render (mirrors include/splat_render.h).
 typedef struct splat_levels {
-  int mode;           // 0 single level (H, W); 1 octave routing; 2 coarse/fine split by index
-  int max_octaves;    // mode 1: levels 0..max_octaves, level o on (max(8, H >> o), max(8, W >> o))
+  int mode;           // 0 single level (H, W); 1 octave routing; 2 coarse/fine split by index; 3 a batch of images
+  int max_octaves;    // mode 1: levels 0..max_octaves, level o on (max(8, H >> o), max(8, W >> o)); mode 3: images
   float base_texels;  // mode 1: o = clamp(ceil(log2(max(max(sy, sx) * min(H, W) / base_texels, 1e-6))), 0, max_octaves)
-  int n_coarse;       // mode 2: splats [0, n_coarse) render on (coarse_H, coarse_W) as level 1, the rest on (H, W)
+  int n_coarse;       // mode 2: splats [0, n_coarse) render on (coarse_H, coarse_W) as level 1, the rest on (H, W);
+                      // mode 3: splats [l n_coarse, (l + 1) n_coarse) are image l, level l, on its own (H, W)
   int coarse_H, coarse_W;
 } splat_levels;
 }
@@ -224,6 +225,14 @@ inline int make_levels(int H, int W, int TILE, const splat_levels* lv, LevelTabl
     t.n = 2;
     t.H[0] = H; t.W[0] = W;
     t.H[1] = lv->coarse_H; t.W[1] = lv->coarse_W;
+    r.n_coarse = lv->n_coarse;
+  } else if (mode == 3) {
+    if (lv->max_octaves < 1 || lv->max_octaves > kMaxLevels || lv->n_coarse < 1) return 1;
+    if ((long long)H * W * lv->max_octaves > 0x7fffffffLL) return 1;   // pixel slots are 32-bit
+    t.n = lv->max_octaves;
+    for (int l = 0; l < t.n; ++l) {
+      t.H[l] = H; t.W[l] = W;
+    }
     r.n_coarse = lv->n_coarse;
   } else {
     return 1;

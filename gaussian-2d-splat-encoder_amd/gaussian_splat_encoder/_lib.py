@@ -23,7 +23,8 @@ _LL = ctypes.c_longlong
 
 
 class SplatLevels(ctypes.Structure):
-    """struct splat_levels: mode 0 single canvas, 1 octave routing, 2 coarse/fine split by index."""
+    """struct splat_levels: mode 0 single canvas, 1 octave routing, 2 coarse/fine split by index, 3 a batch of
+    `max_octaves` images of `n_coarse` splats each."""
     _fields_ = [("mode", _I), ("max_octaves", _I), ("base_texels", _F), ("n_coarse", _I),
                 ("coarse_H", _I), ("coarse_W", _I)]
 
@@ -61,6 +62,7 @@ _SIGS = {
     "splat_upsample_adjoint_workspace_bytes": (_SZ, [_I, _I, _I, _I, _LV]),
     "splat_upsample_adjoint": (_I, [_I, _I, _I, _I, _LV, _U, _VP, _VP, _VP, _VP, _SZ, _VP]),
     "splat_reduce_pairs": (_I, [_VP, _VP, _VP, _LL, _I, _I, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP]),
+    "splat_reduce_images": (_I, [_VP, _VP, _LL, _I, _I, _VP, _VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP]),
     "splat_exact_fwd": (_I, [_VP, _I, _I, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP]),
     "splat_exact_bwd_workspace_bytes": (_SZ, [_I, _I, _I]),
     "splat_exact_bwd": (_I, [_VP, _I, _I, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,

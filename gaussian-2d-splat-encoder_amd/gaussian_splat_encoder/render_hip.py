@@ -224,6 +224,11 @@ class TileBins:
         return self.gid_b, self.starts_b, self.ntx, self.nt
 
     @property
+    def n_images(self):
+        """Images that share this binning (a merged batch, one level each), else 1."""
+        return self.lv.max_octaves if self.lv is not None and self.lv.mode == 3 else 1
+
+    @property
     def n_levels(self):
         return 1 if self.geom is None else len(self.geom)
 
@@ -572,6 +577,31 @@ def _composite_buffers(B, P, C, dev):
             t.as_strided((B, P), (P, 1), n * (C + 1)), t.as_strided((B, P, C), (P * C, C, 1), n * (C + 2)))
 
 
+_MAX_ROWS = 1024   # tile rows of a level table that the binning's row plan takes
+
+
+def _batch_levels(B, N, H, W, TILE):
+    """The level table that renders a batch of B images as one (every image a level, each launch covering all of them),
+    or None: one image, or more than a level table or the row plan holds (the images then go one after another)."""
+    if 1 < B <= _lib.MAX_LEVELS and N > 0 and B * -(-H // TILE) <= _MAX_ROWS and B * H * W < 1 << 30 and B * N < 1 << 27:
+        return SplatLevels(3, B, 0.0, N, 0, 0)
+    return None
+
+
+def _flat_batch(t):
+    """[B, N, ...] as one image's [1, B N, ...] (None stays None)."""
+    return None if t is None else _f32(t).view(1, -1, *t.shape[2:])
+
+
+def _wide_launches(bins, tots):
+    """[(flags, (first level, last level + 1))]: the tile launches of the images in a merged batch, one for all of them
+    when they take the same number of waves per tile."""
+    w = [_wide(bins.TILE, bins.ntiles0, t) for t in tots]
+    if all(x == w[0] for x in w):
+        return [(w[0], (0, len(w)))]
+    return [(x, (b, b + 1)) for b, x in enumerate(w)]
+
+
 def _forward_cull(mu, scale, color, opacity, bg, theta, H, W, TILE=8, cutoff=3.0, max_pairs=None, odds=False,
                   with_maps=True, scale_is_log=False, plan=None):
     """Composite forward (render_triton.py:538-567): out [B,P,C], (T, asum, fg), bins. plan: a _BwdPlan to
@@ -579,38 +609,51 @@ def _forward_cull(mu, scale, color, opacity, bg, theta, H, W, TILE=8, cutoff=3.0
     B, N, C = color.shape
     P = H * W
     dev = mu.device
-    bins = _bin(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, with_maps, scale_is_log=scale_is_log,
-                defer=True)
+    lv = _batch_levels(B, N, H, W, TILE) if B > 1 and max_pairs is None else None
+    if lv is not None:   # one binning and one launch per step for the whole batch
+        bins = _bin(_flat_batch(mu), _flat_batch(scale), _flat_batch(color), _flat_batch(opacity), _flat_batch(theta), H,
+                    W, TILE, cutoff, None, with_maps, lv, scale_is_log, True)
+    else:
+        bins = _bin(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, with_maps, scale_is_log=scale_is_log,
+                    defer=True)
     out, T, asum, fg = _composite_buffers(B, P, C, dev)
     bgf = _f32(bg)
     flags = FLAG_ODDS if odds else 0
     lib, stream = _lib.load(), _lib.stream_ptr(dev)
 
+    nt = bins.ntiles0
+
+    def launch_one(b, wide, lev, mask):
+        comp = (_bptr(bgf, b), _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b))
+        if not kernel_timer.enabled:
+            return _render_fwd(lib, bins, b, C, flags | wide, lev, mask, comp, (None,) * 3, stream)
+        ev = kernel_timer.record("fwd")
+        try:
+            _render_fwd(lib, bins, b, C, flags | wide, lev, mask, comp, (None,) * 3, stream)
+        finally:
+            kernel_timer.close("fwd", ev)
+
     def launch(tots):
-        for b in range(B):
-            comp = (_bptr(bgf, b), _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b))
-            if not kernel_timer.enabled:
-                _render_fwd(lib, bins, b, C, flags | _wide(TILE, bins.nt, tots[b]), (0, 1), 1, comp, (None,) * 3,
-                            stream)
-                continue
-            ev = kernel_timer.record("fwd")
-            try:
-                _render_fwd(lib, bins, b, C, flags | _wide(TILE, bins.nt, tots[b]), (0, 1), 1, comp, (None,) * 3,
-                            stream)
-            finally:
-                kernel_timer.close("fwd", ev)
+        if lv is None:
+            for b in range(B):
+                launch_one(b, _wide(TILE, nt, tots[b]), (0, 1), 1)
+        else:
+            for wide, lev in _wide_launches(bins, tots):
+                launch_one(0, wide, lev, (1 << B) - 1)
 
     if bins.pending is not None:   # queued on the speculative pair list before the count is read
-        spec = _speculated_levels(bins)[0]
-        launch([spec])
+        spec = _speculated_levels(bins)
+        launch(spec)
         if plan is not None:         # the backward's buffers, allocated while the GPU works towards the count
             plan.allocate(bins, B, N, C, dev, lib, bins.pending.cap)
         # launched again when the pair phase was redone, or when the count asks for another number of waves per
         # tile than the speculated one (they group the per-pixel sums: the image depends on the inputs alone)
-        if _finish(bins) or _wide(TILE, bins.nt, bins.tot_b[0]) != _wide(TILE, bins.nt, spec):
-            launch(bins.tot_b)
+        redone = _finish(bins)
+        tots = bins.tot_b if lv is None else bins.level_tot_b[0]
+        if redone or any(_wide(TILE, nt, t) != _wide(TILE, nt, s) for t, s in zip(tots, spec)):
+            launch(tots)
     else:
-        launch(bins.tot_b)
+        launch(bins.tot_b if lv is None else bins.level_tot_b[0])
     if plan is not None:
         plan.bind(bins, B, N, C, dev, lib, stream, flags, (bgf, T, asum, fg))
     return out, (T, asum, fg), bins
@@ -622,7 +665,7 @@ class _BwdPlan:
     of the two backward launches per image, complete but for the upstream gradient's pointer. The backward then runs
     two C-ABI calls per image (render_triton.py:723-765 in two kernels)."""
 
-    __slots__ = ("grads", "sums", "ns", "cap", "bwd_head", "bwd_tail", "red_args", "lsc", "has_th", "keep")
+    __slots__ = ("grads", "sums", "ns", "cap", "bwd_head", "bwd_tail", "red_args", "lsc", "has_th", "keep", "merged")
 
     def __init__(self, has_th, lsc=None):
         self.has_th = has_th
@@ -631,7 +674,7 @@ class _BwdPlan:
         self.sums = None
 
     def allocate(self, bins, B, N, C, dev, lib, cap):
-        """Gradient outputs and one buffer for the per-pair sums of every image (ns floats each, 16-byte aligned)
+        """Gradient outputs and one buffer for the per-pair sums of every binning (ns floats each, 16-byte aligned)
         followed by the per-tile background partials (the kernels take both by pointer)."""
         self.grads = _grads_bg_out(B, N, C, dev, self.has_th)
         ns = _SUMS_FLOATS.get(cap)
@@ -639,7 +682,8 @@ class _BwdPlan:
             if len(_SUMS_FLOATS) > 1024:
                 _SUMS_FLOATS.clear()
             ns = _SUMS_FLOATS[cap] = (lib.splat_pair_sums_bytes(max(cap, 1)) // 4 + 3) & ~3
-        self.sums = torch.empty(B * ns + C * bins.ntiles0, device=dev)
+        # a merged batch has one binning and a set of partials per image, else every image has its own in turn
+        self.sums = torch.empty(len(bins.tot_b) * ns + B * (C * bins.ntiles0 + 3), device=dev)
         self.ns = ns
         self.cap = cap
 
@@ -653,8 +697,17 @@ class _BwdPlan:
         self.keep = bgf   # the kernels read the background through its pointer
         lvr = None if bins.lv is None else _lib.ctypes.byref(bins.lv)
         sums0 = self.sums.data_ptr()
-        bgp = sums0 + 4 * B * ns
+        bgp = sums0 + 4 * len(tots) * ns
         self.bwd_head, self.bwd_tail, self.red_args = [], [], []
+        self.merged = bins.n_images > 1
+        if self.merged:
+            self.bwd_head = [(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), bins.p(0, "pq"), tots[0], C, bins.H,
+                              bins.W, bins.TILE, flags | w, lvr, *lev, (1 << B) - 1, ptr(bgf), ptr(T), ptr(asum), ptr(fg))
+                             for w, lev in _wide_launches(bins, bins.level_tot_b[0])]
+            self.bwd_tail = (None, None, None, sums0, bgp, stream)
+            self.red_args = (bins.p(0, "rec"), bins.p(0, "off"), tots[0], B * N, C, sums0, bgp, bins.ntiles0, B,
+                             ptr(self.lsc), ptr(g_mu), ptr(g_scale), ptr(g_th), ptr(g_op), ptr(g_col), ptr(g_bg), stream)
+            return
         for b in range(B):
             sb = sums0 + 4 * ns * b
             self.bwd_head.append((bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"), bins.p(b, "pq"), tots[b], C,
@@ -676,7 +729,19 @@ class _BwdPlan:
             go = grad_out.permute(0, 2, 3, 1).contiguous().float()
             g0 = go.data_ptr()
         timed = kernel_timer.enabled
-        for b in range(B):
+        if self.merged:
+            ev = kernel_timer.record("bwd") if timed else None
+            try:
+                for head in self.bwd_head:
+                    check(lib.splat_render_bwd(*head, g0, *self.bwd_tail), "splat_render_bwd")
+            finally:
+                kernel_timer.close("bwd", ev)
+            ev = kernel_timer.record("reduce") if timed else None
+            try:
+                check(lib.splat_reduce_images(*self.red_args), "splat_reduce_images")
+            finally:
+                kernel_timer.close("reduce", ev)
+        for b in range(0 if self.merged else B):
             if not timed:
                 check(lib.splat_render_bwd(*self.bwd_head[b], g0 + 4 * img * b, *self.bwd_tail[b]), "splat_render_bwd")
                 check(lib.splat_reduce_pairs(*self.red_args[b]), "splat_reduce_pairs")
@@ -843,6 +908,13 @@ def _backward_cull(grad_out, mu, scale, color, opacity, bg, theta, T, asum, fg, 
 
 def _backward_cull_raw(grad_out, bg, lsc, B, N, C, dev, has_th, T, asum, fg, bins, odds):
     """_backward_cull on what it reads: grad_out [B,P,C], bg, the raw log-scales lsc (or None) and shapes."""
+    if bins.n_images > 1:   # a merged batch
+        lib = _lib.load()
+        plan = _BwdPlan(has_th, lsc)
+        bgf = _f32(bg)
+        plan.bind(bins, B, N, C, dev, lib, _lib.stream_ptr(dev), FLAG_ODDS if odds else 0, (bgf, T, asum, fg))
+        go = grad_out.view(B, bins.H, bins.W, C).permute(0, 3, 1, 2)
+        return plan.run(lib, go, bins.H, bins.W, C)
     g_mu, g_scale, g_col, g_op, g_th, g_bg = _grads_bg_out(B, N, C, dev, has_th)
     grads = (g_mu, g_scale, g_col, g_op, g_th)
     go, bgf = _f32(grad_out), _f32(bg)

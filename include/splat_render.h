@@ -54,6 +54,10 @@ extern "C" {
  *     (8, 8) on share one level (their fields are summed after the same upsample); H, W <= 8 << 11.
  *   mode 2, coarse/fine split (render_triton.py:879-922): splats [0, n_coarse) render on
  *     (coarse_H, coarse_W) as level 1, the rest on (H, W).
+ *   mode 3, a batch of max_octaves images (1..12) of n_coarse splats each on canvases of their own (H, W): splats
+ *     [l n_coarse, (l + 1) n_coarse) are image l, its level; nothing is upsampled. The composite takes any range of
+ *     images: image l's pixels at out/T/asum/fg/gout + l H W, its background at bg[l, C], its background partials
+ *     (C ntiles + 3) & ~3 floats after the previous image's.
  * Level l takes global tile ids [tbase[l], tbase[l+1]) and packed pixel slots [pbase[l], pbase[l+1]) of
  * the FIELDS buffers; splat_levels_geometry reports them. */
 typedef struct splat_levels {
@@ -240,6 +244,10 @@ int splat_upsample_adjoint(int C, int H, int W, int TILE, const splat_levels *lv
 int splat_reduce_pairs(const float *rec, const int *offsets, const int *pair_splat, long long tot, int N,
                        int C, const float *pair_sums, const float *bg_part, int nparts, const float *log_scale,
                        float *g_mu, float *g_scale, float *g_theta, float *g_op, float *g_color, float *g_bg, void *stream);
+/* The same for a batch of images (levels mode 3): g_bg[images, C] from nparts partials per image. */
+int splat_reduce_images(const float *rec, const int *offsets, long long tot, int N, int C, const float *pair_sums,
+                        const float *bg_part, int nparts, int images, const float *log_scale, float *g_mu,
+                        float *g_scale, float *g_theta, float *g_op, float *g_color, float *g_bg, void *stream);
 
 /* Exact (unculled) path: every pixel sums every splat; pixel centres py[P], px[P] supplied by the caller.
  * Replaces _render_fwd_kernel / _render_bwd_kernel and their wrappers, render_triton.py:58-303. */
