@@ -1189,8 +1189,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter_units(const int4* __restrict
   }
 }
 
-// One workgroup of kRowThreads per tile row and chunk of at most kRowCols tile columns (blockIdx.y = global
-// row r, blockIdx.x = chunk of cw columns). Counting: the spans of the row's units (kRowUnits per round) give
+// One workgroup of kRowThreads per tile row and chunk of at most kRowCols tile columns (RowChunks). Counting: the spans of the row's units (kRowUnits per round) give
 // the row's pairs before c0 and a difference array over the chunk's columns (LDS atomics), so the chunk's tile
 // starts follow. Writing: the units meeting the chunk are listed in LDS in unit order (their index and span),
 // their splat ids and splat-major indices gathered for the listed units only, then each wave owns the columns
@@ -1205,16 +1204,23 @@ constexpr int kRowWaves = kRowThreads / 64;
 constexpr int kRowItems = 4;                          // units per thread and round
 constexpr int kRowUnits = kRowThreads * kRowItems;   // 2048 units per round
 constexpr int kRowCols = 128;                         // columns per chunk, at most
+constexpr int kCoarseChunks = 16;                     // chunks per row of a coarse level, at most
 constexpr int kRowHold = 4;                           // rounds whose spans stay in registers
 constexpr int kRowList = 2048;                        // units meeting the chunk listed at once, at most
 static_assert(kRowList >= kRowUnits, "a round fits the list");
+
+// The workgroups of the expansion: level l's rows are cut into nch[l] chunks of cw[l] columns, and its workgroups are
+// [wbase[l], wbase[l + 1]), row by row.
+struct RowChunks {
+  int cw[kMaxLevels], nch[kMaxLevels], wbase[kMaxLevels + 1];
+};
 
 // CPW > 0 (chunks of at most CPW columns per wave): each wave keeps its columns' running positions in
 // registers; CPW = 0: in LDS (s_diff), read and advanced by the owning wave.
 template <int CPW>
 __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const long long* __restrict__ info, int cap,
-                                                            const int2* __restrict__ rtot, int cw,
-                                                            const int* __restrict__ ug, const int* __restrict__ uq,
+                                                            const int2* __restrict__ rtot,
+                                                            RowChunks RC, const int* __restrict__ ug, const int* __restrict__ uq,
                                                             const int* __restrict__ uspan, int* __restrict__ gid_sorted,
                                                             int* __restrict__ tile_starts, int* __restrict__ pair_splat,
                                                             int* __restrict__ pair_q) {
@@ -1226,22 +1232,24 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
   __shared__ int s_n;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int t = threadIdx.x;
-  const int r = blockIdx.y;
-  const int l = level_of_row(L, r);
+  const int wg = (int)gridDim.x - 1 - (int)blockIdx.x;   // the coarsest level, with the longest lists, first
+  int l = 0;
+  while (l + 1 < L.n && wg >= RC.wbase[l + 1]) ++l;
+  const int r = L.rbase[l] + (wg - RC.wbase[l]) / RC.nch[l];
   const int ntx = L.ntx[l];
-  const int c0 = blockIdx.x * cw;
-  if (c0 >= ntx) return;
+  const int2 mine = rtot[r];   // units and pairs of the row
+  const int cw = RC.cw[l], c0 = (wg - RC.wbase[l]) % RC.nch[l] * cw;
   const int c1 = min(c0 + cw, ntx), ncol = c1 - c0;
   const int tile0 = L.tbase[l] + (r - L.rbase[l]) * ntx + c0;
   const int nt = L.tbase[L.n];
-  // units and pairs of the rows before r and of row r (loaded before the pair count is known: one round trip)
+  // units and pairs of the rows before r (loaded before the pair count is known: one round trip)
   int us = 0, pr = 0;
   for (int i = t; i < r; i += kRowThreads) {
     const int2 e = rtot[i];
     us += e.x;
     pr += e.y;
   }
-  const int row_units = rtot[r].x;
+  const int row_units = mine.x;
   const int tot = pair_count(info, cap);
   if (tot == 0) {   // no pairs (or a speculative launch past its capacity): the empty list
     if (t < ncol) tile_starts[tile0 + t] = 0;
@@ -1676,20 +1684,30 @@ int bin_pairs_launch(const int* rect, const int* offsets, const void* ws_count, 
                                               cp.nb, ug, uq, uspan);
     int rc = check_launch("k_scatter_units");
     if (rc) return rc;
-    int mxtx = 1;
-    for (int l = 0; l < L.n; ++l) mxtx = L.ntx[l] > mxtx ? L.ntx[l] : mxtx;
-    // chunks of at most kRowCols columns, about 8 per row of the widest level (measured: 4 to 12 chunks, 256 to
-    // 1024 threads, 2 to 8 units per thread; this is the fastest at 768 x 768 and 2048 x 2048)
-    const int cw = min(kRowCols, max(8, div_up(mxtx, 8)));
-    const dim3 grid(div_up(mxtx, cw), cp.nrows);
+    // Level 0, and the images of a batch: chunks of at most kRowCols columns, about 8 per row of the widest level
+    // (measured: 4 to 12 chunks, 256 to 1024 threads, 2 to 8 units per thread; this is the fastest at 768 x 768 and
+    // 2048 x 2048). Coarse levels hold few rows of long lists (27,000 pairs in a row of 12 tiles at 768 x 768): up to
+    // kCoarseChunks chunks per row. One workgroup per chunk and no more: taken as columns of a grid as wide as level 0's,
+    // the coarse rows' only chunks all fell on one XCD, and after level 0's (octave render at 768 x 768 with the encoder's
+    // splats: 59 us; spread 45 us, and the coarsest level first 32 us).
+    const bool batch = L.n > 1 && L.H[1] == L.H[0] && L.W[1] == L.W[0];
+    RowChunks RC{};
+    int cw = 1;
+    for (int l = 0; l < L.n; ++l) {
+      RC.cw[l] = min(kRowCols, l == 0 || batch ? max(8, div_up(L.ntx[l], 8)) : div_up(L.ntx[l], kCoarseChunks));
+      RC.nch[l] = div_up(L.ntx[l], RC.cw[l]);
+      RC.wbase[l + 1] = RC.wbase[l] + RC.nch[l] * (L.rbase[l + 1] - L.rbase[l]);
+      cw = max(cw, RC.cw[l]);
+    }
+    const int grid = RC.wbase[L.n];
     if (cw <= 2 * kRowWaves)
-      k_expand_row<2><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, cw, ug, uq, uspan, gid_sorted, tile_starts,
+      k_expand_row<2><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, RC, ug, uq, uspan, gid_sorted, tile_starts,
                                                      pair_splat, pair_q);
     else if (cw <= 4 * kRowWaves)
-      k_expand_row<4><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, cw, ug, uq, uspan, gid_sorted, tile_starts,
+      k_expand_row<4><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, RC, ug, uq, uspan, gid_sorted, tile_starts,
                                                      pair_splat, pair_q);
     else
-      k_expand_row<0><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, cw, ug, uq, uspan, gid_sorted, tile_starts,
+      k_expand_row<0><<<grid, kRowThreads, 0, st>>>(L, dinfo, t, rtot, RC, ug, uq, uspan, gid_sorted, tile_starts,
                                                      pair_splat, pair_q);
     return check_launch("k_expand_row");
   }

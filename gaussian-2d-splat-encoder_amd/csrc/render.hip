@@ -265,6 +265,48 @@ __device__ __forceinline__ TileAt split_item(const LevelTable& L, const SplitTab
   return tile_of(L, L.tbase[l] + j / s, l);
 }
 
+// Work items of an auto split launch over the coarse levels (tiles [t0, t1), global ids; every tile's list in chunks of
+// the same length): tile t takes the items [auto_base(t), auto_base(t + 1)), at least as many as it has chunks and at
+// least one, so an item finds its tile from the tile starts alone (auto_item) and no count has to be known at the launch.
+// The chunk length follows from the pairs of these tiles: 32 while that makes at most kAutoItems chunks, else 64. Equal
+// chunks keep the waves even where a level's lists are not, and the sums' grouping depends on the inputs alone. Measured
+// (forward + its combine / backward, us) at 32, 64, 128 and 256: 960,000 pairs 67 / 63, 64 / 57, 72 / 63, 83 / 78;
+// 390,000 pairs, forward 38, 35, 41, 61; 43,000 pairs 12 / 10, 15 / 12, 19 / 17, 26 / 25. (Each level's lists in equal
+// numbers of chunks of 128 pairs on average: 62 / 65, 46, 17 / 17.) kAutoItems also bounds the launch while the count is
+// between the two: 8,192, with the items without work past the card's 8 waves per SIMD, cost 390,000 pairs 7 us.
+constexpr int kAutoItems = 4096;
+__host__ __device__ __forceinline__ int auto_shift(long long pairs) {   // log2 of the chunk length
+  return pairs <= 32LL * kAutoItems ? 5 : 6;
+}
+struct AutoItem {
+  int t, g0, g1;       // tile and its chunk's pairs; t < 0: no work
+  int nchunk, part;    // the tile's chunks, its first item
+};
+// Item `item`, by the whole wave: a 64-way search over the tiles' first items (two or three rounds of loads).
+__device__ __forceinline__ AutoItem auto_item(const int* __restrict__ starts, int t0, int t1, int item, int lane) {
+  AutoItem r{-1, 0, 0, 0, 0};
+  const int b = starts[t0], sh = auto_shift(starts[t1] - b);
+  auto first = [&](int i) { return ((starts[t0 + i] - b) >> sh) + i; };   // strictly increasing in i
+  int lo = 0, n = t1 - t0;
+  if (item >= first(n)) return r;
+  while (n > 1) {
+    const int step = (n + 63) >> 6, i = lane * step;
+    const bool le = i < n && first(lo + i) <= item;   // a prefix of the lanes, lane 0 among them
+    const int k = (__popcll(__ballot(le)) - 1) * step;
+    lo += k;
+    n = min(step, n - k);
+  }
+  const int f = first(lo), g0 = starts[t0 + lo], g1 = starts[t0 + lo + 1];
+  r.nchunk = (g1 - g0 + (1 << sh) - 1) >> sh;
+  const int c = item - f;
+  if (c >= max(r.nchunk, 1)) return r;
+  r.t = t0 + lo;
+  r.g0 = g0 + (c << sh);
+  r.g1 = min(g1, r.g0 + (1 << sh));
+  r.part = f;
+  return r;
+}
+
 // Pixel centres (render_triton.py:455-456, (i + 0.5) / size in float32) of a tile: lane j < TILE divides for row j
 // and lane TILE + j for column j, one division for the wave, and each lane takes its own row's and column's by
 // shuffles; l is the lane's pixel within the tile, (py0, px0) the centre of its reference pixel: the middle one
@@ -383,18 +425,26 @@ __host__ __device__ constexpr int split_part_floats() { return (2 + C) * tile_th
 
 // FIELDS forward of the split work items of the coarse levels (SplitTable): one workgroup per item, the tile's
 // pixels one per thread, over the item's chunk of the tile's pair list (in pair order, as fwd_tile_pixel walks
-// it). A level with split 1 writes its fields; otherwise the item writes partial sums for k_fields_combine.
-template <int C, bool ODDS, int TILE>
+// it). A level with split 1 writes its fields; otherwise the item writes partial sums for k_fields_combine. AUTO: the
+// items of an auto split launch over the tiles [t0, t1) instead, `nitems` of them in the buffer `part` (more are not
+// written: the launch was planned for fewer pairs and is repeated).
+template <int C, bool ODDS, int TILE, bool AUTO>
 __global__ __launch_bounds__(tile_threads(TILE)) void k_fwd_fields_split(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L,
     SplitTable P, int nitems, float* __restrict__ slog, float* __restrict__ sa, float* __restrict__ sac,
-    float* __restrict__ part) {
+    float* __restrict__ part, int t0, int t1) {
   constexpr int NT = tile_threads(TILE);
   __shared__ float2 s_uv[NT / 64][64];
   const int item = xcd_swizzle(blockIdx.x, nitems);
-  int chunk, nsplit;
-  const TileAt ta = split_item(L, P, item, &chunk, &nsplit);
   const int th = (int)threadIdx.x, lane = th & 63;
+  int chunk, nsplit;
+  AutoItem ai;
+  if constexpr (AUTO) {
+    ai = auto_item(starts, t0, t1, item, lane);
+    if (ai.t < 0) return;
+  }
+  const TileAt ta = AUTO ? tile_of(L, ai.t, level_of(L, ai.t)) : split_item(L, P, item, &chunk, &nsplit);
+  if (AUTO && !((L.mask >> ta.l) & 1)) return;
   const int wid = __builtin_amdgcn_readfirstlane(th >> 6);
   const int yp = ta.ty * TILE + th / TILE, xp = ta.tx * TILE + th % TILE;
   const bool valid = th < TILE * TILE && yp < ta.H && xp < ta.W;
@@ -403,17 +453,25 @@ __global__ __launch_bounds__(tile_threads(TILE)) void k_fwd_fields_split(
   // the reference pixel: the middle one, or the canvas' last row / column where the tile extends past it
   const float py0 = uniform_f(((float)min(ta.ty * TILE + TILE / 2, ta.H - 1) + 0.5f) / (float)ta.H);
   const float px0 = uniform_f(((float)min(ta.tx * TILE + TILE / 2, ta.W - 1) + 0.5f) / (float)ta.W);
-  int g0 = starts[ta.t];
-  const int g1t = starts[ta.t + 1];
-  const int len = ((g1t - g0 + nsplit - 1) / nsplit + 3) & ~3;
-  g0 = min(g1t, g0 + chunk * len);
-  const int g1 = min(g1t, g0 + len);
+  int g0, g1;
+  if constexpr (AUTO) {
+    g0 = ai.g0;
+    g1 = ai.g1;
+    nsplit = ai.nchunk;
+  } else {
+    g0 = starts[ta.t];
+    const int g1t = starts[ta.t + 1];
+    const int len = ((g1t - g0 + nsplit - 1) / nsplit + 3) & ~3;
+    g0 = min(g1t, g0 + chunk * len);
+    g1 = min(g1t, g0 + len);
+  }
   float sl = 0.f, s_a = 0.f, sc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) sc[c] = 0.f;
   fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, s_uv[wid], lane, sl, s_a, sc);
   if (nsplit > 1) {
-    float* dst = part + (size_t)(P.pibase[ta.l] + item - P.ibase[ta.l]) * split_part_floats<C, TILE>() + th;
+    const int slot = AUTO ? item : P.pibase[ta.l] + item - P.ibase[ta.l];
+    float* dst = part + (size_t)slot * split_part_floats<C, TILE>() + th;
     dst[0] = sl;
     dst[NT] = s_a;
 #pragma unroll
@@ -460,6 +518,49 @@ __global__ __launch_bounds__(tile_threads(TILE)) void k_fields_combine(LevelTabl
   sa[pp] = s_a;
 #pragma unroll
   for (int c = 0; c < C; ++c) sac[pp * C + c] = sc[c];
+}
+
+// Fields of the coarse tiles of more than one chunk of an auto split launch: workgroup = tile, its chunks' partial sums
+// added in chunk order, in kAutoCombine contiguous shares (one per tile_threads(TILE) threads) that are added in order.
+constexpr int kAutoCombine = 4;
+template <int C, int TILE>
+__global__ __launch_bounds__(tile_threads(TILE) * kAutoCombine) void k_fields_combine_auto(
+    LevelTable L, const int* __restrict__ starts, int t0, int t1, const float* __restrict__ part, int nitems,
+    float* __restrict__ slog, float* __restrict__ sa, float* __restrict__ sac) {
+  constexpr int NT = tile_threads(TILE), K = 2 + C;
+  __shared__ float s_p[kAutoCombine - 1][K][NT];
+  const int t = t0 + blockIdx.x;
+  const int b = starts[t0], sh = auto_shift(starts[t1] - b), g0 = starts[t], n = (starts[t + 1] - g0 + (1 << sh) - 1) >> sh;
+  const int first = ((g0 - b) >> sh) + (int)blockIdx.x;
+  if (n < 2 || first + n > nitems) return;   // written by its item, or a launch that is repeated
+  const TileAt ta = tile_of(L, t, level_of(L, t));
+  if (!((L.mask >> ta.l) & 1)) return;
+  const int w = (int)threadIdx.x / NT, th = (int)threadIdx.x - w * NT;
+  const int per = (n + kAutoCombine - 1) / kAutoCombine, c0 = min(n, w * per), c1 = min(n, c0 + per);
+  const float* src = part + (size_t)(first + c0) * split_part_floats<C, TILE>() + th;
+  float v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = 0.f;
+  for (int c = c0; c < c1; ++c, src += split_part_floats<C, TILE>()) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += src[k * NT];
+  }
+  if (w > 0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) s_p[w - 1][k][th] = v[k];
+  }
+  __syncthreads();
+  const int yp = ta.ty * TILE + th / TILE, xp = ta.tx * TILE + th % TILE;
+  if (w > 0 || !(th < TILE * TILE && yp < ta.H && xp < ta.W)) return;
+#pragma unroll
+  for (int i = 0; i < kAutoCombine - 1; ++i)
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] += s_p[i][k][th];
+  const size_t pp = (size_t)ta.pb + (size_t)yp * ta.W + xp;
+  slog[pp] = v[0] * kLn2;
+  sa[pp] = v[1];
+#pragma unroll
+  for (int c = 0; c < C; ++c) sac[pp * C + c] = v[2 + c];
 }
 
 // Per-pixel upstream terms of the backward (render_triton.py:640-654). Masked pixels give zeros.
@@ -1005,14 +1106,15 @@ __host__ __device__ constexpr int bg_stride(int C, int ntiles) { return (C * nti
 // covering a 1/L share of the tile's pixels (whole rows when that share is at least a row) and the L partial
 // sums are combined with xor shuffles. At 5 waves per SIMD (at most 96 VGPRs, no spills) there are enough waves
 // to cover the latency of the VALU, LDS and transcendental pipes.
-// SPLIT (FIELDS only, S = 1): workgroup = a work item of the SplitTable, the item's chunk of its tile's pairs.
-template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S, bool SPLIT = false>
+// SPLIT (FIELDS only, S = 1): workgroup = a work item of the SplitTable (1) or of the auto split launch over the tiles
+// [tb0, tb1) (2), the item's chunk of its tile's pairs.
+template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S, int SPLIT = 0>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) void k_bwd_cull(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L, int tb0,
     int ntiles, const float* __restrict__ bg, const float* __restrict__ Tin, const float* __restrict__ asum_in,
     const float* __restrict__ fg_in, const float* __restrict__ gout, float* __restrict__ dslog,
     float* __restrict__ dsa, float* __restrict__ dsac, const int* __restrict__ pair_q, float* __restrict__ psum,
-    float* __restrict__ bg_part, SplitTable P) {
+    float* __restrict__ bg_part, SplitTable P, int tb1) {
   static_assert(!SPLIT || (FIELDS && S == 1), "split items: FIELDS backward, one wave per item");
   constexpr bool UPS = MODE == kUps, BATCH = MODE == kBatch;
   constexpr int NP = TILE * TILE;
@@ -1021,10 +1123,17 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
   __shared__ float s_pya[TILE], s_pxa[TILE];
   __shared__ int s_defer_w[S][128], s_mi_w[S][128];
   int chunk = 0, nsplit = 1;
-  const TileAt ta = SPLIT ? split_item(L, P, xcd_swizzle(blockIdx.x, ntiles), &chunk, &nsplit) : tile_at(L, tb0, ntiles);
+  const int lane = threadIdx.x & 63;
+  AutoItem ai;
+  if constexpr (SPLIT == 2) {
+    ai = auto_item(starts, tb0, tb1, xcd_swizzle(blockIdx.x, ntiles), lane);
+    if (ai.t < 0 || ai.nchunk == 0) return;
+  }
+  const TileAt ta = SPLIT == 2   ? tile_of(L, ai.t, level_of(L, ai.t))
+                    : SPLIT == 1 ? split_item(L, P, xcd_swizzle(blockIdx.x, ntiles), &chunk, &nsplit)
+                                 : tile_at(L, tb0, ntiles);
   if (!((L.mask >> ta.l) & 1)) return;
   const int t = ta.t;
-  const int lane = threadIdx.x & 63;
   const int wid = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;   // wave-uniform
   int* s_defer = s_defer_w[wid];
   int* s_mi = s_mi_w[wid];
@@ -1076,8 +1185,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
   const float py0 = tc.py0, px0 = tc.px0, py1 = tc.py1, px1 = tc.px1;
   const float pym = py0 + tc.cy, pxm = px0 + tc.cx;   // the middle of the box of the tile's pixel centres
   const float rH = uniform_f(hw_rcp(fH)), rW = uniform_f(hw_rcp(fW));   // for ring_pixel_m's bound only
-  int g0 = starts[t], g1 = starts[t + 1];
-  if (SPLIT) {   // the item's chunk: whole passes of 64 pairs where the tile's list allows
+  int g0 = SPLIT == 2 ? ai.g0 : starts[t], g1 = SPLIT == 2 ? ai.g1 : starts[t + 1];
+  if (SPLIT == 1) {   // the item's chunk: whole passes of 64 pairs where the tile's list allows
     const int len = (((g1 - g0 + nsplit - 1) / nsplit) + 63) & ~63;
     g0 = min(g1, g0 + chunk * len);
     g1 = min(g1, g0 + len);
@@ -2329,10 +2438,11 @@ int splat_render_bwd(const float* rec, const int* gid_sorted, const int* tile_st
         if (TT == 8 && (flags & kFlagWide))
           launch_tile_kernel(k_bwd_cull<CC, FL, OD, UP, TT, 16>, ntiles, 64 * 16, st, rec, gid_sorted, tile_starts, L,
                              tb0, ntiles, bg, T, asum, fg, gout, dslog, dsa, dsac, pair_q, pair_sums, bg_part,
-                             SplitTable{});
+                             SplitTable{}, 0);
         else
           launch_tile_kernel(k_bwd_cull<CC, FL, OD, UP, TT, 1>, ntiles, 64, st, rec, gid_sorted, tile_starts, L, tb0,
-                             ntiles, bg, T, asum, fg, gout, dslog, dsa, dsac, pair_q, pair_sums, bg_part, SplitTable{});
+                             ntiles, bg, T, asum, fg, gout, dslog, dsa, dsac, pair_q, pair_sums, bg_part, SplitTable{},
+                             0);
         return check_launch("k_bwd_cull");
       });
     });
@@ -2417,11 +2527,11 @@ int splat_render_fields_split(const float* rec, const int* gid_sorted, const int
     return with_tile(TILE, [&](auto tt) {
       constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
       if (flags & kFlagOdds)
-        launch_tile_kernel(k_fwd_fields_split<CC, true, TT>, nitems, tile_threads(TT), st, rec, gid_sorted,
-                           tile_starts, L, P, nitems, slog, sa, sac, part);
+        launch_tile_kernel(k_fwd_fields_split<CC, true, TT, false>, nitems, tile_threads(TT), st, rec, gid_sorted,
+                           tile_starts, L, P, nitems, slog, sa, sac, part, 0, 0);
       else
-        launch_tile_kernel(k_fwd_fields_split<CC, false, TT>, nitems, tile_threads(TT), st, rec, gid_sorted,
-                           tile_starts, L, P, nitems, slog, sa, sac, part);
+        launch_tile_kernel(k_fwd_fields_split<CC, false, TT, false>, nitems, tile_threads(TT), st, rec, gid_sorted,
+                           tile_starts, L, P, nitems, slog, sa, sac, part, 0, 0);
       if (ncomb) k_fields_combine<CC, TT><<<ncomb, tile_threads(TT), 0, st>>>(L, P, part, slog, sa, sac);
       return check_launch("k_fwd_fields_split");
     });
@@ -2451,14 +2561,107 @@ int splat_render_fields_split_bwd(const float* rec, const int* gid_sorted, const
     return with_tile(TILE, [&](auto tt) {
       constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
       if (flags & kFlagOdds)
-        launch_tile_kernel(k_bwd_cull<CC, true, true, kPlain, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
+        launch_tile_kernel(k_bwd_cull<CC, true, true, kPlain, TT, 1, 1>, nitems, 64, st, rec, gid_sorted,
                            tile_starts, L, 0, nitems, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
-                           pair_q, pair_sums, nullptr, P);
+                           pair_q, pair_sums, nullptr, P, 0);
       else
-        launch_tile_kernel(k_bwd_cull<CC, true, false, kPlain, TT, 1, true>, nitems, 64, st, rec, gid_sorted,
+        launch_tile_kernel(k_bwd_cull<CC, true, false, kPlain, TT, 1, 1>, nitems, 64, st, rec, gid_sorted,
                            tile_starts, L, 0, nitems, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
-                           pair_q, pair_sums, nullptr, P);
+                           pair_q, pair_sums, nullptr, P, 0);
       return check_launch("k_bwd_cull(split)");
+    });
+  });
+}
+
+// Items of an auto split launch over `ntiles` tiles that hold at most `cap` pairs (auto_base of the last tile's end).
+static long long auto_items(long long cap, int ntiles) {
+  return min(cap >> 5, max((long long)kAutoItems, cap >> 6)) + ntiles;
+}
+
+// Host: level table and items of an auto split launch over the coarse levels of `lv`.
+static int auto_levels(const char* who, int C, int H, int W, int TILE, int flags, const splat_levels* lv,
+                       unsigned levmask, long long cap, LevelTable* L, int* ntiles, long long* items) {
+  if (flags & ~kFlagOdds) return set_error(kInvalid, "%s: flags=%d (only ODDS)", who, flags);
+  if (cap < 0 || cap > 0x7fffffffLL - 64) return set_error(kInvalid, "%s: cap=%lld", who, cap);
+  if (H < 1 || W < 1 || C < 1 || C > kMaxC || (lv && lv->mode == 3) || make_levels(H, W, TILE, lv, L, nullptr))
+    return set_error(kInvalid, "%s: C=%d H=%d W=%d or bad levels", who, C, H, W);
+  L->mask &= levmask & ~1u;
+  *ntiles = L->mask ? L->tbase[L->n] - L->tbase[1] : 0;
+  *items = *ntiles ? auto_items(cap, *ntiles) : 0;
+  if (*items > 0x3fffffffLL) return set_error(kOverflow, "%s: %lld work items", who, *items);
+  return kOk;
+}
+
+size_t splat_fields_auto_workspace_bytes(int C, int H, int W, int TILE, const splat_levels* lv, unsigned levmask,
+                                         long long cap) {
+  LevelTable L;
+  int ntiles;
+  long long items;
+  if ((TILE != 4 && TILE != 8 && TILE != 16) ||
+      auto_levels("splat_fields_auto_workspace_bytes", C, H, W, TILE, 0, lv, levmask, cap, &L, &ntiles, &items))
+    return 0;
+  return split_part_bytes(C, TILE, items);
+}
+
+int splat_render_fields_auto(const float* rec, const int* gid_sorted, const int* tile_starts, int C, int H, int W,
+                             int TILE, int flags, const splat_levels* lv, unsigned levmask, long long cap, float* slog,
+                             float* sa, float* sac, void* ws, size_t ws_bytes, void* stream) {
+  LevelTable L;
+  int ntiles;
+  long long items;
+  if (int e = auto_levels("splat_render_fields_auto", C, H, W, TILE, flags, lv, levmask, cap, &L, &ntiles, &items)) return e;
+  if (!rec || !gid_sorted || !tile_starts || !slog || !sa || !sac)
+    return set_error(kInvalid, "splat_render_fields_auto: null pointer");
+  if (items == 0) return kOk;
+  if (!ws || ws_bytes < split_part_bytes(C, TILE, items))
+    return set_error(kWorkspace, "splat_render_fields_auto: workspace of %zu bytes, %zu needed", ws_bytes,
+                     split_part_bytes(C, TILE, items));
+  hipStream_t st = (hipStream_t)stream;
+  float* part = (float*)ws;
+  const int t0 = L.tbase[1], t1 = L.tbase[L.n];
+  return with_c(C, [&](auto cc) {
+    return with_tile(TILE, [&](auto tt) {
+      constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
+      if (flags & kFlagOdds)
+        launch_tile_kernel(k_fwd_fields_split<CC, true, TT, true>, (unsigned)items, tile_threads(TT), st, rec,
+                           gid_sorted, tile_starts, L, SplitTable{}, (int)items, slog, sa, sac, part, t0, t1);
+      else
+        launch_tile_kernel(k_fwd_fields_split<CC, false, TT, true>, (unsigned)items, tile_threads(TT), st, rec,
+                           gid_sorted, tile_starts, L, SplitTable{}, (int)items, slog, sa, sac, part, t0, t1);
+      k_fields_combine_auto<CC, TT><<<ntiles, tile_threads(TT) * kAutoCombine, 0, st>>>(L, tile_starts, t0, t1, part,
+                                                                                        (int)items, slog, sa, sac);
+      return check_launch("k_fwd_fields_split");
+    });
+  });
+}
+
+int splat_render_fields_auto_bwd(const float* rec, const int* gid_sorted, const int* tile_starts, const int* pair_q,
+                                 long long tot, int C, int H, int W, int TILE, int flags, const splat_levels* lv,
+                                 unsigned levmask, long long cap, float* dslog, float* dsa, float* dsac,
+                                 float* pair_sums, void* stream) {
+  LevelTable L;
+  int ntiles;
+  long long items;
+  if (int e = auto_levels("splat_render_fields_auto_bwd", C, H, W, TILE, flags, lv, levmask, cap, &L, &ntiles, &items))
+    return e;
+  if (tot < 0 || tot > 0x7fffffffLL - 64) return set_error(kInvalid, "splat_render_fields_auto_bwd: tot=%lld", tot);
+  if (!rec || !gid_sorted || !tile_starts || !pair_sums || !dslog || !dsa || !dsac || (tot > 0 && !pair_q))
+    return set_error(kInvalid, "splat_render_fields_auto_bwd: null pointer");
+  if (items == 0) return kOk;
+  hipStream_t st = (hipStream_t)stream;
+  const int t0 = L.tbase[1], t1 = L.tbase[L.n];
+  return with_c(C, [&](auto cc) {
+    return with_tile(TILE, [&](auto tt) {
+      constexpr int CC = decltype(cc)::value, TT = decltype(tt)::value;
+      if (flags & kFlagOdds)
+        launch_tile_kernel(k_bwd_cull<CC, true, true, kPlain, TT, 1, 2>, (unsigned)items, 64, st, rec, gid_sorted,
+                           tile_starts, L, t0, (int)items, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
+                           pair_q, pair_sums, nullptr, SplitTable{}, t1);
+      else
+        launch_tile_kernel(k_bwd_cull<CC, true, false, kPlain, TT, 1, 2>, (unsigned)items, 64, st, rec, gid_sorted,
+                           tile_starts, L, t0, (int)items, nullptr, nullptr, nullptr, nullptr, nullptr, dslog, dsa, dsac,
+                           pair_q, pair_sums, nullptr, SplitTable{}, t1);
+      return check_launch("k_bwd_cull(auto split)");
     });
   });
 }

@@ -59,6 +59,10 @@ _SIGS = {
                                        _SZ, _VP]),
     "splat_render_fields_split_bwd": (_I, [_VP, _VP, _VP, _VP, _LL, _I, _I, _I, _I, _I, _LV, _I, _I, _U, _VP, _VP,
                                            _VP, _VP, _VP, _VP]),
+    "splat_fields_auto_workspace_bytes": (_SZ, [_I, _I, _I, _I, _LV, _U, _LL]),
+    "splat_render_fields_auto": (_I, [_VP, _VP, _VP, _I, _I, _I, _I, _I, _LV, _U, _LL, _VP, _VP, _VP, _VP, _SZ, _VP]),
+    "splat_render_fields_auto_bwd": (_I, [_VP, _VP, _VP, _VP, _LL, _I, _I, _I, _I, _I, _LV, _U, _LL, _VP, _VP, _VP, _VP,
+                                          _VP]),
     "splat_upsample_adjoint_workspace_bytes": (_SZ, [_I, _I, _I, _I, _LV]),
     "splat_upsample_adjoint": (_I, [_I, _I, _I, _I, _LV, _U, _VP, _VP, _VP, _VP, _SZ, _VP]),
     "splat_reduce_pairs": (_I, [_VP, _VP, _VP, _LL, _I, _I, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP]),

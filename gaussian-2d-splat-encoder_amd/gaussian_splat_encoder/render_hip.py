@@ -176,6 +176,7 @@ class TileBins:
         self.H, self.W, self.TILE, self.ntx, self.nt = H, W, TILE, ntx, nt
         self.blocks, self.pairs, self.with_maps = blocks, pairs, with_maps
         self.lv, self.geom, self.npix, self.level_tot_b = lv, geom, npix, level_tot_b
+        self.n_images = lv.max_octaves if lv is not None and lv.mode == 3 else 1   # that share it, one level each
         self.pending = None   # a _Pending while the pair count of a deferred binning is unread
         self._views = {}
         self._ptrs = {}
@@ -222,11 +223,6 @@ class TileBins:
 
     def as_tuple(self):
         return self.gid_b, self.starts_b, self.ntx, self.nt
-
-    @property
-    def n_images(self):
-        """Images that share this binning (a merged batch, one level each), else 1."""
-        return self.lv.max_octaves if self.lv is not None and self.lv.mode == 3 else 1
 
     @property
     def n_levels(self):
@@ -276,6 +272,7 @@ def _lv_key(lv):
 _GEOM = {}          # (H, W, TILE, levels) -> levels_geometry result
 _PAIRS_HW = {}      # binning configuration -> most pairs one image needed so far (sizes the next capacity)
 _LEVELS_SEEN = {}   # binning configuration -> per-level pair totals of its last binning (plans deferred launches)
+_MASK_SEEN = {}     # binning configuration -> levels that held pairs in any call
 _WS1 = {}           # binning configuration -> count-phase workspace bytes
 _tls = threading.local()
 
@@ -510,7 +507,7 @@ _SPLIT_MAX = 64
 
 
 def _level_splits(bins, lt, mask):
-    """Chunks per tile of every level for the split FIELDS launches over the coarse levels (ctypes int array):
+    """For splat_render_fields_split, which takes the numbers of chunks from its caller: chunks per tile of every level for the split FIELDS launches over the coarse levels (ctypes int array):
     a level in `mask` gets about _SPLIT_PAIRS pairs per chunk on average over its tiles (1 to _SPLIT_MAX chunks),
     so a dense coarse level's few tiles with long pair lists are spread over many workgroups; level 0 and levels
     outside `mask` get 1 (unused)."""
@@ -525,13 +522,9 @@ def _level_splits(bins, lt, mask):
     return sp
 
 
-def _fwd_order(bins, lt, mask, held):
-    """What the summation order of a levels forward launched for per-level totals lt over the levels in `mask`
-    depends on, over the levels in `held`: each coarse level's chunks per tile (their partial sums are added in
-    chunk order) and the level-0 composite's waves per tile."""
-    sp = _level_splits(bins, lt, mask & ~1)
-    return (tuple(sp[l] for l in range(1, bins.n_levels) if (held >> l) & 1),
-            _wide(bins.TILE, bins.ntiles0, lt[0]))
+def _coarse_cap(pairs):
+    """Pairs a launch over the coarse levels is sized for when the count read is expected to be about `pairs`."""
+    return pairs + (pairs >> 4) + 1024
 
 
 def _fields_buffers(npix, C, dev):
@@ -540,23 +533,23 @@ def _fields_buffers(npix, C, dev):
     return slog, sa, sac.view(npix, C)
 
 
-_SPLIT_WS = {}   # (C, H, W, TILE, levels, mask, splits) -> split-launch workspace bytes
+_AUTO_WS = {}    # (C, H, W, TILE, levels, mask, cap) -> auto split launch workspace bytes
 _ADJ_WS = {}     # (C, H, W, TILE, levels) -> upsample-adjoint workspace bytes
 
 
-def _fields_split_fwd(lib, bins, b, C, odd, lt, mask, fl, stream):
-    """FIELDS forward of the coarse levels in `mask` of image b into the packed fields fl, one split launch."""
-    L = bins.n_levels
+def _fields_coarse_fwd(lib, bins, b, C, odd, cap, mask, fl, stream):
+    """FIELDS forward of the coarse levels in `mask` of image b, of at most `cap` pairs, into the packed fields fl."""
     lvr = _lib.ctypes.byref(bins.lv)
-    sp = _level_splits(bins, lt, mask)
-    key = (C, bins.H, bins.W, bins.TILE, _lv_key(bins.lv), mask, tuple(sp))
-    nb = _SPLIT_WS.get(key)
+    key = (C, bins.H, bins.W, bins.TILE, _lv_key(bins.lv), mask, cap)
+    nb = _AUTO_WS.get(key)
     if nb is None:
-        nb = _SPLIT_WS[key] = lib.splat_fields_split_workspace_bytes(C, bins.H, bins.W, bins.TILE, lvr, 1, L, mask, sp)
-    ws = _ws(nb, fl[0].device) if nb else None
-    check(lib.splat_render_fields_split(bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"), C, bins.H, bins.W,
-                                        bins.TILE, odd, lvr, 1, L, mask, sp, *[ptr(t) for t in fl], ptr(ws), nb,
-                                        stream), "splat_render_fields_split")
+        if len(_AUTO_WS) > 1024:
+            _AUTO_WS.clear()
+        nb = _AUTO_WS[key] = lib.splat_fields_auto_workspace_bytes(C, bins.H, bins.W, bins.TILE, lvr, mask, cap)
+    ws = _ws(nb, fl[0].device)
+    check(lib.splat_render_fields_auto(bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"), C, bins.H, bins.W,
+                                       bins.TILE, odd, lvr, mask, cap, *[ptr(t) for t in fl], ptr(ws), nb, stream),
+          "splat_render_fields_auto")
 
 
 def _render_fwd(lib, bins, b, C, flags, lev, mask, comp, fields, stream):
@@ -602,6 +595,40 @@ def _wide_launches(bins, tots):
     return [(x, (b, b + 1)) for b, x in enumerate(w)]
 
 
+def _forward_cull_batch(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, odds, with_maps, scale_is_log, plan, lv):
+    """_forward_cull of a batch merged by `lv` (_batch_levels): one binning, and one launch per step for every image."""
+    B, N, C = color.shape
+    dev = mu.device
+    bins = _bin(_flat_batch(mu), _flat_batch(scale), _flat_batch(color), _flat_batch(opacity), _flat_batch(theta), H, W,
+                TILE, cutoff, None, with_maps, lv, scale_is_log, True)
+    out, T, asum, fg = _composite_buffers(B, H * W, C, dev)
+    bgf = _f32(bg)
+    flags = FLAG_ODDS if odds else 0
+    lib, stream = _lib.load(), _lib.stream_ptr(dev)
+    comp = (bgf, out, T, asum, fg)
+
+    def launch(tots):
+        for wide, lev in _wide_launches(bins, tots):
+            ev = kernel_timer.record("fwd") if kernel_timer.enabled else None
+            try:
+                _render_fwd(lib, bins, 0, C, flags | wide, lev, (1 << B) - 1, comp, (None,) * 3, stream)
+            finally:
+                kernel_timer.close("fwd", ev)
+
+    if bins.pending is not None:   # as in _forward_cull, per image
+        spec = _speculated_levels(bins)
+        launch(spec)
+        if plan is not None:
+            plan.allocate(bins, B, N, C, dev, lib, bins.pending.cap)
+        if _finish(bins) or _wide_launches(bins, bins.level_tot_b[0]) != _wide_launches(bins, spec):
+            launch(bins.level_tot_b[0])
+    else:
+        launch(bins.level_tot_b[0])
+    if plan is not None:
+        plan.bind(bins, B, N, C, dev, lib, stream, flags, (bgf, T, asum, fg))
+    return out, (T, asum, fg), bins
+
+
 def _forward_cull(mu, scale, color, opacity, bg, theta, H, W, TILE=8, cutoff=3.0, max_pairs=None, odds=False,
                   with_maps=True, scale_is_log=False, plan=None):
     """Composite forward (render_triton.py:538-567): out [B,P,C], (T, asum, fg), bins. plan: a _BwdPlan to
@@ -609,51 +636,43 @@ def _forward_cull(mu, scale, color, opacity, bg, theta, H, W, TILE=8, cutoff=3.0
     B, N, C = color.shape
     P = H * W
     dev = mu.device
-    lv = _batch_levels(B, N, H, W, TILE) if B > 1 and max_pairs is None else None
-    if lv is not None:   # one binning and one launch per step for the whole batch
-        bins = _bin(_flat_batch(mu), _flat_batch(scale), _flat_batch(color), _flat_batch(opacity), _flat_batch(theta), H,
-                    W, TILE, cutoff, None, with_maps, lv, scale_is_log, True)
-    else:
-        bins = _bin(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, with_maps, scale_is_log=scale_is_log,
-                    defer=True)
+    if B > 1 and max_pairs is None:
+        lv = _batch_levels(B, N, H, W, TILE)
+        if lv is not None:
+            return _forward_cull_batch(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, odds, with_maps,
+                                       scale_is_log, plan, lv)
+    bins = _bin(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, with_maps, scale_is_log=scale_is_log,
+                defer=True)
     out, T, asum, fg = _composite_buffers(B, P, C, dev)
     bgf = _f32(bg)
     flags = FLAG_ODDS if odds else 0
     lib, stream = _lib.load(), _lib.stream_ptr(dev)
 
-    nt = bins.ntiles0
-
-    def launch_one(b, wide, lev, mask):
-        comp = (_bptr(bgf, b), _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b))
-        if not kernel_timer.enabled:
-            return _render_fwd(lib, bins, b, C, flags | wide, lev, mask, comp, (None,) * 3, stream)
-        ev = kernel_timer.record("fwd")
-        try:
-            _render_fwd(lib, bins, b, C, flags | wide, lev, mask, comp, (None,) * 3, stream)
-        finally:
-            kernel_timer.close("fwd", ev)
-
     def launch(tots):
-        if lv is None:
-            for b in range(B):
-                launch_one(b, _wide(TILE, nt, tots[b]), (0, 1), 1)
-        else:
-            for wide, lev in _wide_launches(bins, tots):
-                launch_one(0, wide, lev, (1 << B) - 1)
+        for b in range(B):
+            comp = (_bptr(bgf, b), _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b))
+            if not kernel_timer.enabled:
+                _render_fwd(lib, bins, b, C, flags | _wide(TILE, bins.nt, tots[b]), (0, 1), 1, comp, (None,) * 3,
+                            stream)
+                continue
+            ev = kernel_timer.record("fwd")
+            try:
+                _render_fwd(lib, bins, b, C, flags | _wide(TILE, bins.nt, tots[b]), (0, 1), 1, comp, (None,) * 3,
+                            stream)
+            finally:
+                kernel_timer.close("fwd", ev)
 
     if bins.pending is not None:   # queued on the speculative pair list before the count is read
-        spec = _speculated_levels(bins)
-        launch(spec)
+        spec = _speculated_levels(bins)[0]
+        launch([spec])
         if plan is not None:         # the backward's buffers, allocated while the GPU works towards the count
             plan.allocate(bins, B, N, C, dev, lib, bins.pending.cap)
         # launched again when the pair phase was redone, or when the count asks for another number of waves per
         # tile than the speculated one (they group the per-pixel sums: the image depends on the inputs alone)
-        redone = _finish(bins)
-        tots = bins.tot_b if lv is None else bins.level_tot_b[0]
-        if redone or any(_wide(TILE, nt, t) != _wide(TILE, nt, s) for t, s in zip(tots, spec)):
-            launch(tots)
+        if _finish(bins) or _wide(TILE, bins.nt, bins.tot_b[0]) != _wide(TILE, bins.nt, spec):
+            launch(bins.tot_b)
     else:
-        launch(bins.tot_b if lv is None else bins.level_tot_b[0])
+        launch(bins.tot_b)
     if plan is not None:
         plan.bind(bins, B, N, C, dev, lib, stream, flags, (bgf, T, asum, fg))
     return out, (T, asum, fg), bins
@@ -797,13 +816,13 @@ def _forward_levels(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, ma
     lib, stream = _lib.load(), _lib.stream_ptr(dev)
     nt0 = bins.ntiles0
 
-    def launch(b, lt, mask):
-        """The launches of image b for per-level pair totals lt (they size the coarse levels' split and pick the
-        16-wave composite) over the levels in mask (a level in mask that holds no pair renders zeros)."""
+    def launch(b, lt, mask, cap):
+        """The launches of image b for per-level pair totals lt (level 0's picks the 16-wave composite) over the levels
+        in mask (a level in mask that holds no pair renders zeros), the coarse ones' for up to cap pairs."""
         ev = kernel_timer.record("fwd")
         try:
             if mask & ~1:
-                _fields_split_fwd(lib, bins, b, C, odd, lt, mask & ~1, fl, stream)
+                _fields_coarse_fwd(lib, bins, b, C, odd, cap, mask & ~1, fl, stream)
             _render_fwd(lib, bins, b, C, FLAG_UPS | odd | _wide(TILE, nt0, lt[0]), (0, 1), mask,
                         (_bptr(bgf, b), _bptr(out, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b)), fl, stream)
         finally:
@@ -811,20 +830,23 @@ def _forward_levels(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, ma
 
     if bins.pending is not None:   # queued on the speculative pair list and levels before the count is read
         lt_spec = _speculated_levels(bins)
-        mask_spec = _mask_of(lt_spec)
-        launch(0, lt_spec, mask_spec)
+        # every level that held a pair in some call of this configuration: one that comes and goes costs its (zero)
+        # fields, not a second launch
+        mask_spec = _MASK_SEEN[bins.pending.key] = _MASK_SEEN.get(bins.pending.key, 0) | _mask_of(lt_spec)
+        cap = _coarse_cap(sum(lt_spec[1:]))
+        launch(0, lt_spec, mask_spec, cap)
         if plan is not None:         # the backward's buffers, allocated while the GPU works towards the count
             plan.allocate(bins, B, N, C, dev, lib, bins.pending.cap)
         redone = _finish(bins)
         lt, held = bins.level_tot_b[0], bins.level_mask(0)
-        # launched again when the pair phase was redone, when a level holding pairs was left out, or when the
-        # count asks for another summation order than the speculated totals gave
-        if redone or held & ~mask_spec or _fwd_order(bins, lt_spec, mask_spec, held) != _fwd_order(bins, lt, held,
-                                                                                                     held):
-            launch(0, lt, held)
+        # launched again when the pair phase was redone, when a level holding pairs was left out or the coarse levels hold
+        # more pairs than planned, or when the count asks for another number of waves per tile than the speculated one
+        if redone or held & ~mask_spec or sum(lt[1:]) > cap or _wide(TILE, nt0, lt[0]) != _wide(TILE, nt0, lt_spec[0]):
+            launch(0, lt, held, sum(lt[1:]))
     else:
         for b in range(B):
-            launch(b, bins.level_tot_b[b], bins.level_mask(b))
+            lt = bins.level_tot_b[b]
+            launch(b, lt, bins.level_mask(b), sum(lt[1:]))
     if plan is not None:
         plan.bind(bins, B, N, C, dev, lib, stream, odd, (bgf, T, asum, fg))
     return out, (T, asum, fg), bins
@@ -980,11 +1002,10 @@ def _backward_levels(grad_out, color, bg, has_theta, T, asum, fg, bins, odds, lo
             if mask & ~1:
                 check(lib.splat_upsample_adjoint(C, bins.H, bins.W, bins.TILE, lvr, mask, *[ptr(t) for t in dS],
                                                  ptr(adj_ws), adj_ws.numel(), stream), "splat_upsample_adjoint")
-                check(lib.splat_render_fields_split_bwd(bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"),
-                                                        bins.p(b, "pq"), bins.tot_b[b], C, bins.H, bins.W, bins.TILE,
-                                                        odd, lvr, 1, L, mask & ~1, _level_splits(bins, lt, mask & ~1),
-                                                        *[ptr(t) for t in dS], ptr(sums), stream),
-                      "splat_render_fields_split_bwd")
+                check(lib.splat_render_fields_auto_bwd(bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"),
+                                                       bins.p(b, "pq"), bins.tot_b[b], C, bins.H, bins.W, bins.TILE, odd,
+                                                       lvr, mask & ~1, sum(lt[1:]), *[ptr(t) for t in dS], ptr(sums),
+                                                       stream), "splat_render_fields_auto_bwd")
         finally:
             kernel_timer.close("bwd", ev)
         _reduce(lib, bins, b, C, sums, bg_part, grads, _bptr(g_bg, b), stream, lsc)
@@ -1053,8 +1074,7 @@ class _LevelsBwdPlan:
             if mask & ~1:
                 adj = (C, bins.H, bins.W, bins.TILE, lvr, mask, *ds, ptr(self.adj), self.adj_n, stream)
                 split = (bins.p(b, "rec"), bins.p(b, "gid"), bins.p(b, "starts"), bins.p(b, "pq"), tots[b], C, bins.H,
-                         bins.W, bins.TILE, odd, lvr, 1, L, mask & ~1, _level_splits(bins, lt, mask & ~1), *ds, sb,
-                         stream)
+                         bins.W, bins.TILE, odd, lvr, mask & ~1, sum(lt[1:]), *ds, sb, stream)
             sl = lambda t: None if N == 0 else _bptr(t, b)
             red = (bins.p(b, "rec") if N else None, bins.p(b, "off") if N else None, None, tots[b], N, C, sb, bgp, nt0,
                    sl(self.lsc), sl(g_mu), sl(g_scale), sl(g_th), sl(g_op), sl(g_col), _bptr(g_bg, b), stream)
@@ -1071,7 +1091,7 @@ class _LevelsBwdPlan:
                 check(lib.splat_render_bwd(*head, g0 + 4 * img * b, *tail), "splat_render_bwd")
                 if adj is not None:
                     check(lib.splat_upsample_adjoint(*adj), "splat_upsample_adjoint")
-                    check(lib.splat_render_fields_split_bwd(*split), "splat_render_fields_split_bwd")
+                    check(lib.splat_render_fields_auto_bwd(*split), "splat_render_fields_auto_bwd")
             finally:
                 kernel_timer.close("bwd", ev)
             ev = kernel_timer.record("reduce")

@@ -225,6 +225,20 @@ int splat_render_fields_split_bwd(const float *rec, const int *gid_sorted, const
                                   int lev_begin, int lev_end, unsigned levmask, const int *splits, float *dslog,
                                   float *dsa, float *dsac, float *pair_sums, void *stream);
 
+/* The same over every coarse level of levmask, with chunks of one length for all tiles that the kernels choose from the
+ * pairs found in tile_starts (32 or 64): no split has to be planned, and the sums' grouping depends on the pair list
+ * alone. cap: a bound of the coarse levels' pairs (sizes the launch and the workspace; with more pairs than cap the
+ * forward's fields are not complete and the backward's sums neither). */
+size_t splat_fields_auto_workspace_bytes(int C, int H, int W, int TILE, const splat_levels *lv, unsigned levmask,
+                                         long long cap);
+int splat_render_fields_auto(const float *rec, const int *gid_sorted, const int *tile_starts, int C, int H, int W,
+                             int TILE, int flags, const splat_levels *lv, unsigned levmask, long long cap,
+                             float *slog, float *sa, float *sac, void *ws, size_t ws_bytes, void *stream);
+int splat_render_fields_auto_bwd(const float *rec, const int *gid_sorted, const int *tile_starts, const int *pair_q,
+                                 long long tot, int C, int H, int W, int TILE, int flags, const splat_levels *lv,
+                                 unsigned levmask, long long cap, float *dslog, float *dsa, float *dsac,
+                                 float *pair_sums, void *stream);
+
 /* Backward of the upsample: the exact adjoint of the bilinear upsample of every masked coarse level,
  * from the level-0 upstream dslog/dsa/dsac[0, P) into the coarse levels' packed slots, deterministic
  * (two gather passes, no atomics). Replaces the autograd of F.interpolate at render_triton.py:864-876. */

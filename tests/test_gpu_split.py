@@ -145,3 +145,53 @@ def test_split_argument_checks(dev):
     assert lib.splat_render_fields_split(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), C, 128, 128, 8,
                                          RH.FLAG_FIELDS, lvr, 1, L, mask, sp1, *[t.data_ptr() for t in fl], None, 0,
                                          _lib.stream_ptr(dev)) == 1
+
+
+def auto_shift(pairs):
+    """log2 of the chunk length of an auto split launch (32 while that makes at most 4,096 chunks, else 64)."""
+    return 5 if pairs <= 32 * 4096 else 6
+
+
+@pytest.mark.parametrize("TILE,n,px,H,W", [(8, 2500, 24.0, 128, 128), (4, 300, 30.0, 96, 72), (16, 2500, 24.0, 160, 96),
+                                           (8, 40, 10.0, 300, 40), (8, 60000, 30.0, 512, 512)])
+@pytest.mark.parametrize("odds", [0, 1])
+def test_auto_split_equals_plain_launch(dev, TILE, n, px, H, W, odds):
+    """The auto split forward and backward against the unsplit kernels on the same pair list: tiles without pairs, of one
+    chunk and of many, each chunk length; the same bits whatever bound the launch is sized for."""
+    lib = _lib.load()
+    bins, C = scene_bins(dev, H, W, TILE, n=n, px=px)
+    flags = RH.FLAG_ODDS if odds else 0
+    coarse = sum(bins.level_tot_b[0][1:])
+    mask = ((1 << bins.n_levels) - 1) & ~1
+    lvr, s = ctypes.byref(bins.lv), _lib.stream_ptr(dev)
+    ref = run_plain_fwd(lib, bins, C, flags, mask, dev)
+    P0 = bins.geom[1][4]
+    got = []
+    for cap in (coarse, coarse + 1000, 3 * coarse):
+        fl = tuple(torch.full_like(t, float("nan")) for t in ref)
+        nb = lib.splat_fields_auto_workspace_bytes(C, H, W, TILE, lvr, mask, cap)
+        ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=dev)
+        _lib.check(lib.splat_render_fields_auto(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), C, H, W, TILE, flags,
+                                                lvr, mask, cap, *[t.data_ptr() for t in fl], ws.data_ptr(), nb, s), "fwd")
+        got.append(fl)
+        for a, b in zip(fl, ref):
+            assert close(a[P0:], b[P0:], 1e-5)
+    for fl in got[1:]:
+        assert all(torch.equal(a[P0:], b[P0:]) for a, b in zip(fl, got[0]))
+    dS = upstream(bins, C, dev, 3)
+    tot, R = bins.tot_b[0], 6 + C
+    ref_s, ps = torch.zeros(tot, R, device=dev), []
+    RH._render_bwd(lib, bins, 0, C, RH.FLAG_FIELDS | flags, (1, bins.n_levels), mask, (None,) * 5 + dS, ref_s, None, s)
+    for cap in (coarse, 2 * coarse):
+        sums = torch.zeros(tot, R, device=dev)
+        _lib.check(lib.splat_render_fields_auto_bwd(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), bins.p(0, "pq"),
+                                                    tot, C, H, W, TILE, flags, lvr, mask, cap, *[t.data_ptr() for t in dS],
+                                                    sums.data_ptr(), s), "bwd")
+        ps.append(sums)
+        for k in range(R):
+            assert close(sums[:, k], ref_s[:, k], 1e-5), k
+    assert torch.equal(*ps)
+    nb = lib.splat_fields_auto_workspace_bytes(C, H, W, TILE, lvr, mask, coarse)
+    assert nb >= 4 * (2 + C) * max(64, TILE * TILE) * (coarse >> auto_shift(coarse))
+    assert lib.splat_render_fields_auto(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), C, H, W, TILE, flags, lvr,
+                                        mask, coarse, *[t.data_ptr() for t in ref], ws.data_ptr(), nb - 1, s) == 5
