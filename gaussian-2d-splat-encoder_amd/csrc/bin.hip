@@ -75,6 +75,69 @@ __device__ __forceinline__ int block256_excl(int v, int* s_w, int& total) {
 constexpr int kSumCols = 1 + kMaxLevels;
 constexpr int kMaxRows = 1024;   // the row plan takes level tables of at most this many tile rows
 
+// Activated scale (sy, sx) of splat g (`scale` holds raw log-scales with act).
+__device__ __forceinline__ float2 splat_scale(const float* __restrict__ scale, int g, int act) {
+  const float2 s = reinterpret_cast<const float2*>(scale)[g];
+  return act ? make_float2(activate_scale(s.x), activate_scale(s.y)) : s;
+}
+
+// Decoded record of splat g (RecSlot), with centre m = (y, x) and activated scale s.
+struct SplatRecord {
+  float4 r[4];
+};
+template <int C>
+__device__ __forceinline__ SplatRecord splat_record(float2 m, float2 s, const float* __restrict__ theta,
+                                                    const float* __restrict__ opacity, const float* __restrict__ color,
+                                                    int g) {
+  float sn = 0.f, cs = 1.f;
+  if (theta) {   // the float32 values nearest cos and sin of the float32 angle (double sincos, rounded once)
+    double sd, cd;
+    sincos((double)theta[g], &sd, &cd);
+    sn = (float)sd;
+    cs = (float)cd;
+  }
+  const float ky = kWhiten / s.x, kx = kWhiten / s.y;
+  float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
+  col.x = color[(size_t)g * C];
+  if (C > 1) col.y = color[(size_t)g * C + 1];
+  if (C > 2) col.z = color[(size_t)g * C + 2];
+  if (C > 3) col.w = color[(size_t)g * C + 3];
+  const float op = opacity[g];
+  return {{make_float4(m.x, m.y, cs * ky, sn * ky), make_float4(-sn * kx, cs * kx, op, log2f(op)), col,
+           make_float4(s.x, s.y, cs, sn)}};
+}
+
+// Tile rect (tx0, ty0, width, level) of splat g and its height *h (not positive: an empty or inverted rect).
+__device__ __forceinline__ int4 splat_rect(float2 m, float2 s, int g, const LevelTable& L, const Routing& R, float fT,
+                                           float cutoff, int* h) {
+  int lev = 0;
+  // level: render_triton.py:925-932 + 950-952 (octave), :904-913 (coarse/fine split)
+  if (R.mode == 1) {
+    const float px = fmaxf(s.x, s.y) * R.rep;
+    const float o = ceilf(log2f(fmaxf(px * R.inv_base, 1e-6f)));
+    lev = (int)fminf(fmaxf(o, 0.f), (float)R.max_oct);
+  } else if (R.mode == 2) {
+    lev = g < R.n_coarse ? 1 : 0;
+  } else if (R.mode == 3) {
+    lev = min(g / R.n_coarse, L.n - 1);
+  }
+  const float fH = (float)L.H[lev], fW = (float)L.W[lev];
+  const float xmax = (float)(L.ntx[lev] - 1);
+  const float ymax = (float)((L.tbase[lev + 1] - L.tbase[lev]) / L.ntx[lev] - 1);
+  // render_triton.py:367-377, one rounding per operation.
+  const float cx = m.y * fW;
+  const float cy = m.x * fH;
+  const float rr = cutoff * fmaxf(s.x, s.y);
+  const float rx = rr * fW;
+  const float ry = rr * fH;
+  const int tx0 = (int)fminf(fmaxf(floorf((cx - rx) / fT), 0.f), xmax);
+  const int tx1 = (int)fminf(fmaxf(floorf((cx + rx) / fT), 0.f), xmax);
+  const int ty0 = (int)fminf(fmaxf(floorf((cy - ry) / fT), 0.f), ymax);
+  const int ty1 = (int)fminf(fmaxf(floorf((cy + ry) / fT), 0.f), ymax);
+  *h = ty1 - ty0 + 1;
+  return make_int4(tx0, ty0, tx1 - tx0 + 1, lev);
+}
+
 // Reach of a splat (exact path): the box (y0, y1, x0, x1) outside which its falloff exp2(-m) and opacity * falloff =
 // exp2(log2(op) - m), m = u^2 + v^2, are zero in float32 (v_exp_f32 flushes results below 2^-126): the bounding box
 // of the ellipse m <= 127.5 + max(log2(op), 0), in which 1.5 covers the rounding of m, slightly widened for the box's
@@ -123,59 +186,25 @@ __global__ __launch_bounds__(kBlock) void k_decode_count(
   float4 box = make_float4(INFINITY, -INFINITY, INFINITY, -INFINITY);   // the splat's reach (exact path)
   if (g < N) {
     const float2 m = reinterpret_cast<const float2*>(mu)[g];      // (y, x)
-    float2 s = reinterpret_cast<const float2*>(scale)[g];   // (sy, sx), or raw log-scales with act
-    if (act) s = make_float2(activate_scale(s.x), activate_scale(s.y));
-    float sn = 0.f, cs = 1.f;
-    if (theta) {   // the float32 values nearest cos and sin of the float32 angle (double sincos, rounded once)
-      double sd, cd;
-      sincos((double)theta[g], &sd, &cd);
-      sn = (float)sd;
-      cs = (float)cd;
-    }
-    const float ky = kWhiten / s.x, kx = kWhiten / s.y;
-    float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
-    col.x = color[(size_t)g * C];
-    if (C > 1) col.y = color[(size_t)g * C + 1];
-    if (C > 2) col.z = color[(size_t)g * C + 2];
-    if (C > 3) col.w = color[(size_t)g * C + 3];
+    const float2 s = splat_scale(scale, g, act);
+    const SplatRecord d = splat_record<C>(m, s, theta, opacity, color, g);
     const int t = threadIdx.x;
-    s_rec[rec_slot(t, 0)] = make_float4(m.x, m.y, cs * ky, sn * ky);
-    const float op = opacity[g];
-    s_rec[rec_slot(t, 1)] = make_float4(-sn * kx, cs * kx, op, log2f(op));
-    s_rec[rec_slot(t, 2)] = col;
-    s_rec[rec_slot(t, 3)] = make_float4(s.x, s.y, cs, sn);
+    s_rec[rec_slot(t, 0)] = d.r[0];
+    s_rec[rec_slot(t, 1)] = d.r[1];
+    s_rec[rec_slot(t, 2)] = d.r[2];
+    s_rec[rec_slot(t, 3)] = d.r[3];
     if (!BIN && reach) {
-      box = splat_reach(m, s, cs, sn, op, col);
+      box = splat_reach(m, s, d.r[3].z, d.r[3].w, d.r[1].z, d.r[2]);
       reach[g] = box;
     }
     if (BIN) {
-      // level: render_triton.py:925-932 + 950-952 (octave), :904-913 (coarse/fine split)
-      if (R.mode == 1) {
-        const float px = fmaxf(s.x, s.y) * R.rep;
-        const float o = ceilf(log2f(fmaxf(px * R.inv_base, 1e-6f)));
-        lev = (int)fminf(fmaxf(o, 0.f), (float)R.max_oct);
-      } else if (R.mode == 2) {
-        lev = g < R.n_coarse ? 1 : 0;
-      } else if (R.mode == 3) {
-        lev = min(g / R.n_coarse, L.n - 1);
-      }
-      const float fH = (float)L.H[lev], fW = (float)L.W[lev];
-      const float xmax = (float)(L.ntx[lev] - 1);
-      const float ymax = (float)((L.tbase[lev + 1] - L.tbase[lev]) / L.ntx[lev] - 1);
-      // render_triton.py:367-377, one rounding per operation.
-      const float cx = m.y * fW;
-      const float cy = m.x * fH;
-      const float rr = cutoff * fmaxf(s.x, s.y);
-      const float rx = rr * fW;
-      const float ry = rr * fH;
-      const int tx0 = (int)fminf(fmaxf(floorf((cx - rx) / fT), 0.f), xmax);
-      const int tx1 = (int)fminf(fmaxf(floorf((cx + rx) / fT), 0.f), xmax);
-      const int ty0 = (int)fminf(fmaxf(floorf((cy - ry) / fT), 0.f), ymax);
-      const int ty1 = (int)fminf(fmaxf(floorf((cy + ry) / fT), 0.f), ymax);
-      const int w = tx1 - tx0 + 1, h = ty1 - ty0 + 1;
+      int h;
+      const int4 rc = splat_rect(m, s, g, L, R, fT, cutoff, &h);
+      lev = rc.w;
+      const int ty0 = rc.y, w = rc.z;
       bad = (w < 1) || (h < 1);
       cnt = bad ? 0 : w * h;
-      rect[g] = make_int4(tx0, ty0, w, lev);   // the rect height is not needed past this point
+      rect[g] = rc;   // the rect height is not needed past this point
       counts[g] = cnt;
       if (cnt) {
         if (rowhist) {   // rows [r0, r0 + h) each get one unit of w pairs
@@ -1459,6 +1488,210 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
   flush();
 }
 
+// ---------------------------------------------------------------------------------------------- small plan
+// The whole binning of a small problem in one workgroup and one launch (small_plan): with four launches, each a chain of
+// memory round trips over a handful of workgroups, a 64 x 64 render of 1,024 splats spent 25 us in them and more in the gaps
+// between them, against 17 us here (a forward 49 -> 38 us). Per tile one bit per splat (LDS): a splat's place in the tile's list is the number
+// of bits below its own, which is splat order without a sort. DECODE: all of splat_bin, the pair list for up to `cap`
+// pairs; where there are more, the row plan's histogram instead (the host asks for the pair phase again); else the pair
+// phase alone, from rect and offsets. A splat's tiles are walked by its own thread, so lists past kSmallPairs pairs go to
+// the row plan: 300,000 pairs (2,048 splats over 150 tiles each) would take about 100 us here.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallMaxN = 2 * kSmallThreads;   // one splat per thread, or two consecutive ones
+constexpr int kSmallLds = 60 * 1024;
+constexpr int kSmallPairs = 24576;
+
+__host__ __device__ __forceinline__ int small_words(int N) { return (N + 31) >> 5; }
+// LDS bytes: masks [words][tiles], their prefix counts (16 bits), tile starts
+__host__ __device__ __forceinline__ size_t small_lds(int N, int nt) {
+  return (size_t)small_words(N) * nt * 4 + (size_t)nt * 4 + (size_t)small_words(N) * nt * 2;
+}
+// The row plan's histogram fits them: a row needs a word per 256 splats and one more, and has at least one tile.
+static_assert(kSmallMaxN / kBlock + 1 <= kSmallMaxN / 32 + 1, "words per row");
+
+template <int C, bool DECODE, int IT>
+__global__ __launch_bounds__(kSmallThreads) void k_bin_small(
+    const float* __restrict__ mu, const float* __restrict__ scale, const float* __restrict__ theta,
+    const float* __restrict__ opacity, const float* __restrict__ color, int N, LevelTable L, Routing R, float fT,
+    float cutoff, int act, float4* __restrict__ rec, int4* __restrict__ rect, int* __restrict__ offsets,
+    long long* __restrict__ info, long long* __restrict__ mirror, int cap, int* __restrict__ gid_sorted,
+    int* __restrict__ tile_starts, int* __restrict__ pair_splat, int* __restrict__ pair_q, int2* __restrict__ rowhist,
+    int2* __restrict__ rtot, int nb) {
+  extern __shared__ int s_dyn[];
+  constexpr int NW = kSmallThreads / 64;
+  __shared__ int s_w[NW], s_lev[kMaxLevels], s_bad;
+  const int nt = L.tbase[L.n], W = small_words(N);
+  unsigned* mask = reinterpret_cast<unsigned*>(s_dyn);
+  int* start = s_dyn + (size_t)W * nt;
+  unsigned short* pre = reinterpret_cast<unsigned short*>(start + nt);
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  for (int i = t; i < W * nt; i += kSmallThreads) mask[i] = 0u;
+  if (t < kMaxLevels) s_lev[t] = 0;
+  if (t == 0) s_bad = 0;
+  int4 rc[IT];
+  int hh[IT], cnt[IT], sum = 0;
+  bool bad = false;
+  float2 m[IT], s[IT];
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int g = t * IT + k;
+    cnt[k] = hh[k] = 0;
+    rc[k] = make_int4(0, 0, 0, 0);
+    if (g < N) {
+      if (DECODE) {
+        m[k] = reinterpret_cast<const float2*>(mu)[g];
+        s[k] = splat_scale(scale, g, act);
+        rc[k] = splat_rect(m[k], s[k], g, L, R, fT, cutoff, &hh[k]);
+        const bool b = rc[k].z < 1 || hh[k] < 1;
+        bad |= b;
+        cnt[k] = b ? 0 : rc[k].z * hh[k];
+        rect[g] = rc[k];
+      } else {
+        rc[k] = rect[g];
+        cnt[k] = offsets[g + 1] - offsets[g];
+        hh[k] = cnt[k] > 0 ? cnt[k] / rc[k].z : 0;
+      }
+    }
+    sum += cnt[k];
+  }
+  const int inc = wave_incl_scan<int>(sum, lane);
+  if (lane == 63) s_w[wv] = inc;
+  __syncthreads();   // also: the masks are zero
+  int off = inc - sum, tot = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const int x = s_w[w];
+    if (w < wv) off += x;
+    tot += x;
+  }
+  int o0[IT];
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int g = t * IT + k;
+    o0[k] = off;
+    if (DECODE && g < N) offsets[g] = off;
+    if (DECODE && g == N - 1) offsets[N] = tot;
+    if (DECODE && cnt[k]) atomicAdd(&s_lev[rc[k].w], cnt[k]);
+    off += cnt[k];
+    const int h = cnt[k] ? hh[k] : 0;
+    const int tb = L.tbase[rc[k].w] + rc[k].x, ntx = L.ntx[rc[k].w];
+    for (int y = 0; y < h; ++y)
+      for (int x = 0; x < rc[k].z; ++x)
+        atomicOr(&mask[(g >> 5) * nt + tb + (rc[k].y + y) * ntx + x], 1u << (g & 31));
+  }
+  if (DECODE && bad) s_bad = 1;
+  __syncthreads();
+  const bool flagged = DECODE ? s_bad != 0 : info && (info[1] & 3);
+  if (DECODE) {   // the totals first: the host waits for them
+    if (t == 0) {
+      put_info(info, mirror, 0, tot);
+      put_info(info, mirror, 1, s_bad ? 1 : 0);
+    }
+    if (t < L.n) put_info(info, mirror, 2 + t, s_lev[t]);
+    if (mirror && t < 64) __threadfence_system();
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int g = t * IT + k;
+      if (g < N) {
+        const SplatRecord d = splat_record<C>(m[k], s[k], theta, opacity, color, g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rec[(size_t)g * 4 + i] = d.r[i];
+      }
+    }
+  }
+  if (tot == 0 || tot > cap || flagged) {   // the empty list (render_triton.py:392-394), or one the host asks for again
+    for (int i = t; i <= nt; i += kSmallThreads) tile_starts[i] = 0;
+    if (t == 0) gid_sorted[0] = 0;
+    if (!DECODE || !rowhist || flagged || tot == 0) return;
+    // what the count pass and its row scan leave for the row plan: rows x (nb blocks' units, then pairs) in the masks'
+    // and starts' place (nb + 1 <= W + 1 words per row, and at least as many tiles as rows)
+    __syncthreads();
+    const int nrows = L.rbase[L.n], K = nb + 1;
+    for (int i = t; i < nrows * K; i += kSmallThreads) s_dyn[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int r0 = L.rbase[rc[k].w] + rc[k].y;
+      for (int y = 0; y < (cnt[k] ? hh[k] : 0); ++y) {
+        atomicAdd(&s_dyn[(r0 + y) * K + (t * IT + k) / kBlock], 1);
+        atomicAdd(&s_dyn[(r0 + y) * K + nb], rc[k].z);
+      }
+    }
+    __syncthreads();
+    for (int r = t; r < nrows; r += kSmallThreads) {
+      int run = 0;
+      for (int b = 0; b < nb; ++b) {
+        rowhist[(size_t)r * nb + b] = make_int2(run, 0);
+        run += s_dyn[r * K + b];
+      }
+      rtot[r] = make_int2(run, s_dyn[r * K + nb]);
+    }
+    return;
+  }
+  // per tile: the bits before each word (the words in `parts` shares, one thread each), then the tiles' starts
+  __shared__ int s_part[kSmallThreads];
+  const int parts = max(1, min(W, kSmallThreads / nt)), share = (W + parts - 1) / parts;
+  int run = 0;
+  for (int i0 = 0; i0 < nt; i0 += kSmallThreads) {   // more than one round only with one part
+    const int part = parts > 1 ? t / nt : 0, i = parts > 1 ? t - part * nt : i0 + t;
+    const int w0 = min(W, part * share), w1 = min(W, w0 + share);
+    const bool act = part < parts && i < nt;
+    int c = 0;
+    if (act)
+      for (int w = w0; w < w1; ++w) c += __popc(mask[w * nt + i]);
+    int before = 0;
+    if (parts > 1) {
+      s_part[t] = c;
+      __syncthreads();
+      c = 0;
+      if (act)
+        for (int k = 0; k < parts; ++k) {   // independent loads
+          const int x = s_part[k * nt + i];
+          before += k < part ? x : 0;
+          c += x;
+        }
+    }
+    if (act)
+      for (int w = w0, b = before; w < w1; ++w) {
+        pre[w * nt + i] = (unsigned short)b;
+        b += __popc(mask[w * nt + i]);
+      }
+    if (part > 0) c = 0;   // the tile's count, once
+    const int ic = wave_incl_scan<int>(c, lane);
+    __syncthreads();   // s_w has been read
+    if (lane == 63) s_w[wv] = ic;
+    __syncthreads();
+    int st = run + ic - c;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const int x = s_w[w];
+      if (w < wv) st += x;
+      run += x;
+    }
+    if (act && part == 0) {
+      start[i] = st;
+      tile_starts[i] = st;
+    }
+  }
+  if (t == 0) tile_starts[nt] = tot;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int g = t * IT + k;
+    const int h = cnt[k] ? hh[k] : 0;
+    const int tb = L.tbase[rc[k].w] + rc[k].x, ntx = L.ntx[rc[k].w], wd = (g >> 5) * nt;
+    int q = o0[k];
+    for (int y = 0; y < h; ++y)
+      for (int x = 0; x < rc[k].z; ++x, ++q) {
+        const int i = tb + (rc[k].y + y) * ntx + x;
+        const int p = start[i] + pre[wd + i] + __popc(mask[wd + i] & ((1u << (g & 31)) - 1u));
+        gid_sorted[p] = g;
+        if (pair_q) pair_q[p] = q;
+        if (pair_splat) pair_splat[q] = g;
+      }
+  }
+}
+
 // ----------------------------------------------------------------------------------------------------
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -1532,6 +1765,11 @@ static CountPlan plan_count(const LevelTable& L, int N) {
   }
   c.total = o;
   return c;
+}
+
+// The small plan takes problems whose bit masks fit 60 KB of LDS.
+static bool small_plan(const LevelTable& L, int N) {
+  return N >= 1 && N <= kSmallMaxN && small_lds(N, L.tbase[L.n]) <= (size_t)kSmallLds;
 }
 
 static size_t unit_bytes(long long tot) { return align256(sizeof(int) * (size_t)(tot > 0 ? tot : 1)); }
@@ -1659,6 +1897,26 @@ int bin_count_launch(const float* mu, const float* scale, const float* theta, co
   return check_launch("splat_bin_count");
 }
 
+// Launch of a small problem's whole binning (k_bin_small). Arguments already validated.
+int bin_small_launch(const float* mu, const float* scale, const float* theta, const float* opacity, const float* color,
+                     int C, int N, const LevelTable& L, const Routing& R, int TILE, float cutoff, int flags, float* rec,
+                     int* rect, int* offsets, long long* info, long long* mirror, int cap, int* gid_sorted,
+                     int* tile_starts, int* pair_splat, int* pair_q, void* ws, hipStream_t st) {
+  const CountPlan cp = plan_count(L, N);
+  int2* rowhist = cp.rows ? (int2*)((char*)ws + cp.off_rowhist) : nullptr;
+  int2* rtot = cp.rows ? (int2*)((char*)ws + cp.off_rtot) : nullptr;
+#define SPLAT_SMALL(CC) (N <= kSmallThreads ? k_bin_small<CC, true, 1> : k_bin_small<CC, true, 2>)
+  auto kernel = SPLAT_SMALL(4);
+  switch (C) { case 1: kernel = SPLAT_SMALL(1); break; case 2: kernel = SPLAT_SMALL(2); break;
+               case 3: kernel = SPLAT_SMALL(3); break; default: break; }
+#undef SPLAT_SMALL
+  kernel<<<1, kSmallThreads, small_lds(N, L.tbase[L.n]), st>>>(
+      mu, scale, theta, opacity, color, N, L, R, (float)TILE, cutoff, (flags & kFlagLogScale) ? 1 : 0,
+      reinterpret_cast<float4*>(rec), reinterpret_cast<int4*>(rect), offsets, info, mirror, cap, gid_sorted, tile_starts,
+      pair_splat, pair_q, rowhist, rtot, cp.nb);
+  return check_launch("k_bin_small");
+}
+
 // Launches of the pair phase. Exact (dinfo NULL): `t` is the pair count. Speculative (dinfo = the count
 // phase's device info): `t` is the capacity the buffers and the grids are sized for, and the kernels take
 // the count from dinfo (an empty list when it exceeds t). Arguments already validated; ws holds
@@ -1671,6 +1929,14 @@ int bin_pairs_launch(const int* rect, const int* offsets, const void* ws_count, 
     k_fill_i32<<<div_up(nt + 1, 256), 256, 0, st>>>(tile_starts, nt + 1, 0);
     k_fill_i32<<<1, 64, 0, st>>>(gid_sorted, 1, 0);
     return check_launch("splat_bin_pairs(empty)");
+  }
+  if (small_plan(L, N) && t <= kSmallPairs) {   // from rect and offsets alone
+    auto kernel = N <= kSmallThreads ? k_bin_small<1, false, 1> : k_bin_small<1, false, 2>;
+    kernel<<<1, kSmallThreads, small_lds(N, nt), st>>>(
+        nullptr, nullptr, nullptr, nullptr, nullptr, N, L, Routing{}, 1.f, 0.f, 0, nullptr,
+        reinterpret_cast<int4*>(const_cast<int*>(rect)), const_cast<int*>(offsets), const_cast<long long*>(dinfo), nullptr,
+        t, gid_sorted, tile_starts, pair_splat, pair_q, nullptr, nullptr, 0);
+    return check_launch("k_bin_small");
   }
   const CountPlan cp = plan_count(L, N);
   if (cp.rows) {
@@ -1974,8 +2240,11 @@ int splat_bin(const float* mu, const float* scale, const float* theta, const flo
   volatile long long* ih = info_host;
   if (mirror)
     for (int i = 0; i < ninfo; ++i) ih[i] = kUnsetInfo;
-  int rc = bin_count_launch(mu, scale, theta, opacity, color, C, N, L, R, TILE, cutoff, flags, rec, rect, offsets,
-                            info, mirror, ws_count, st);
+  const bool small = spec && pair_cap <= kSmallPairs && small_plan(L, N);   // count and pair phase in one launch
+  int rc = small ? bin_small_launch(mu, scale, theta, opacity, color, C, N, L, R, TILE, cutoff, flags, rec, rect, offsets,
+                                    info, mirror, (int)pair_cap, gid_sorted, tile_starts, pair_splat, pair_q, ws_count, st)
+                 : bin_count_launch(mu, scale, theta, opacity, color, C, N, L, R, TILE, cutoff, flags, rec, rect,
+                                    offsets, info, mirror, ws_count, st);
   if (rc) return rc;
   if (!mirror) {   // pageable totals: a copy and the event read_totals waits for
     hipEvent_t ev = readback_event();
@@ -1983,7 +2252,7 @@ int splat_bin(const float* mu, const float* scale, const float* theta, const flo
         hipEventRecord(ev, st) != hipSuccess)
       return set_error(kHipError, "splat_bin: queueing the read of the pair totals failed");
   }
-  if (spec) {
+  if (spec && !small) {
     rc = bin_pairs_launch(rect, offsets, ws_count, N, L, (int)pair_cap, info, gid_sorted, tile_starts, pair_splat, pair_q,
                           ws_pairs, st);
     if (rc) return rc;
