@@ -2,8 +2,8 @@
 // render_triton.py:423-517 (forward) and 602-720 (backward), plus the exact (unculled) path of :58-266.
 //
 // Forward: one wave64 per TILE x TILE tile (8 x 8 = one pixel per lane). The tile's pair list is walked in
-// pair order; the pair's splat id and its decoded record are wave-uniform, so they are read with scalar
-// loads into SGPRs and every lane evaluates its own pixel. Per pixel-pair: whitened offsets u, v; falloff
+// pair order, 64 pairs at a time: the wave's lanes gather the decoded records into LDS, and every lane evaluates its
+// own pixel of every pair. Per pixel-pair: whitened offsets u, v; falloff
 // exp2(-(u^2 + v^2)); a = min(op * falloff, 1 - 1e-4); S_log += log2(1 - a) (scaled by ln 2 once);
 // S_a += w; S_ac += w * colour, with w = a or the odds a / (1 - a).
 //
@@ -63,6 +63,14 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
          (__int_as_float(__builtin_amdgcn_readlane(b, 32)) + __int_as_float(__builtin_amdgcn_readlane(b, 48)));
 }
 
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// d[i] = a of lane 4 (lane / 4) + i, times the lane's own b, plus c[i]: sixteen 4 x 4 outer products, one per quad of
+// lanes, each element rounded as one FMA. Takes every lane of the wave, masked or not (EXEC does not apply).
+__device__ __forceinline__ floatx4 outer4(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
 // A value every lane of the wave holds, as a wave-uniform (scalar) value.
 __device__ __forceinline__ float uniform_f(float x) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
@@ -82,71 +90,91 @@ __device__ __forceinline__ float2 offsets_at(float py0, float px0, float gy, flo
   return make_float2(fmaf(B, dx, pu) + fmaf(A, dy, -pu), fmaf(D, dx, pv) + fmaf(Cc, dy, -pv));
 }
 
-// One pixel-pair of the per-tile forward: (u0, v0) are the pair's whitened offsets at the tile's reference pixel
-// centre, (ly, lx) the lane's pixel centre relative to it, so u = A ly + B lx + u0 and v = Cc ly + D lx + v0.
-// t carries the running product of the group's (1 - a) factors.
-template <int C, bool ODDS, bool CLAMP>
-__device__ __forceinline__ void fwd_tile_pair(const float* __restrict__ r, float2 uv0, float ly, float lx, float& t,
-                                              float& s_a, float* sc) {
-  const float u = fmaf(r[R_A], ly, fmaf(r[R_B], lx, uv0.x));
-  const float v = fmaf(r[R_CC], ly, fmaf(r[R_D], lx, uv0.y));
-  const float fo = hw_exp2(-fmaf(u, u, fmaf(v, v, -r[R_LOP])));
-  const float a = CLAMP ? fminf(fo, kClamp) : fo;
-  float w;
-  if (ODDS) {
-    const float oma = one_minus_alpha(1.f - a, fo, fmaf(u, u, v * v), r[R_OP], 1.f - r[R_OP]);
-    w = a * hw_rcp(oma);
-    t *= oma;
-  } else {
-    w = a;
-    t = fmaf(-a, t, t);   // t (1 - a), one rounding
-  }
-  s_a += w;
+// A wave's batch of up to 64 pairs of the per-tile forward in LDS (floats): whitened offsets (u0, v0) at the tile's
+// reference pixel centre, rotation columns (B, D) and (A, Cc), the rows of the colour sums (1 and three channels, or
+// four), log2 of the opacity and the opacity.
+enum FwdBatch : int { F_UV = 0, F_BD = 128, F_AC = 256, F_COL = 384, F_LOP = 640, F_OP = 704, kFwdBatch = 768 };
+
+// N (4 or 8) pixel-pairs of the per-tile forward, pairs j .. j + N - 1 of the batch sb, with (ly, lx) the lane's pixel
+// centre relative to the reference pixel: u = A ly + (B lx + u0) and v = Cc ly + (D lx + v0) of two pairs come from
+// three matrix instructions (outer4; eight FMAs otherwise), and S_a with the colour sums, acc = (S_a, S_ac[0..2])
+// (C = 4: S_ac alone), from one per pair (four FMAs). sl adds log2 of the product of the (1 - a) factors: each is
+// >= 1e-4, so the product of eight stays >= 1e-32, a normal float.
+// What bounds it is the vector unit's issue: an FMA takes it about 4.4 cycles, one of these matrix instructions about 9,
+// so 2.5 of them do the work of 8 FMAs (35 cycles) in 22; each change between the two kinds costs about 8 more, hence the
+// three phases, kept apart by scheduling barriers, over as many pairs as the registers of eight waves per SIMD hold (seven
+// with the odds, which keep the opacities too). f32 matrix instructions don't run beside the vector unit's, whatever
+// their size. 768 x 768, 92,160 splats: 54.4-54.9 us with FMAs on records from scalar loads, 58.0 us with the kinds
+// interleaved as the compiler orders them, 51.5-52.6 us so (2048 x 2048: 761, 855, 720 us); the coarse levels' launch,
+// whose few waves also waited for the scalar loads, 55.1 -> 44.5 us, its composite with the odds 70.1 -> 60.4 us.
+template <int C, bool ODDS, bool CLAMP, int N>
+__device__ __forceinline__ void fwd_group(const float* sb, int j, int quad, float ly, float lx, float& sl, float& s_a,
+                                          floatx4& acc) {
+  floatx4 uv[N / 2];   // u, v of pair j + 2 k, then of pair j + 2 k + 1
+  float g[3][N / 2], gc[N], lop[N], op[N], w[N];
 #pragma unroll
-  for (int c = 0; c < C; ++c) sc[c] = fmaf(w, r[R_COL + c], sc[c]);
-}
-
-// Pairs [b0, b1) of one batch (their offsets at the reference pixel in s_uv[0, b1 - b0)), in groups of four:
-// ids and records through scalar loads, offsets by LDS broadcast. The (1 - a) factors of eight pairs (two
-// groups) are multiplied before one log2: each factor is >= 1e-4, so the product stays >= 1e-32, a normal float.
-template <int C, bool ODDS, bool CLAMP>
-__device__ __forceinline__ void fwd_group4(const float* __restrict__ rec, const int* __restrict__ gid, int i, int j,
-                                           const float2* s_uv, float ly, float lx, float& t, float& s_a, float* sc) {
-  const float* r0 = rec + (size_t)gid[i] * kRec;
-  const float* r1 = rec + (size_t)gid[i + 1] * kRec;
-  const float* r2 = rec + (size_t)gid[i + 2] * kRec;
-  const float* r3 = rec + (size_t)gid[i + 3] * kRec;
-  fwd_tile_pair<C, ODDS, CLAMP>(r0, s_uv[j], ly, lx, t, s_a, sc);
-  fwd_tile_pair<C, ODDS, CLAMP>(r1, s_uv[j + 1], ly, lx, t, s_a, sc);
-  fwd_tile_pair<C, ODDS, CLAMP>(r2, s_uv[j + 2], ly, lx, t, s_a, sc);
-  fwd_tile_pair<C, ODDS, CLAMP>(r3, s_uv[j + 3], ly, lx, t, s_a, sc);
-}
-
-template <int C, bool ODDS, bool CLAMP>
-__device__ __forceinline__ void fwd_batch(const float* __restrict__ rec, const int* __restrict__ gid, int b0, int b1,
-                                          const float2* s_uv, float ly, float lx, float& sl, float& s_a, float* sc) {
-  int i = b0;
-  for (; i + 8 <= b1; i += 8) {
-    float t = 1.f;
-    fwd_group4<C, ODDS, CLAMP>(rec, gid, i, i - b0, s_uv, ly, lx, t, s_a, sc);
-    fwd_group4<C, ODDS, CLAMP>(rec, gid, i + 4, i + 4 - b0, s_uv, ly, lx, t, s_a, sc);
-    sl += hw_log2(t);
+  for (int k = 0; k < N / 2; ++k) {
+    const float* b = sb + 2 * (j + 2 * k) + quad;
+    g[0][k] = b[F_UV];
+    g[1][k] = b[F_BD];
+    g[2][k] = b[F_AC];
   }
-  if (i < b1) {   // at most seven pairs left: one product, one log2
-    float t = 1.f;
-    if (i + 4 <= b1) {
-      fwd_group4<C, ODDS, CLAMP>(rec, gid, i, i - b0, s_uv, ly, lx, t, s_a, sc);
-      i += 4;
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < N / 2; ++k) uv[k] = outer4(g[0][k], 1.f, floatx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+  for (int k = 0; k < N / 2; ++k) uv[k] = outer4(g[1][k], lx, uv[k]);
+#pragma unroll
+  for (int k = 0; k < N / 2; ++k) uv[k] = outer4(g[2][k], ly, uv[k]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < N; k += 4) {
+    const floatx4 l4 = *reinterpret_cast<const floatx4*>(sb + F_LOP + j + k);
+    floatx4 o4 = l4;
+    if (ODDS) o4 = *reinterpret_cast<const floatx4*>(sb + F_OP + j + k);
+    for (int e = 0; e < 4; ++e) {
+      lop[k + e] = l4[e];
+      op[k + e] = o4[e];
     }
-    for (; i < b1; ++i) fwd_tile_pair<C, ODDS, CLAMP>(rec + (size_t)gid[i] * kRec, s_uv[i - b0], ly, lx, t, s_a, sc);
-    sl += hw_log2(t);
   }
+#pragma unroll
+  for (int k = 0; k < N; ++k) gc[k] = sb[F_COL + 4 * (j + k) + quad];
+  float t = 1.f;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float u = uv[k / 2][2 * (k & 1)], v = uv[k / 2][2 * (k & 1) + 1];
+    const float fo = hw_exp2(-fmaf(u, u, fmaf(v, v, -lop[k])));
+    const float a = CLAMP ? fminf(fo, kClamp) : fo;
+    if (ODDS) {
+      const float oma = one_minus_alpha(1.f - a, fo, fmaf(u, u, v * v), op[k], 1.f - op[k]);
+      w[k] = a * hw_rcp(oma);
+      t *= oma;
+    } else {
+      w[k] = a;
+      t = fmaf(-a, t, t);   // t (1 - a), one rounding
+    }
+    if (C > 3) s_a += w[k];
+  }
+  sl += hw_log2(t);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < N; ++k) acc = outer4(gc[k], w[k], acc);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The n pairs of a batch (n rounded up to four: the batch's fill adds nothing).
+template <int C, bool ODDS, bool CLAMP>
+__device__ __forceinline__ void fwd_batch(const float* sb, int n, int quad, float ly, float lx, float& sl, float& s_a,
+                                          floatx4& acc) {
+  int j = 0;
+  for (; j + 4 < n; j += 8) fwd_group<C, ODDS, CLAMP, 8>(sb, j, quad, ly, lx, sl, s_a, acc);
+  if (j < n) fwd_group<C, ODDS, CLAMP, 4>(sb, j, quad, ly, lx, sl, s_a, acc);
 }
 
 // Forward sums of one pixel over pairs [i0, i1) of the tile's list, in batches of 64 pairs. At the start of a
-// batch lane j computes the offsets (u0, v0) of pair j at the tile's reference pixel centre (py0, px0) into the
-// wave's LDS row s_uv, and a ballot tells whether any pair of the batch can reach the alpha clamp; the pixel loop
-// then reads the offsets by broadcast while the pairs' ids and records come through scalar loads (SGPR operands).
+// batch lane j gathers pair j's record and writes what the pixel loop needs of it to the wave's LDS batch sb, with
+// the offsets (u0, v0) at the tile's reference pixel centre (py0, px0), and a ballot tells whether any pair of the
+// batch can reach the alpha clamp; lanes past the list write a pair of falloff 0.
 // The reference pixel is the tile's middle one (inside the canvas), so that its offsets and the pixels' own offsets
 // from it stay within about half the pair's whitened span over the tile: their rounding, about one ulp of that
 // size, is shared by the tile's pixels (for a splat far smaller than the tile, a span of hundreds, a few 1e-5 of
@@ -154,26 +182,46 @@ __device__ __forceinline__ void fwd_batch(const float* __restrict__ rec, const i
 // S_log is accumulated in log2 units, one log2 per eight pairs (see fwd_batch).
 template <int C, bool ODDS>
 __device__ __forceinline__ void fwd_tile_pixel(const float* __restrict__ rec, const int* __restrict__ gid, int i0,
-                                               int i1, float py0, float px0, float ly, float lx, float2* s_uv,
+                                               int i1, float py0, float px0, float ly, float lx, float* sb,
                                                int lane, float& sl, float& s_a, float* sc) {
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int quad = lane & 3;
   for (int b0 = i0; b0 < i1; b0 += 64) {
-    const int b1 = min(i1, b0 + 64);
+    const int n = min(i1 - b0, 64);
     bool clamp = false;
-    if (b0 + lane < b1) {
+    float2 uv = make_float2(0.f, 0.f), bd = uv, ac = uv;
+    float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
+    float lop = -1e30f, op = 0.f;
+    if (lane < n) {
       const float4* r4 = reinterpret_cast<const float4*>(rec) + (size_t)gid[b0 + lane] * 4;
       const float4 r0 = r4[0];   // gy, gx, A, B
       const float4 r1 = r4[1];   // Cc, D, op, log2(op)
-      s_uv[lane] = offsets_at(py0, px0, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
+      const float4 r2 = r4[2];
+      uv = offsets_at(py0, px0, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y);
+      bd = make_float2(r0.w, r1.y);
+      ac = make_float2(r0.z, r1.x);
+      col = C < 4 ? make_float4(1.f, r2.x, r2.y, r2.z) : r2;
+      lop = r1.w;
+      op = r1.z;
       clamp = __float_as_uint(r1.z) > kNoClampOpBits;
     }
+    *reinterpret_cast<float2*>(sb + F_UV + 2 * lane) = uv;
+    *reinterpret_cast<float2*>(sb + F_BD + 2 * lane) = bd;
+    *reinterpret_cast<float2*>(sb + F_AC + 2 * lane) = ac;
+    *reinterpret_cast<float4*>(sb + F_COL + 4 * lane) = col;
+    sb[F_LOP + lane] = lop;
+    if (ODDS) sb[F_OP + lane] = op;
     const bool any_clamp = __ballot(clamp) != 0;
     wave_lds_sync();
     if (any_clamp)
-      fwd_batch<C, ODDS, true>(rec, gid, b0, b1, s_uv, ly, lx, sl, s_a, sc);
+      fwd_batch<C, ODDS, true>(sb, n, quad, ly, lx, sl, s_a, acc);
     else
-      fwd_batch<C, ODDS, false>(rec, gid, b0, b1, s_uv, ly, lx, sl, s_a, sc);
+      fwd_batch<C, ODDS, false>(sb, n, quad, ly, lx, sl, s_a, acc);
     wave_lds_sync();
   }
+  if (C < 4) s_a = acc[0];
+#pragma unroll
+  for (int c = 0; c < C; ++c) sc[c] = acc[C < 4 ? c + 1 : c];
 }
 
 template <int C>
@@ -345,14 +393,14 @@ __host__ __device__ constexpr int fwd_threads() { return tile_threads(TILE) * S;
 enum Composite : int { kPlain = 0, kUps = 1, kBatch = 2 };
 
 template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S>
-__global__ __launch_bounds__((fwd_threads<TILE, S>())) void k_fwd_cull(
+__global__ __launch_bounds__((fwd_threads<TILE, S>())) __attribute__((amdgpu_waves_per_eu(S == 16 ? 4 : ODDS ? 7 : 8))) void k_fwd_cull(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L, int tb0,
     int ntiles, const float* __restrict__ bg, float* __restrict__ out, float* __restrict__ Tout,
     float* __restrict__ asum_out, float* __restrict__ fg_out, float* __restrict__ slog, float* __restrict__ sa,
     float* __restrict__ sac) {
   constexpr bool UPS = MODE == kUps, BATCH = MODE == kBatch;
   constexpr int NW = fwd_threads<TILE, S>() / 64;   // waves per workgroup
-  __shared__ float2 s_uv[NW][64];
+  __shared__ float4 s_batch[NW][kFwdBatch / 4];
   const TileAt ta = tile_at(L, tb0, ntiles);
   if (!((L.mask >> ta.l) & 1)) return;
   const int lane = (int)(threadIdx.x & 63);
@@ -372,23 +420,25 @@ __global__ __launch_bounds__((fwd_threads<TILE, S>())) void k_fwd_cull(
   float sl = 0.f, s_a = 0.f, sc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) sc[c] = 0.f;
-  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, s_uv[wid], lane, sl, s_a, sc);
+  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane, sl, s_a, sc);
   if (S > 1) {
-    __shared__ float s_part[S > 1 ? S - 1 : 1][2 + C][64];
+    static_assert((2 + C) * 64 <= kFwdBatch, "a wave's partial sums take the place of its batch");
     if (wv > 0) {
-      s_part[wv - 1][0][l] = sl;
-      s_part[wv - 1][1][l] = s_a;
+      float* part = reinterpret_cast<float*>(s_batch[wid]) + l;
+      part[0] = sl;
+      part[64] = s_a;
 #pragma unroll
-      for (int c = 0; c < C; ++c) s_part[wv - 1][2 + c][l] = sc[c];
+      for (int c = 0; c < C; ++c) part[64 * (2 + c)] = sc[c];
     }
     __syncthreads();
     if (wv > 0) return;
 #pragma unroll
-    for (int w = 0; w < S - 1; ++w) {
-      sl += s_part[w][0][l];
-      s_a += s_part[w][1][l];
+    for (int w = 1; w < S; ++w) {
+      const float* part = reinterpret_cast<const float*>(s_batch[S > 1 ? w : 0]) + l;
+      sl += part[0];
+      s_a += part[64];
 #pragma unroll
-      for (int c = 0; c < C; ++c) sc[c] += s_part[w][2 + c][l];
+      for (int c = 0; c < C; ++c) sc[c] += part[64 * (2 + c)];
     }
   }
   if (!valid) return;
@@ -429,12 +479,12 @@ __host__ __device__ constexpr int split_part_floats() { return (2 + C) * tile_th
 // items of an auto split launch over the tiles [t0, t1) instead, `nitems` of them in the buffer `part` (more are not
 // written: the launch was planned for fewer pairs and is repeated).
 template <int C, bool ODDS, int TILE, bool AUTO>
-__global__ __launch_bounds__(tile_threads(TILE)) void k_fwd_fields_split(
+__global__ __launch_bounds__(tile_threads(TILE)) __attribute__((amdgpu_waves_per_eu(ODDS ? 7 : 8))) void k_fwd_fields_split(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L,
     SplitTable P, int nitems, float* __restrict__ slog, float* __restrict__ sa, float* __restrict__ sac,
     float* __restrict__ part, int t0, int t1) {
   constexpr int NT = tile_threads(TILE);
-  __shared__ float2 s_uv[NT / 64][64];
+  __shared__ float4 s_batch[NT / 64][kFwdBatch / 4];
   const int item = xcd_swizzle(blockIdx.x, nitems);
   const int th = (int)threadIdx.x, lane = th & 63;
   int chunk, nsplit;
@@ -468,7 +518,7 @@ __global__ __launch_bounds__(tile_threads(TILE)) void k_fwd_fields_split(
   float sl = 0.f, s_a = 0.f, sc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) sc[c] = 0.f;
-  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, s_uv[wid], lane, sl, s_a, sc);
+  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane, sl, s_a, sc);
   if (nsplit > 1) {
     const int slot = AUTO ? item : P.pibase[ta.l] + item - P.ibase[ta.l];
     float* dst = part + (size_t)slot * split_part_floats<C, TILE>() + th;
