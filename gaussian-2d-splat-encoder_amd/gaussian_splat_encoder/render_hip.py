@@ -34,6 +34,10 @@ class PairBudgetExceeded(RuntimeError):
     (render_triton.py:51-55, raised at :378-385)."""
 
 
+class _PairRangeExceeded(PairBudgetExceeded):
+    """More pairs in one binning than its int32 pair index counts."""
+
+
 def _dev_check(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -394,7 +398,7 @@ def _settle(p, rc, pb):
     if rc == 1 and info_np[1] & 1:
         raise ValueError("binning: a splat has an empty tile rect (negative cutoff or scale)")
     if rc == 4:
-        raise PairBudgetExceeded(f"binning: {tot} pairs exceed the int32 pair index range")
+        raise _PairRangeExceeded(f"binning: {tot} pairs exceed the int32 pair index range")
     redone = rc == _lib.STATUS_CAPACITY
     if redone:
         pb = _pair_buffers(lib, p.N, p.nt, tot, p.with_maps, p.dev, p.geo)
@@ -639,8 +643,12 @@ def _forward_cull(mu, scale, color, opacity, bg, theta, H, W, TILE=8, cutoff=3.0
     if B > 1 and max_pairs is None:
         lv = _batch_levels(B, N, H, W, TILE)
         if lv is not None:
-            return _forward_cull_batch(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, odds, with_maps,
-                                       scale_is_log, plan, lv)
+            try:
+                return _forward_cull_batch(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, odds, with_maps,
+                                           scale_is_log, plan, lv)
+            except _PairRangeExceeded:   # the images together; each has an index range of its own below
+                if plan is not None:
+                    plan.sums = None     # allocated for one binning of them all
     bins = _bin(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, with_maps, scale_is_log=scale_is_log,
                 defer=True)
     out, T, asum, fg = _composite_buffers(B, P, C, dev)

@@ -41,3 +41,29 @@ def test_batch_equals_single_calls(dev, B, n, H, W, TILE, big):
     gb = torch.autograd.grad(img, L, gout)
     for x, y in zip(ga, gb):
         assert torch.equal(x, y)
+
+
+def test_batch_past_the_pair_range(dev, monkeypatch):
+    """Images whose pairs together pass the int32 pair index, while each image's own do not (here: the status of such a
+    count, given for a merged binning only), are rendered one after another: a speculated call, then a first one."""
+    B, n, H, W = 3, 300, 40, 56
+    scene = scene_of(B, n, H, W, dev, False)
+    gout = torch.randn(B, 3, H, W, generator=torch.Generator().manual_seed(B)).to(dev)
+    kw = dict(H=H, W=W, cull=True)
+    single = [device_run(RH.render_alpha_full_triton, [t[b:b + 1] for t in scene], gout[b:b + 1], **kw) for b in range(B)]
+    device_run(RH.render_alpha_full_triton, scene, gout, **kw)
+    settle, calls = RH._settle, []
+
+    def past_the_range(p, rc, pb):
+        calls.append(p.geo[3])
+        return settle(p, rc if p.geo[3] is None else 4, pb)
+    monkeypatch.setattr(RH, "_settle", past_the_range)
+    for first in (False, True):
+        if first:
+            RH._PAIRS_HW.clear()
+        out, g = device_run(RH.render_alpha_full_triton, scene, gout, **kw)
+        for b, (o1, g1) in enumerate(single):
+            assert torch.equal(out[b], o1[0]), b
+            for k in NAMES:
+                assert torch.equal(g[k][b], g1[k][0]), (b, k)
+    assert sum(c is not None for c in calls) == 2 and sum(c is None for c in calls) == 2 * B
