@@ -322,9 +322,14 @@ __device__ __forceinline__ TileAt split_item(const LevelTable& L, const SplitTab
 // 390,000 pairs, forward 38, 35, 41, 61; 43,000 pairs 12 / 10, 15 / 12, 19 / 17, 26 / 25. (Each level's lists in equal
 // numbers of chunks of 128 pairs on average: 62 / 65, 46, 17 / 17.) kAutoItems also bounds the launch while the count is
 // between the two: 8,192, with the items without work past the card's 8 waves per SIMD, cost 390,000 pairs 7 us.
+// Past kAutoMaxItems chunks (2^23 pairs) the length doubles instead of their number: at 64 pairs a chunk of 16 x 16 tiles
+// leaves 80 bytes of partial sums per pair, 85 GB for 2^30 pairs, whose launch would also pass 2^32 threads.
 constexpr int kAutoItems = 4096;
+constexpr int kAutoMaxItems = 1 << 17;
 __host__ __device__ __forceinline__ int auto_shift(long long pairs) {   // log2 of the chunk length
-  return pairs <= 32LL * kAutoItems ? 5 : 6;
+  int sh = pairs <= 32LL * kAutoItems ? 5 : 6;
+  while (pairs >> sh > kAutoMaxItems) ++sh;
+  return sh;
 }
 struct AutoItem {
   int t, g0, g1;       // tile and its chunk's pairs; t < 0: no work
@@ -2625,7 +2630,7 @@ int splat_render_fields_split_bwd(const float* rec, const int* gid_sorted, const
 
 // Items of an auto split launch over `ntiles` tiles that hold at most `cap` pairs (auto_base of the last tile's end).
 static long long auto_items(long long cap, int ntiles) {
-  return min(cap >> 5, max((long long)kAutoItems, cap >> 6)) + ntiles;
+  return min(cap >> 5, max((long long)kAutoItems, min(cap >> 6, (long long)kAutoMaxItems))) + ntiles;
 }
 
 // Host: level table and items of an auto split launch over the coarse levels of `lv`.

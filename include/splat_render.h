@@ -226,9 +226,10 @@ int splat_render_fields_split_bwd(const float *rec, const int *gid_sorted, const
                                   float *dsa, float *dsac, float *pair_sums, void *stream);
 
 /* The same over every coarse level of levmask, with chunks of one length for all tiles that the kernels choose from the
- * pairs found in tile_starts (32 or 64): no split has to be planned, and the sums' grouping depends on the pair list
- * alone. cap: a bound of the coarse levels' pairs (sizes the launch and the workspace; with more pairs than cap the
- * forward's fields are not complete and the backward's sums neither). */
+ * pairs found in tile_starts (32 or 64; past 2^23 pairs as long as makes 2^17 chunks at most): no split has to be
+ * planned, and the sums' grouping depends on the pair list alone. cap: a bound of the coarse levels' pairs (sizes the
+ * launch and the workspace; with more pairs than cap the forward's fields are not complete and the backward's sums
+ * neither). */
 size_t splat_fields_auto_workspace_bytes(int C, int H, int W, int TILE, const splat_levels *lv, unsigned levmask,
                                          long long cap);
 int splat_render_fields_auto(const float *rec, const int *gid_sorted, const int *tile_starts, int C, int H, int W,

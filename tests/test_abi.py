@@ -37,6 +37,18 @@ def test_workspace_queries_without_gpu():
     assert lib.splat_pair_sums_bytes(1_836_494) == 40 * 1_836_494
 
 
+def test_auto_split_workspace_stays_bounded():
+    """The partial sums of an auto split launch: at most 2^17 chunks and one per tile whatever the pair count, so that a
+    launch for 2^31 pairs neither needs more scratch than its pairs do nor passes 2^32 threads (256 per chunk here)."""
+    lib = _lib.load()
+    lv = ctypes.byref(_lib.SplatLevels(2, 0, 0.0, 100, 256, 256))
+    ask = lambda cap: lib.splat_fields_auto_workspace_bytes(3, 2048, 2048, 16, lv, 2, cap)   # noqa: E731
+    part, tiles = 4 * 5 * 256, 256
+    assert ask(64 << 17) == part * ((1 << 17) + tiles)
+    for cap in (1 << 24, 1 << 30, 0x7fffffff - 64):
+        assert ask(cap) == part * ((1 << 17) + tiles)
+
+
 def test_invalid_arguments_are_reported_not_launched():
     lib = _lib.load()
     rc = lib.splat_render_fwd(None, None, None, 3, 64, 64, 8, 0, None, 0, 1, 1, None, None, None, None, None, None,

@@ -195,3 +195,32 @@ def test_auto_split_equals_plain_launch(dev, TILE, n, px, H, W, odds):
     assert nb >= 4 * (2 + C) * max(64, TILE * TILE) * (coarse >> auto_shift(coarse))
     assert lib.splat_render_fields_auto(bins.p(0, "rec"), bins.p(0, "gid"), bins.p(0, "starts"), C, H, W, TILE, flags, lvr,
                                         mask, coarse, *[t.data_ptr() for t in ref], ws.data_ptr(), nb - 1, s) == 5
+
+
+@pytest.mark.parametrize("TILE,n", [(8, 520), (4, 140)])
+def test_auto_split_of_many_pairs(dev, TILE, n):
+    """Past 2^23 pairs the chunks grow to 128: fields and pair sums against the unsplit kernels, odds weights."""
+    H = W = 1024
+    lib, C = _lib.load(), 3
+    mu, ls, col, op, bg, th = random_scene(n + 50, H, W, seed=7, dev=dev, ls_mean_px=4.0, op_max=0.1)
+    ls[:, :n] = 1.0   # every tile of the coarse canvas
+    bins = RH._bin(mu, activate_scale(ls), col, op, th, H, W, TILE, 3.0, lv=_lib.SplatLevels(2, 0, 0.0, n, H, W))
+    tot, coarse = bins.tot_b[0], bins.level_tot_b[0][1]
+    assert 1 << 23 < coarse < 1 << 24
+    lvr, s, P0 = ctypes.byref(bins.lv), _lib.stream_ptr(dev), bins.geom[1][4]
+    ref = run_plain_fwd(lib, bins, C, RH.FLAG_ODDS, 2, dev)
+    fl = tuple(torch.full_like(t, float("nan")) for t in ref)
+    nb = lib.splat_fields_auto_workspace_bytes(C, H, W, TILE, lvr, 2, coarse)
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    ptrs = [bins.p(0, k) for k in ("rec", "gid", "starts")]
+    _lib.check(lib.splat_render_fields_auto(*ptrs, C, H, W, TILE, RH.FLAG_ODDS, lvr, 2, coarse, *[t.data_ptr() for t in fl],
+                                            ws.data_ptr(), nb, s), "fwd")
+    for a, b in zip(fl, ref):
+        assert close(a[P0:], b[P0:], 1e-5)
+    dS = upstream(bins, C, dev, 3)
+    ref_s, sums = torch.zeros(tot, 6 + C, device=dev), torch.zeros(tot, 6 + C, device=dev)
+    RH._render_bwd(lib, bins, 0, C, RH.FLAG_FIELDS | RH.FLAG_ODDS, (1, 2), 2, (None,) * 5 + dS, ref_s, None, s)
+    _lib.check(lib.splat_render_fields_auto_bwd(*ptrs, bins.p(0, "pq"), tot, C, H, W, TILE, RH.FLAG_ODDS, lvr, 2, coarse,
+                                                *[t.data_ptr() for t in dS], sums.data_ptr(), s), "bwd")
+    for k in range(6 + C):
+        assert close(sums[:, k], ref_s[:, k], 1e-5), k
