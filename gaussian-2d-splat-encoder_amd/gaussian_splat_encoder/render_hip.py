@@ -294,6 +294,15 @@ def _align(n):
     return (n + 255) & ~255
 
 
+_MAX_PAIRS = 0x7fffffff - 64   # most pairs of a binning (its pair index is 32-bit)
+
+
+def _with_slack(pairs):
+    """Pairs a call's buffers and launches are sized for when its count is expected to be about `pairs`: some more, but
+    no more than a binning can hold."""
+    return min(pairs + (pairs >> 4) + 1024, _MAX_PAIRS)
+
+
 _CARVE_OFF = {}   # tuple of sizes -> sub-buffer offsets (the renders of one configuration repeat their sizes)
 _PAIRS_WS = {}    # (binning configuration, capacity) -> pair-phase workspace bytes
 _SUMS_FLOATS = {}   # capacity -> floats of one image's per-pair sums (16-byte aligned)
@@ -432,7 +441,7 @@ def _bin_impl(mu, scale, color, opacity, theta, H, W, TILE, cutoff, max_pairs, w
     stream = _lib.stream_ptr(dev)
     key = (N, H, W, TILE, float(cutoff), _lv_key(lv))
     hw = _PAIRS_HW.get(key, 0)
-    cap = hw + (hw >> 4) + 1024 if hw else 0
+    cap = _with_slack(hw) if hw else 0
     info_t, info_np = _info_host()
     info_p = info_t.data_ptr()
     geo = (H, W, TILE, lvr)
@@ -524,11 +533,6 @@ def _level_splits(bins, lt, mask):
             if tiles:
                 sp[l] = max(1, min(_SPLIT_MAX, -(-int(lt[l]) // (_SPLIT_PAIRS * tiles))))
     return sp
-
-
-def _coarse_cap(pairs):
-    """Pairs a launch over the coarse levels is sized for when the count read is expected to be about `pairs`."""
-    return pairs + (pairs >> 4) + 1024
 
 
 def _fields_buffers(npix, C, dev):
@@ -841,7 +845,7 @@ def _forward_levels(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, ma
         # every level that held a pair in some call of this configuration: one that comes and goes costs its (zero)
         # fields, not a second launch
         mask_spec = _MASK_SEEN[bins.pending.key] = _MASK_SEEN.get(bins.pending.key, 0) | _mask_of(lt_spec)
-        cap = _coarse_cap(sum(lt_spec[1:]))
+        cap = _with_slack(sum(lt_spec[1:]))
         launch(0, lt_spec, mask_spec, cap)
         if plan is not None:         # the backward's buffers, allocated while the GPU works towards the count
             plan.allocate(bins, B, N, C, dev, lib, bins.pending.cap)

@@ -323,3 +323,17 @@ def test_octave_dense_coarse_level(dev, odds):
     bins = run_levels(*scene, H, W, 8, octave_lv(), odds=odds, seed=11)
     lt = bins.level_tot_b[0]
     assert max(RH._level_splits(bins, lt, bins.level_mask(0) & ~1)) >= 4, "the scene must split a coarse level"
+
+
+def test_octave_expecting_pairs_near_the_index_range(dev, monkeypatch):
+    """After a call of nearly 2^31 pairs, most of them on coarse levels, the next one's buffers and launches are sized for
+    no more pairs than a binning holds (here: the remembered counts of such a call)."""
+    H = W = 64
+    mu, ls, col, op, bg, th = random_scene(500, H, W, seed=5, dev=dev, ls_mean_px=6.0)
+    with torch.no_grad():
+        first = RH.render_alpha_octave(mu, ls, col, op, bg, H, W, theta=th)
+        key, = [k for k in RH._PAIRS_HW if k[:3] == (500, H, W) and k[-1] is not None]
+        n = 0x7fffffff - 64
+        monkeypatch.setitem(RH._PAIRS_HW, key, n)
+        monkeypatch.setitem(RH._LEVELS_SEEN, key, [24] + [0] * (len(RH._LEVELS_SEEN[key]) - 2) + [n - 24])
+        assert torch.equal(RH.render_alpha_octave(mu, ls, col, op, bg, H, W, theta=th), first)
