@@ -1491,15 +1491,19 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
 // ---------------------------------------------------------------------------------------------- small plan
 // The whole binning of a small problem in one workgroup and one launch (small_plan): with four launches, each a chain of
 // memory round trips over a handful of workgroups, a 64 x 64 render of 1,024 splats spent 25 us in them and more in the gaps
-// between them, against 17 us here (a forward 49 -> 38 us). Per tile one bit per splat (LDS): a splat's place in the tile's list is the number
-// of bits below its own, which is splat order without a sort. DECODE: all of splat_bin, the pair list for up to `cap`
-// pairs; where there are more, the row plan's histogram instead (the host asks for the pair phase again); else the pair
-// phase alone, from rect and offsets. A splat's tiles are walked by its own thread, so lists past kSmallPairs pairs go to
-// the row plan: 300,000 pairs (2,048 splats over 150 tiles each) would take about 100 us here.
+// between them, against 17 us here (a forward 49 -> 38 us). Per tile one bit per splat (LDS): a splat's place in the tile's
+// list is the number of bits below its own, which is splat order without a sort. DECODE: all of splat_bin, the pair list
+// for up to `cap` pairs; where there are more, the row plan's histogram instead (the host asks for the pair phase again);
+// else the pair phase alone, from rect and offsets. Lists past kSmallPairs pairs go to the row plan: 300,000 pairs (2,048
+// splats over 150 tiles each) would take about 100 us here. A splat's thread walks its own tiles up to kSmallWalk of them
+// (35 ns a step, twice), larger rects are walked by the waves: a binning of 4 splats over all 4,900 tiles of 560 x 560 takes
+// 23 us, by the row plan 27 us, with every rect walked by its own thread 408 us.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallMaxN = 2 * kSmallThreads;   // one splat per thread, or two consecutive ones
 constexpr int kSmallLds = 60 * 1024;
 constexpr int kSmallPairs = 24576;
+constexpr int kSmallWalk = 32;
+constexpr int kSmallLarge = kSmallPairs / (kSmallWalk + 1);
 
 __host__ __device__ __forceinline__ int small_words(int N) { return (N + 31) >> 5; }
 // LDS bytes: masks [words][tiles], their prefix counts (16 bits), tile starts
@@ -1508,6 +1512,8 @@ __host__ __device__ __forceinline__ size_t small_lds(int N, int nt) {
 }
 // The row plan's histogram fits them: a row needs a word per 256 splats and one more, and has at least one tile.
 static_assert(kSmallMaxN / kBlock + 1 <= kSmallMaxN / 32 + 1, "words per row");
+static_assert(kSmallLds / 10 < 1 << 15 && kSmallMaxN <= 1 << 15,
+              "a large rect's sizes (10 bytes per tile at least) and its splat take 16 bits each");
 
 template <int C, bool DECODE, int IT>
 __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
@@ -1519,7 +1525,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
     int2* __restrict__ rtot, int nb) {
   extern __shared__ int s_dyn[];
   constexpr int NW = kSmallThreads / 64;
-  __shared__ int s_w[NW], s_lev[kMaxLevels], s_bad;
+  __shared__ int s_w[NW], s_lev[kMaxLevels], s_bad, s_nlarge;
+  __shared__ int4 s_large[kSmallLarge];   // first tile, width | height << 16, tiles per row | splat << 16, first pair
   const int nt = L.tbase[L.n], W = small_words(N);
   unsigned* mask = reinterpret_cast<unsigned*>(s_dyn);
   int* start = s_dyn + (size_t)W * nt;
@@ -1527,7 +1534,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   for (int i = t; i < W * nt; i += kSmallThreads) mask[i] = 0u;
   if (t < kMaxLevels) s_lev[t] = 0;
-  if (t == 0) s_bad = 0;
+  if (t == 0) s_bad = s_nlarge = 0;
   int4 rc[IT];
   int hh[IT], cnt[IT], sum = 0;
   bool bad = false;
@@ -1564,6 +1571,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
     if (w < wv) off += x;
     tot += x;
   }
+  const bool over = tot > cap;   // `over` pairs are asked for again by the host
   int o0[IT];
 #pragma unroll
   for (int k = 0; k < IT; ++k) {
@@ -1572,12 +1580,10 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
     if (DECODE && g < N) offsets[g] = off;
     if (DECODE && g == N - 1) offsets[N] = tot;
     if (DECODE && cnt[k]) atomicAdd(&s_lev[rc[k].w], cnt[k]);
+    if (cnt[k] > kSmallWalk && !over)   // at most kSmallLarge of them, since tot <= cap <= kSmallPairs
+      s_large[atomicAdd(&s_nlarge, 1)] = make_int4(L.tbase[rc[k].w] + rc[k].y * L.ntx[rc[k].w] + rc[k].x,
+                                                   rc[k].z | hh[k] << 16, L.ntx[rc[k].w] | g << 16, off);
     off += cnt[k];
-    const int h = cnt[k] ? hh[k] : 0;
-    const int tb = L.tbase[rc[k].w] + rc[k].x, ntx = L.ntx[rc[k].w];
-    for (int y = 0; y < h; ++y)
-      for (int x = 0; x < rc[k].z; ++x)
-        atomicOr(&mask[(g >> 5) * nt + tb + (rc[k].y + y) * ntx + x], 1u << (g & 31));
   }
   if (DECODE && bad) s_bad = 1;
   __syncthreads();
@@ -1589,6 +1595,31 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
     }
     if (t < L.n) put_info(info, mirror, 2 + t, s_lev[t]);
     if (mirror && t < 64) __threadfence_system();
+  }
+  // f(splat, tile, splat-major index) for every pair: a small rect's by its own thread, the large ones' by the waves, in
+  // even shares while there are fewer of them than waves
+  auto pairs = [&](auto&& f) {
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int h = cnt[k] && cnt[k] <= kSmallWalk ? hh[k] : 0;
+      const int ntx = L.ntx[rc[k].w], tb = L.tbase[rc[k].w] + rc[k].y * ntx + rc[k].x;
+      int q = o0[k];
+      for (int y = 0; y < h; ++y)
+        for (int x = 0; x < rc[k].z; ++x, ++q) f(t * IT + k, tb + y * ntx + x, q);
+    }
+    const int nlarge = s_nlarge, share = nlarge > 0 && nlarge < NW ? NW / nlarge : 1;   // waves per large rect
+    for (int i = wv / share; i < nlarge; i += NW / share) {
+      const int4 e = s_large[i];
+      const int w = e.y & 0xffff, n = w * (e.y >> 16), ntx = e.z & 0xffff;
+      for (int j = wv % share * 64 + lane; j < n; j += 64 * share) {
+        const int y = j / w;
+        f(e.z >> 16, e.x + y * ntx + (j - y * w), e.w + j);
+      }
+    }
+  };
+  const bool none = tot == 0 || over || flagged;
+  if (!none) pairs([&](int g, int i, int) { atomicOr(&mask[(g >> 5) * nt + i], 1u << (g & 31)); });
+  if (DECODE) {
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
       const int g = t * IT + k;
@@ -1599,13 +1630,12 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
       }
     }
   }
-  if (tot == 0 || tot > cap || flagged) {   // the empty list (render_triton.py:392-394), or one the host asks for again
+  if (none) {   // the empty list (render_triton.py:392-394), or one the host asks for again
     for (int i = t; i <= nt; i += kSmallThreads) tile_starts[i] = 0;
     if (t == 0) gid_sorted[0] = 0;
     if (!DECODE || !rowhist || flagged || tot == 0) return;
     // what the count pass and its row scan leave for the row plan: rows x (nb blocks' units, then pairs) in the masks'
     // and starts' place (nb + 1 <= W + 1 words per row, and at least as many tiles as rows)
-    __syncthreads();
     const int nrows = L.rbase[L.n], K = nb + 1;
     for (int i = t; i < nrows * K; i += kSmallThreads) s_dyn[i] = 0;
     __syncthreads();
@@ -1628,6 +1658,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
     }
     return;
   }
+  __syncthreads();   // the masks are complete
   // per tile: the bits before each word (the words in `parts` shares, one thread each), then the tiles' starts
   __shared__ int s_part[kSmallThreads];
   const int parts = max(1, min(W, kSmallThreads / nt)), share = (W + parts - 1) / parts;
@@ -1675,21 +1706,13 @@ __global__ __launch_bounds__(kSmallThreads) void k_bin_small(
   }
   if (t == 0) tile_starts[nt] = tot;
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < IT; ++k) {
-    const int g = t * IT + k;
-    const int h = cnt[k] ? hh[k] : 0;
-    const int tb = L.tbase[rc[k].w] + rc[k].x, ntx = L.ntx[rc[k].w], wd = (g >> 5) * nt;
-    int q = o0[k];
-    for (int y = 0; y < h; ++y)
-      for (int x = 0; x < rc[k].z; ++x, ++q) {
-        const int i = tb + (rc[k].y + y) * ntx + x;
-        const int p = start[i] + pre[wd + i] + __popc(mask[wd + i] & ((1u << (g & 31)) - 1u));
-        gid_sorted[p] = g;
-        if (pair_q) pair_q[p] = q;
-        if (pair_splat) pair_splat[q] = g;
-      }
-  }
+  pairs([&](int g, int i, int q) {
+    const int wd = (g >> 5) * nt + i;
+    const int p = start[i] + pre[wd] + __popc(mask[wd] & ((1u << (g & 31)) - 1u));
+    gid_sorted[p] = g;
+    if (pair_q) pair_q[p] = q;
+    if (pair_splat) pair_splat[q] = g;
+  });
 }
 
 // ----------------------------------------------------------------------------------------------------

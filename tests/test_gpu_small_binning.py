@@ -1,6 +1,8 @@
 """The one-launch binning of small problems at the edges of its range: pair lists and maps bit-exact against the oracle's
 binning, for the first call of a configuration (count read first) and later ones (one launch), with capacities exceeded."""
 
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -76,3 +78,72 @@ def test_small_binning_errors(dev):
         RH._bin(mu, -sc, col, op, th, 64, 64, 8, 3.0)
     with pytest.raises(RH.PairBudgetExceeded):
         RH._bin(mu, sc, col, op, th, 64, 64, 8, 3.0, max_pairs=10)
+
+
+def takes_one_launch(H, W, TILE, n):
+    """small_plan: the masks, their counts and the tile starts in 60 KB."""
+    nt = binning.tile_grid(H, W, TILE)[2]
+    words = (n + 31) // 32
+    return n <= 2048 and 4 * nt * (words + 1) + 2 * words * nt <= 60 * 1024
+
+
+def rect_scene(n, big, H, W, dev, seed=1):
+    """n splats of about a pixel, every (n // big)-th of them as wide as the canvas."""
+    mu, ls, col, op, _, th = random_scene(n, H, W, seed=seed, dev=dev, ls_mean_px=1.0, ls_std=0.1)
+    if big:
+        ls[:, ::n // big] = 1.0
+    return mu, activate_scale(ls), col, op, th
+
+
+@pytest.mark.parametrize("H,W,TILE,n,big", [
+    (560, 560, 8, 4, 4), (560, 560, 8, 5, 1), (512, 512, 8, 32, 4), (400, 300, 8, 9, 9), (180, 200, 8, 45, 15),
+    (180, 200, 8, 32, 16), (180, 200, 8, 34, 17), (48, 48, 8, 600, 300), (32, 64, 8, 700, 350), (8, 264, 8, 1500, 500),
+    (8, 256, 8, 1500, 500), (1300, 700, 16, 3, 2)])
+def test_small_binning_of_large_rects(dev, H, W, TILE, n, big):
+    """Few splats over many tiles, and many just above and at the number of tiles that one thread walks."""
+    assert takes_one_launch(H, W, TILE, n)
+    scene = rect_scene(n, big, H, W, dev)
+    other = rect_scene(n, 0, H, W, dev, seed=2)
+    for mu, sc, col, op, th in (scene, scene, other, scene):
+        bins = RH._bin(mu, sc, col, op, th, H, W, TILE, 3.0)
+        assert bins.tot_b[0] <= 24576 - 1024 - 24576 // 16
+        check(bins, 0, mu[0].cpu().numpy(), sc[0].cpu().numpy(), H, W, TILE, 3.0)
+
+
+@pytest.mark.parametrize("n,big", [(1, 1), (4, 4), (32, 4)])
+def test_small_binning_of_large_rects_takes_no_longer(dev, monkeypatch, n, big):
+    """A few canvas-wide splats (4,900 tiles each) in one launch take no longer than by the row plan, which a remembered
+    count past the one launch's capacity selects: within a factor of two, the least of ten measurements each."""
+    H = W = 560
+    args = rect_scene(n, big, H, W, dev)
+
+    def us():
+        best = float("inf")
+        for _ in range(10):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                RH._bin(*args, H, W, 8, 3.0)
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t0) / 20 * 1e6)
+        return best
+    RH._bin(*args, H, W, 8, 3.0)
+    key, = [k for k in RH._PAIRS_HW if k[:4] == (n, H, W, 8)]
+    small = us()
+    monkeypatch.setitem(RH._PAIRS_HW, key, 100000)
+    rows = us()
+    print(f"{n} splats, {big} over the canvas: one launch {small:.1f} us, row plan {rows:.1f} us", flush=True)
+    assert small <= 2 * rows
+
+
+@pytest.mark.parametrize("H,W,TILE,n,px", [(136, 152, 8, 992, 2.0), (1, 287, 1, 1120, 1.0), (1100, 1, 1, 100, 20.0)])
+def test_small_binning_at_the_edges_of_its_rule(dev, H, W, TILE, n, px):
+    """Masks at the most LDS that the rule allows (with the static arrays past 64 KB), and more tile rows than the row plan
+    takes, where a count past the capacity is redone by the pair sort."""
+    assert takes_one_launch(H, W, TILE, n)
+    scenes = [random_scene(n, H, W, seed=n + k, dev=dev, ls_mean_px=px * f, margin=0.2) for k, f in ((0, 1.0), (1, 16.0))]
+    for k in (0, 0, 1, 1, 0):
+        mu, ls, col, op, _, th = scenes[k]
+        sc = activate_scale(ls)
+        bins = RH._bin(mu, sc, col, op, th, H, W, TILE, 3.0)
+        check(bins, 0, mu[0].cpu().numpy(), sc[0].cpu().numpy(), H, W, TILE, 3.0)
