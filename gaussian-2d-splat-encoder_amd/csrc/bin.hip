@@ -1815,6 +1815,12 @@ size_t splat_bin_count_workspace_bytes(int N, int H, int W, int TILE, const spla
   return plan_count(L, N).total;
 }
 
+int splat_bin_takes_rows(int N, int H, int W, int TILE, const splat_levels* lv) {
+  LevelTable L;
+  if (N < 0 || H < 1 || W < 1 || TILE < 1 || make_levels(H, W, TILE, lv, &L, nullptr)) return -1;
+  return plan_count(L, N).rows ? 1 : 0;
+}
+
 int splat_levels_geometry(int H, int W, int TILE, const splat_levels* lv, int* out, int cap) {
   LevelTable L;
   if (H < 1 || W < 1 || TILE < 1 || make_levels(H, W, TILE, lv, &L, nullptr))

@@ -41,6 +41,7 @@ _SIGS = {
     "splat_levels_geometry": (_I, [_I, _I, _I, _LV, _VP, _I]),
     "splat_bin_count": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _LV, _I, _VP, _VP, _VP, _VP, _VP, _SZ,
                              _VP]),
+    "splat_bin_takes_rows": (_I, [_I, _I, _I, _I, _LV]),
     "splat_bin_pairs_workspace_bytes": (_SZ, [_I, _I, _I, _I, _LV, _LL]),
     "splat_bin": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _LV, _I, _LL, _VP, _VP, _VP, _VP, _VP, _VP, _SZ,
                        _LL, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),

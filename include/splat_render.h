@@ -107,7 +107,10 @@ int splat_bin_count(const float *mu, const float *scale, const float *theta, con
  * Optional (NULL skips) maps between the sorted order i and the splat-major pair order q (splat g owns
  * q in [offsets[g], offsets[g+1]), walking its rect row by row), used by the backward:
  * pair_splat[q] = splat of q, pair_q[i] = q of sorted pair i.
- * Replaces render_triton.py:392-409. */
+ * Replaces render_triton.py:392-409. splat_bin_takes_rows: 1 when N splats on the level table take the first of
+ * the two (at most 1,024 tile rows, and rows times blocks of 256 splats at most 2^22), 0 when they take the second,
+ * -1 for bad arguments. */
+int splat_bin_takes_rows(int N, int H, int W, int TILE, const splat_levels *lv);
 size_t splat_bin_pairs_workspace_bytes(int N, int H, int W, int TILE, const splat_levels *lv, long long tot);
 int splat_bin_pairs(const int *rect, const int *offsets, const void *ws_count, int N, int H, int W, int TILE,
                     const splat_levels *lv, long long tot, int *gid_sorted, int *tile_starts,

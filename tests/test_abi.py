@@ -37,6 +37,25 @@ def test_workspace_queries_without_gpu():
     assert lib.splat_pair_sums_bytes(1_836_494) == 40 * 1_836_494
 
 
+def test_batches_are_merged_only_where_the_row_plan_takes_them():
+    """A batch is rendered as one binning only while the merged level table, whose rows and decode blocks both grow with
+    the images, takes the row plan as each image alone does: workspace of three unit arrays, not of the pair sort."""
+    from gaussian_splat_encoder import render_hip as RH
+    lib = _lib.load()
+    merged = 0
+    for n, S in ((1024, 64), (10240, 256), (92160, 768), (163840, 1024), (655360, 2048)):
+        assert lib.splat_bin_takes_rows(n, S, S, 8, None) == 1
+        for B in (2, 3, 4, 8, 12, 13):
+            lv = RH._batch_levels(B, n, S, S, 8)
+            if lv is not None:
+                merged += 1
+                assert lib.splat_bin_pairs_workspace_bytes(B * n, S, S, 8, ctypes.byref(lv), 64) == 3 * 256, (B, n, S)
+    assert merged >= 12
+    for B, n, S in ((8, 163840, 1024), (3, 655360, 2048), (13, 1024, 64)):
+        assert RH._batch_levels(B, n, S, S, 8) is None
+    assert lib.splat_bin_takes_rows(10, 0, 8, 8, None) == -1
+
+
 def test_auto_split_workspace_stays_bounded():
     """The partial sums of an auto split launch: at most 2^17 chunks and one per tile whatever the pair count, so that a
     launch for 2^31 pairs neither needs more scratch than its pairs do nor passes 2^32 threads (256 per chunk here)."""
