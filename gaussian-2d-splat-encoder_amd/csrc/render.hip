@@ -1675,20 +1675,20 @@ __device__ __forceinline__ int exact_fwd_pixel(const ExactPixels& G, int group, 
                  : exact_tile_pixel<16>(G, group, lane >> 2, (lane & 3) * 4 + k);
 }
 
-// Forward. Workgroup = S shares (one per wave) of the splat batches for pixel group blockIdx.x / nsplit; lane = PX
-// pixels. Each wave lists the splats that meet its group and takes them 64 at a time: lane = splat loads their records
-// into LDS (one round trip for 64), lane = pixel reads them by broadcast. Bound by the VALU with PX = 4: a record's LDS
-// reads serve 256 pixels. (Records by scalar loads, one pixel per lane, each four records waiting for their own round trip: 245 us at 512 x 512
-// with 16,384 splats, 770 us for 10,000 unordered pixels and 92,160 splats.)
+// Forward. Workgroup = S shares (one per wave; eight, or one, see exact_fwd_plan) of the splat batches for pixel group
+// blockIdx.x / nsplit; lane = PX pixels. Each wave lists the splats that meet its group and takes them 64 at a time: lane =
+// splat loads their records into LDS (one round trip for 64), lane = pixel reads them by broadcast. Bound by the VALU with
+// PX = 4: a record's LDS reads serve 256 pixels. (Records by scalar loads, one pixel per lane, each four records waiting for
+// their own round trip: 245 us at 512 x 512 with 16,384 splats, 770 us for 10,000 unordered pixels and 92,160 splats.)
 // nsplit > 1: partial sums at part[split][k][slot], k < exact_part, slot = (group PX + pixel) 64 + lane.
 constexpr int kExactFwdWaves = 8;
-template <int C, int PX, bool GRID>
-__global__ __launch_bounds__(64 * kExactFwdWaves) void k_fwd_exact(
+template <int C, int PX, bool GRID, int S>
+__global__ __launch_bounds__(64 * S) void k_fwd_exact(
     const float* __restrict__ rec, const float4* __restrict__ reach, int N, ExactPixels G,
     const float* __restrict__ pyv, const float* __restrict__ pxv, int qi, int qo, const float* __restrict__ bg,
     float* __restrict__ out, float* __restrict__ Tout, float* __restrict__ asum_out, float* __restrict__ fg_out,
     float* __restrict__ part) {
-  constexpr int S = kExactFwdWaves, K = exact_part<C>();
+  constexpr int K = exact_part<C>();
   constexpr int RS = C > 1 ? 12 : 8;   // floats of a staged record: gy, gx, A, B, Cc, D, lop, colour
   __shared__ float4 s_rec4[S][64 * RS / 4];
   __shared__ int s_cand[S][192], s_list[S][128];
@@ -1831,7 +1831,7 @@ __global__ __launch_bounds__(64 * kExactFwdWaves) void k_fwd_exact(
     __syncthreads();   // the records, and pixel k - 1's sums, have been read
     s[k].put(&s_part[wv][0][lane], 64);
     __syncthreads();
-    if (wv == k) {
+    if (wv == k % S) {
       ExactSums<C> o;
       for (int w = 0; w < S; ++w) o.take(&s_part[w][0][lane], 64);
       if (nsplit > 1) {
@@ -2812,8 +2812,12 @@ constexpr int kExactWaves = 8192;   // 8 per SIMD
 // are batches) that take the batches meeting a group in turn, so that a group's waves have the same number of them
 // wherever it lies (shares by the batch's number instead, splats in cell order: 229 against 141 us at 512 x 512), and
 // qo shares of the blocks of 64 batches.
+// Few batches: one wave per group and no shares where the groups alone are nb waves per SIMD and more. Of eight waves all
+// but as many as there are batches only hold LDS and wave slots: 64 splats on 2048 x 2048 307 us with eight, 101 us with
+// one; 256 splats on 1024 x 1024 (4,096 groups) 109 and 100 us, but 1,000,000 listed pixels (3,907 groups) 166 and 182 us,
+// 512 splats on 1024 x 1024 161 and 182 us.
 struct ExactFwdPlan {
-  int px, qi, qo, nsplit;
+  int px, qi, qo, nsplit, waves;
   ExactPixels G;
 };
 ExactFwdPlan exact_fwd_plan(int N, int P, int grid_w, const int* perm) {
@@ -2822,8 +2826,10 @@ ExactFwdPlan exact_fwd_plan(int N, int P, int grid_w, const int* perm) {
   p.px = (P + 255LL) / 256 * nb >= kExactWaves / 2 ? 4 : 1;
   p.G = exact_pixels(P, grid_w, p.px, perm);
   const long long groups = p.G.groups;
-  p.qi = kExactFwdWaves;
-  p.qo = 1;
+  p.waves = nb <= kExactFwdWaves && groups >= 1024 * max(nb, 2LL) ? 1 : kExactFwdWaves;
+  p.qi = p.waves;
+  p.qo = p.nsplit = 1;
+  if (p.waves == 1) return p;
   while (p.qi < 64 && p.qi < nb && groups * p.qi < kExactWaves) p.qi *= 2;
   while (p.qi == 64 && p.qo < 16 && p.qo < blocks && groups * p.qi * p.qo < kExactWaves) ++p.qo;
   p.nsplit = p.qi / kExactFwdWaves * p.qo;
@@ -2881,7 +2887,7 @@ int splat_exact_render(const float* rec, const float* reach, int N, int C, const
     return set_error(kInvalid, "splat_exact_render: bad arguments N=%d C=%d P=%d grid_w=%d", N, C, P, grid_w);
   ExactFwdPlan p = exact_fwd_plan(N, P, grid_w, order);
   if (!ws) {   // without a workspace the shares stay within one workgroup
-    p.qi = kExactFwdWaves;
+    p.qi = p.waves;
     p.qo = p.nsplit = 1;
   } else if (ws_bytes < splat_exact_fwd_workspace_bytes(N, C, P, grid_w)) {
     return set_error(kWorkspace, "splat_exact_render: workspace of %zu bytes, %zu needed", ws_bytes,
@@ -2892,8 +2898,10 @@ int splat_exact_render(const float* rec, const float* reach, int N, int C, const
     constexpr int CC = decltype(cc)::value;
     auto launch = [&](auto npx, auto grid) {
       constexpr int PX = decltype(npx)::value;
-      k_fwd_exact<CC, PX, decltype(grid)::value != 0><<<p.G.groups * p.nsplit, 64 * kExactFwdWaves, 0, st>>>(
-          rec, reinterpret_cast<const float4*>(reach), N, p.G, py, px, p.qi, p.qo, bg, out, T, asum, fg, (float*)ws);
+      constexpr bool GR = decltype(grid)::value != 0;
+      auto kernel = p.waves == 1 ? k_fwd_exact<CC, PX, GR, 1> : k_fwd_exact<CC, PX, GR, kExactFwdWaves>;
+      kernel<<<p.G.groups * p.nsplit, 64 * p.waves, 0, st>>>(rec, reinterpret_cast<const float4*>(reach), N, p.G, py, px,
+                                                             p.qi, p.qo, bg, out, T, asum, fg, (float*)ws);
       if (p.nsplit > 1)
         k_exact_combine<CC, PX><<<(p.G.groups * PX + 3) / 4, 256, 0, st>>>(p.G, p.nsplit, (const float*)ws, bg, out, T,
                                                                           asum, fg);

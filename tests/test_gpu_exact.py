@@ -2,6 +2,7 @@
 splat batches of 64, the shares of both, and the reach boxes that leave out pairs whose every term is an exact zero."""
 
 import math
+import time
 
 import pytest
 import torch
@@ -112,3 +113,60 @@ def test_reach_keeps_values_that_are_not_finite(dev):
         else:
             scene[which][0, 17] = value
         same(run_c(scene, H, W, go, True), run_c(scene, H, W, go, False))
+
+
+def axes(H, W, dev):
+    return R_api._pixel_axes(H, W, dev, torch.float32)
+
+
+@pytest.mark.parametrize("H,W,N", [(256, 512, 64), (256, 504, 64), (250, 517, 65), (2048, 64, 0), (1024, 1024, 1),
+                                   (1000, 1030, 128), (1024, 1024, 256), (1024, 1008, 256), (1448, 1450, 512)])
+def test_few_splats_on_many_pixels(dev, H, W, N):
+    """One wave per pixel group, at the sizes where the rule for it begins and just before: every 61st pixel against a list of
+    those pixels, whose groups take eight waves. The sums of up to 512 terms are grouped another way: 1e-6 of T, of the
+    colours and of S_a relative to its size."""
+    mu, ls, col, op, bg, th = random_scene(N, H, W, seed=N + 1, dev=dev, ls_mean_px=0.05 * W, op_max=0.95, margin=0.1)
+    ys, xs = axes(H, W, dev)
+    full = RH._forward(mu, ls, col, op, bg, ys, xs, th, W, True)[:4]
+    idx = torch.arange(0, H * W, 61, device=dev)
+    some = RH._forward(mu, ls, col, op, bg, ys[idx // W].contiguous(), xs[idx % W].contiguous(), th, 0, True)[:4]
+    for a, b in zip(full, some):
+        a = a[:, idx]
+        assert ((a - b).abs() <= 1e-6 * b.abs().clamp_min(1.0)).all()
+
+
+def test_few_splats_on_many_listed_pixels(dev):
+    """The same for a list: one of every pixel of a canvas against the canvas."""
+    H, W, N = 1024, 1100, 64
+    mu, ls, col, op, bg, th = random_scene(N, H, W, seed=3, dev=dev, ls_mean_px=40.0, op_max=0.95)
+    ys, xs = axes(H, W, dev)
+    full = RH._forward(mu, ls, col, op, bg, ys, xs, th, W, True)[:4]
+    some = RH._forward(mu, ls, col, op, bg, ys.repeat_interleave(W).contiguous(), xs.repeat(H).contiguous(), th, 0, True)[:4]
+    for a, b in zip(full, some):
+        assert ((a - b).abs() <= 1e-6 * b.abs().clamp_min(1.0)).all()
+
+
+def best_us(f, n=10):
+    best = float("inf")
+    for _ in range(8):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(n):
+            f()
+        torch.cuda.synchronize()
+        best = min(best, (time.perf_counter() - t0) / n * 1e6)
+    return best
+
+
+def test_few_splats_on_many_pixels_take_no_longer(dev):
+    """64 splats on 2048 x 2048, bound by the 134 MB that the forward writes: at most five times a copy of as much, most of
+    which the last-level cache holds."""
+    H = W = 2048
+    mu, ls, col, op, bg, th = random_scene(64, H, W, seed=3, dev=dev, ls_mean_px=100.0, op_max=0.95)
+    ys, xs = axes(H, W, dev)
+    src = torch.empty(8 * H * W, device=dev)
+    dst = torch.empty_like(src)
+    copy = best_us(lambda: dst.copy_(src))
+    render = best_us(lambda: RH._forward(mu, ls, col, op, bg, ys, xs, th, W, True))
+    print(f"render {render:.1f} us, copy {copy:.1f} us", flush=True)
+    assert render <= 5 * copy
