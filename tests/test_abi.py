@@ -56,6 +56,15 @@ def test_batches_are_merged_only_where_the_row_plan_takes_them():
     assert lib.splat_bin_takes_rows(10, 0, 8, 8, None) == -1
 
 
+def test_pixel_lists_of_few_splats_are_taken_as_they_are():
+    """Ordering a list costs four launches over its pixels; with few splats there is less to leave out than that."""
+    lib = _lib.load()
+    for n, P in ((1, 1 << 30), (64, 1 << 24), (128, 1000000), (255, 1 << 21), (256, 262143), (92160, 255)):
+        assert lib.splat_exact_order_bytes(n, P) == 0, (n, P)
+    for n, P in ((256, 262144), (4096, 65536), (92160, 10000)):
+        assert lib.splat_exact_order_bytes(n, P) >= 16 * P, (n, P)
+
+
 def test_auto_split_workspace_stays_bounded():
     """The partial sums of an auto split launch: at most 2^17 chunks and one per tile whatever the pair count, so that a
     launch for 2^31 pairs neither needs more scratch than its pairs do nor passes 2^32 threads (256 per chunk here)."""
