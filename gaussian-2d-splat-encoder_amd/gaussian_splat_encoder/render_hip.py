@@ -276,7 +276,8 @@ def _lv_key(lv):
 _GEOM = {}          # (H, W, TILE, levels) -> levels_geometry result
 _PAIRS_HW = {}      # binning configuration -> most pairs one image needed so far (sizes the next capacity)
 _LEVELS_SEEN = {}   # binning configuration -> per-level pair totals of its last binning (plans deferred launches)
-_MASK_SEEN = {}     # binning configuration -> levels that held pairs in any call
+_LEVEL_AGE = {}     # binning configuration -> per level, its calls since one that held pairs there
+_LEVEL_KEEP = 8     # calls without pairs after which a level is no longer planned for
 _WS1 = {}           # binning configuration -> count-phase workspace bytes
 _tls = threading.local()
 
@@ -506,6 +507,15 @@ def _build_tiles(mu, scale, H, W, TILE, cutoff, max_pairs=None):
     dummy_col = torch.zeros((B, N, 1), device=mu.device)
     dummy_op = torch.zeros((B, N), device=mu.device)
     return _bin(mu, scale, dummy_col, dummy_op, None, H, W, TILE, cutoff, max_pairs, with_maps=False).as_tuple()
+
+
+def _planned_mask(key, lt):
+    """The levels that a deferred levels forward renders before its count is read, lt being the totals of the
+    configuration's last binning: those that held pairs in one of its last _LEVEL_KEEP calls. A level that comes and goes
+    costs its (zero) fields, not a second launch, and one that stays empty is dropped."""
+    age = tuple(0 if n > 0 else a + 1 for n, a in zip(lt, _LEVEL_AGE.get(key, (_LEVEL_KEEP,) * len(lt))))
+    _LEVEL_AGE[key] = age
+    return _mask_of([a < _LEVEL_KEEP for a in age])
 
 
 # ----------------------------------------------------------------------------------------------- cull path
@@ -851,9 +861,7 @@ def _forward_levels(mu, scale, color, opacity, bg, theta, H, W, TILE, cutoff, ma
 
     if bins.pending is not None:   # queued on the speculative pair list and levels before the count is read
         lt_spec = _speculated_levels(bins)
-        # every level that held a pair in some call of this configuration: one that comes and goes costs its (zero)
-        # fields, not a second launch
-        mask_spec = _MASK_SEEN[bins.pending.key] = _MASK_SEEN.get(bins.pending.key, 0) | _mask_of(lt_spec)
+        mask_spec = _planned_mask(bins.pending.key, lt_spec)
         cap = _with_slack(sum(lt_spec[1:]))
         launch(0, lt_spec, mask_spec, cap)
         if plan is not None:         # the backward's buffers, allocated while the GPU works towards the count

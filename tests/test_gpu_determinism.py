@@ -41,6 +41,7 @@ def test_c2_runs_bit_identical(dev, entry):
             return RH.render_alpha_octave(mu, ls, col, op, bg, H, W, theta=th)
     RH._PAIRS_HW.clear()      # the first call reads the count before it sizes the pair buffers
     RH._LEVELS_SEEN.clear()
+    RH._LEVEL_AGE.clear()
     ref_out, ref_g = fwd_bwd(fn, leaves, gout)
     runs = [fwd_bwd(fn, leaves, gout) for _ in range(2)]   # speculated capacity and levels
     # other splats of the same configuration: larger scales, so more pairs than the speculated capacity

@@ -337,3 +337,34 @@ def test_octave_expecting_pairs_near_the_index_range(dev, monkeypatch):
         monkeypatch.setitem(RH._PAIRS_HW, key, n)
         monkeypatch.setitem(RH._LEVELS_SEEN, key, [24] + [0] * (len(RH._LEVELS_SEEN[key]) - 2) + [n - 24])
         assert torch.equal(RH.render_alpha_octave(mu, ls, col, op, bg, H, W, theta=th), first)
+
+
+def test_levels_that_stay_empty_are_dropped(dev, monkeypatch):
+    """After a call with splats on coarse octaves, calls whose splats all stay on octave 0 soon render octave 0 alone; a call
+    in between keeps the levels planned for; the images are those of first calls throughout."""
+    H = W = 96
+    mu, small, col, op, bg, th = random_scene(400, H, W, seed=5, dev=dev, ls_mean_px=1.0, ls_std=0.1)
+    ls = small.clone()
+    ls[:, :9] += 2.5 + 0.25 * torch.arange(9, device=dev)[:, None]   # fewer coarse pairs than a launch has to spare
+    masks, render = [], RH._render_fwd
+    monkeypatch.setattr(RH, "_render_fwd", lambda *a: (masks.append(a[6]), render(*a))[1])
+
+    def image(scales):
+        return RH.render_alpha_octave(mu, scales, col, op, bg, H, W, theta=th)
+    with torch.no_grad():
+        RH._PAIRS_HW.clear()
+        RH._LEVELS_SEEN.clear()
+        want = {id(t): image(t) for t in (small, ls)}
+        assert torch.equal(image(ls), want[id(ls)])
+        coarse = masks[-1]
+        assert coarse != 1
+        for _ in range(3):
+            assert torch.equal(image(small), want[id(small)])
+        assert masks[-1] == coarse
+        del masks[:]
+        assert torch.equal(image(ls), want[id(ls)])
+        assert masks == [coarse]   # not launched twice
+        for _ in range(20):
+            assert torch.equal(image(small), want[id(small)])
+        assert masks[-1] == 1
+        assert torch.equal(image(ls), want[id(ls)])
