@@ -1218,9 +1218,9 @@ __global__ __launch_bounds__(kBlock) void k_scatter_units(const int4* __restrict
   }
 }
 
-// One workgroup of kRowThreads per tile row and chunk of at most kRowCols tile columns (RowChunks). Counting: the spans of the row's units (kRowUnits per round) give
-// the row's pairs before c0 and a difference array over the chunk's columns (LDS atomics), so the chunk's tile
-// starts follow. Writing: the units meeting the chunk are listed in LDS in unit order (their index and span),
+// One workgroup of kRowThreads per tile row and chunk of at most kRowCols tile columns (RowChunks). Counting: the spans
+// of the row's units (kRowUnits per round) give the row's pairs before c0 and a difference array over the chunk's
+// columns (LDS atomics), so the chunk's tile starts follow. Writing: the units meeting the chunk are listed in LDS in unit order (their index and span),
 // their splat ids and splat-major indices gathered for the listed units only, then each wave owns the columns
 // j = wave, wave + 8, ...: it walks the list 64 units at a time and, per column, the units covering it (one
 // ballot) are that tile's next pairs in splat order, written by consecutive lanes at the column's running
@@ -1248,8 +1248,8 @@ struct RowChunks {
 // registers; CPW = 0: in LDS (s_diff), read and advanced by the owning wave.
 template <int CPW>
 __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const long long* __restrict__ info, int cap,
-                                                            const int2* __restrict__ rtot,
-                                                            RowChunks RC, const int* __restrict__ ug, const int* __restrict__ uq,
+                                                            const int2* __restrict__ rtot, RowChunks RC,
+                                                            const int* __restrict__ ug, const int* __restrict__ uq,
                                                             const int* __restrict__ uspan, int* __restrict__ gid_sorted,
                                                             int* __restrict__ tile_starts, int* __restrict__ pair_splat,
                                                             int* __restrict__ pair_q) {

@@ -78,8 +78,8 @@ __device__ __forceinline__ float uniform_f(float x) {
 
 // Whitened offsets (u, v) of the pixel centre (py0, px0) from a splat with centre (gy, gx) and rotation rows
 // (A, B), (Cc, D). A tile's pixels add their own offsets from the tile's reference pixel centre (its middle pixel)
-// to these, so their rounding error is shared by the whole tile. The float32 differences py0 - gy, px0 - gx are exact wherever the
-// two lie within a factor of two (Sterbenz), which holds for every tile a splat reaches away from the canvas'
+// to these, so their rounding error is shared by the whole tile. The float32 differences py0 - gy, px0 - gx are exact
+// wherever the two lie within a factor of two (Sterbenz), which holds for every tile a splat reaches away from the canvas'
 // first rows and columns (there the values are small and so is their rounding); each product's rounding error is
 // recovered exactly by an fma and added back, so the result is within about one ulp of the exact offsets (a
 // float64 evaluation rounded once: half an ulp), at a third of the instructions.
@@ -100,13 +100,15 @@ enum FwdBatch : int { F_UV = 0, F_BD = 128, F_AC = 256, F_COL = 384, F_LOP = 640
 // three matrix instructions (outer4; eight FMAs otherwise), and S_a with the colour sums, acc = (S_a, S_ac[0..2])
 // (C = 4: S_ac alone), from one per pair (four FMAs). sl adds log2 of the product of the (1 - a) factors: each is
 // >= 1e-4, so the product of eight stays >= 1e-32, a normal float.
-// What bounds it is the vector unit's issue: an FMA takes it about 4.4 cycles, one of these matrix instructions about 9,
-// so 2.5 of them do the work of 8 FMAs (35 cycles) in 22; each change between the two kinds costs about 8 more, hence the
-// three phases, kept apart by scheduling barriers, over as many pairs as the registers of eight waves per SIMD hold (seven
-// with the odds, which keep the opacities too). f32 matrix instructions don't run beside the vector unit's, whatever
-// their size. 768 x 768, 92,160 splats: 54.4-54.9 us with FMAs on records from scalar loads, 58.0 us with the kinds
-// interleaved as the compiler orders them, 51.5-52.6 us so (2048 x 2048: 761, 855, 720 us); the coarse levels' launch,
-// whose few waves also waited for the scalar loads, 55.1 -> 44.5 us, its composite with the odds 70.1 -> 60.4 us.
+// What bounds it is the vector unit's issue (a probe at 8 waves per SIMD, cycles at 2.4 GHz): an FMA takes 2.4 cycles with
+// vector operands and 4.2 with a scalar one in a stream of such, an exp2 about 14 among FMAs, one of these matrix
+// instructions 8.8 in a row of them and 11.5 between FMAs. So 2.5 of them do in 22 cycles what 8 FMAs on a record in scalar
+// registers did in 34; hence the three phases, kept apart by scheduling barriers, over as many pairs as the registers of
+// eight waves per SIMD hold (seven with the odds, which keep the opacities too). f32 matrix instructions don't run beside
+// the vector unit's, whatever their size. 768 x 768, 92,160 splats: 54.4-54.9 us with FMAs on records from scalar loads,
+// 58.0 us with the kinds interleaved as the compiler orders them, 51.5-52.6 us so (2048 x 2048: 761, 855, 720 us); the
+// coarse levels' launch, whose few waves also waited for the scalar loads, 55.1 -> 44.5 us, its composite with the odds
+// 70.1 -> 60.4 us.
 template <int C, bool ODDS, bool CLAMP, int N>
 __device__ __forceinline__ void fwd_group(const float* sb, int j, int quad, float ly, float lx, float& sl, float& s_a,
                                           floatx4& acc) {
@@ -384,8 +386,9 @@ __device__ __forceinline__ void tile_centres(const TileAt& ta, int l, int lane, 
 // upsampled and added first, and `asum` keeps the unclamped S_a (the clamp_min gradient needs it).
 // Waves sharing one 8x8 tile in the forward: each composites a contiguous share of the tile's pair list for
 // the tile's 64 pixels, and the partial sums are added in wave order through LDS. More waves per tile hide
-// the scalar-load latency of the record stream and even out tiles of different lengths.
-// 8x8 tiles: 4 waves per tile, or 16 with kFlagWide (few tiles with long pair lists: the coarse levels of an
+// the latency of the batches' gathers and even out tiles of different lengths; each has a last batch of its own.
+// 8x8 tiles: 4 waves per tile (768 x 768 / 2048 x 2048 with 92,160 / 655,360 splats: 52.0 / 722 us, with 2 waves 52.0 /
+// 729, with 8 59.4 / 748), or 16 with kFlagWide (few tiles with long pair lists: the coarse levels of an
 // octave render, where a launch may hold a few hundred tiles of thousands of pairs each).
 template <int TILE, bool WIDE>
 __host__ __device__ constexpr int fwd_split() { return TILE == 8 ? (WIDE ? 16 : 4) : 1; }
@@ -393,12 +396,13 @@ template <int TILE, int S>
 __host__ __device__ constexpr int fwd_threads() { return tile_threads(TILE) * S; }
 
 // What a composite launch renders: level 0 alone, level 0 with the coarse levels' upsampled fields added, or the images
-// of a batch (one level each). The batch is a variant of its own: the image's number and offset, kept over the pair loop
-// next to the records' scalar registers, cost a single image 56.5 against 53.8 us at 768 x 768.
+// of a batch (one level each). The batch is a variant of its own for the image's number and offset, which it keeps over the
+// pair loop: a single image takes 52.8 us with them and 52.0 without at 768 x 768.
 enum Composite : int { kPlain = 0, kUps = 1, kBatch = 2 };
 
 template <int C, bool FIELDS, bool ODDS, int MODE, int TILE, int S>
-__global__ __launch_bounds__((fwd_threads<TILE, S>())) __attribute__((amdgpu_waves_per_eu(S == 16 ? 4 : ODDS ? 7 : 8))) void k_fwd_cull(
+__global__ __launch_bounds__((fwd_threads<TILE, S>()))
+__attribute__((amdgpu_waves_per_eu(S == 16 ? 4 : ODDS ? 7 : 8))) void k_fwd_cull(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L, int tb0,
     int ntiles, const float* __restrict__ bg, float* __restrict__ out, float* __restrict__ Tout,
     float* __restrict__ asum_out, float* __restrict__ fg_out, float* __restrict__ slog, float* __restrict__ sa,
@@ -425,7 +429,8 @@ __global__ __launch_bounds__((fwd_threads<TILE, S>())) __attribute__((amdgpu_wav
   float sl = 0.f, s_a = 0.f, sc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) sc[c] = 0.f;
-  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane, sl, s_a, sc);
+  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane,
+                          sl, s_a, sc);
   if (S > 1) {
     static_assert((2 + C) * 64 <= kFwdBatch, "a wave's partial sums take the place of its batch");
     if (wv > 0) {
@@ -478,13 +483,15 @@ __global__ __launch_bounds__((fwd_threads<TILE, S>())) __attribute__((amdgpu_wav
 template <int C, int TILE>
 __host__ __device__ constexpr int split_part_floats() { return (2 + C) * tile_threads(TILE); }
 
-// FIELDS forward of the split work items of the coarse levels (SplitTable): one workgroup per item, the tile's
+// FIELDS forward of the split work items of the coarse levels (SplitTable, whose chunk numbers a C caller plans; the
+// renders take the auto split): one workgroup per item, the tile's
 // pixels one per thread, over the item's chunk of the tile's pair list (in pair order, as fwd_tile_pixel walks
 // it). A level with split 1 writes its fields; otherwise the item writes partial sums for k_fields_combine. AUTO: the
 // items of an auto split launch over the tiles [t0, t1) instead, `nitems` of them in the buffer `part` (more are not
 // written: the launch was planned for fewer pairs and is repeated).
 template <int C, bool ODDS, int TILE, bool AUTO>
-__global__ __launch_bounds__(tile_threads(TILE)) __attribute__((amdgpu_waves_per_eu(ODDS ? 7 : 8))) void k_fwd_fields_split(
+__global__ __launch_bounds__(tile_threads(TILE))
+__attribute__((amdgpu_waves_per_eu(ODDS ? 7 : 8))) void k_fwd_fields_split(
     const float* __restrict__ rec, const int* __restrict__ gid, const int* __restrict__ starts, LevelTable L,
     SplitTable P, int nitems, float* __restrict__ slog, float* __restrict__ sa, float* __restrict__ sac,
     float* __restrict__ part, int t0, int t1) {
@@ -523,7 +530,8 @@ __global__ __launch_bounds__(tile_threads(TILE)) __attribute__((amdgpu_waves_per
   float sl = 0.f, s_a = 0.f, sc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) sc[c] = 0.f;
-  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane, sl, s_a, sc);
+  fwd_tile_pixel<C, ODDS>(rec, gid, g0, g1, py0, px0, py - py0, px - px0, reinterpret_cast<float*>(s_batch[wid]), lane,
+                          sl, s_a, sc);
   if (nsplit > 1) {
     const int slot = AUTO ? item : P.pibase[ta.l] + item - P.ibase[ta.l];
     float* dst = part + (size_t)slot * split_part_floats<C, TILE>() + th;
@@ -1152,7 +1160,8 @@ __host__ __device__ constexpr int bg_stride(int C, int ntiles) { return (C * nti
 
 // Backward over the tiles [tb0, tb0 + ntiles) of the level table (levels without pairs are skipped).
 // Composite (level 0, or the images of a batch): upstream from T/asum/fg/gout (see pixel_upstream for UPS); per-tile
-// partials of sum_p gout * T go to bg_part[l bg_stride + c * ntiles + t] for tile t of level l. FIELDS: upstream from the packed fields.
+// partials of sum_p gout * T go to bg_part[l bg_stride + c * ntiles + t] for tile t of level l. FIELDS: upstream from the
+// packed fields.
 // S waves per tile (S = 1, or 16 with kFlagWide for few tiles with long pair lists: the dense coarse levels of
 // an octave render): the per-pixel upstream terms are staged in LDS once for the tile, then each wave takes a
 // contiguous share of the tile's pair list (every pair's sums are independent) 64 at a time (lane = pair) in
@@ -1199,8 +1208,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(5))) voi
     float2 pb = make_float2(0.f, 0.f);
     if (yp < ta.H && xp < ta.W) {
       const int p = (BATCH ? ta.pb : 0) + yp * ta.W + xp;
-      pixel_upstream<C, FIELDS, UPS>(p, (size_t)ta.pb + p, BATCH ? bg + ta.l * C : bg, Tin, asum_in, fg_in, gout, dslog, dsa, dsac,
-                                     pa, pb, bgp);
+      pixel_upstream<C, FIELDS, UPS>(p, (size_t)ta.pb + p, BATCH ? bg + ta.l * C : bg, Tin, asum_in, fg_in, gout,
+                                     dslog, dsa, dsac, pa, pb, bgp);
     }
     ups.put(l / TILE, l % TILE, pa, pb);
   }

@@ -525,26 +525,6 @@ def _wide(TILE, ntiles, pairs):
     return FLAG_WIDE if TILE == 8 and 0 < ntiles < 2048 and pairs >= 128 * ntiles else 0
 
 
-_SPLIT_PAIRS = 128   # pairs per workgroup the split launches of the coarse levels aim at
-_SPLIT_MAX = 64
-
-
-def _level_splits(bins, lt, mask):
-    """For splat_render_fields_split, which takes the numbers of chunks from its caller: chunks per tile of every level for the split FIELDS launches over the coarse levels (ctypes int array):
-    a level in `mask` gets about _SPLIT_PAIRS pairs per chunk on average over its tiles (1 to _SPLIT_MAX chunks),
-    so a dense coarse level's few tiles with long pair lists are spread over many workgroups; level 0 and levels
-    outside `mask` get 1 (unused)."""
-    geom, L = bins.geom, bins.n_levels
-    sp = (_lib.ctypes.c_int * L)()
-    for l in range(L):
-        sp[l] = 1
-        if l and (mask >> l) & 1:
-            tiles = (geom[l + 1][3] if l + 1 < L else bins.nt) - geom[l][3]
-            if tiles:
-                sp[l] = max(1, min(_SPLIT_MAX, -(-int(lt[l]) // (_SPLIT_PAIRS * tiles))))
-    return sp
-
-
 def _fields_buffers(npix, C, dev):
     """Packed level fields S_log [Pt], S_a [Pt], S_ac [Pt,C], views of one allocation."""
     slog, sa, sac = torch.empty(npix * (2 + C), device=dev).split_with_sizes((npix, npix, npix * C))
@@ -1298,7 +1278,8 @@ def _backward(grad_out, mu, scale, color, opacity, bg, py, px, theta, T, asum, f
     for b in range(B):
         r0 = recs[1 + b].data_ptr()
         check(lib.splat_exact_render_bwd(r0, r0 + 64 * N, N, C, ptr(pyf), ptr(pxf), P, grid_w, ptr(recs[0]),
-                                         _bptr(bgf, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b), _bptr(go, b), _bptr(lsc, b),
+                                         _bptr(bgf, b), _bptr(T, b), _bptr(asum, b), _bptr(fg, b), _bptr(go, b),
+                                         _bptr(lsc, b),
                                          _bptr(g_mu, b), _bptr(g_scale, b), _bptr(g_th, b), _bptr(g_op, b),
                                          _bptr(g_col, b), _bptr(g_bg, b), ptr(ws), ws.numel(), stream),
               "splat_exact_render_bwd")
@@ -1312,7 +1293,6 @@ class _AlphaRender(torch.autograd.Function):
     @staticmethod
     def forward(ctx, mu, scale, color, opacity, bg, theta, py, px, grid_w=0, scale_is_log=False):
         out, T, asum, fg, recs = _forward(mu, scale, color, opacity, bg, py, px, theta, grid_w, scale_is_log)
-        ctx.has_theta = theta is not None
         ctx.recs = recs
         ctx.opts = (grid_w, scale_is_log)
         ctx.save_for_backward(mu, scale, color, opacity, bg, theta, py, px, T, asum, fg)

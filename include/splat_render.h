@@ -215,6 +215,7 @@ int splat_render_bwd(const float *rec, const int *gid_sorted, const int *tile_st
  * the workspace (splat_fields_split_workspace_bytes; 0 when no level is split) and a second kernel adds them
  * in chunk order: deterministic, the same fields as splat_render_fwd with FIELDS up to summation order. The
  * backward's chunks write the per-pair sums as splat_render_bwd with FIELDS does. flags: SPLAT_FLAG_ODDS or 0.
+ * For callers that plan the chunks themselves; the Python renders take splat_render_fields_auto below.
  * Replace the per-octave-group launches of _render_fwd_cull_kernel / _render_bwd_cull_kernel over the coarse
  * groups, render_triton.py:962-978 (forward, per octave) and :768-810 (their backward). */
 size_t splat_fields_split_workspace_bytes(int C, int H, int W, int TILE, const splat_levels *lv, int lev_begin,

@@ -321,8 +321,8 @@ def test_octave_dense_coarse_level(dev, odds):
     H = W = 256
     scene = random_scene(2500, H, W, seed=31, dev=dev, ls_mean_px=24.0, ls_std=0.15, op_max=0.6)
     bins = run_levels(*scene, H, W, 8, octave_lv(), odds=odds, seed=11)
-    lt = bins.level_tot_b[0]
-    assert max(RH._level_splits(bins, lt, bins.level_mask(0) & ~1)) >= 4, "the scene must split a coarse level"
+    longest = bins.starts_b[0].diff()[bins.geom[1][3]:].max().item()
+    assert longest >= 4 * 64, "the scene must split a coarse tile (chunks of at most 64 pairs)"
 
 
 def test_octave_expecting_pairs_near_the_index_range(dev, monkeypatch):
