@@ -1268,6 +1268,7 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
   const int ntx = L.ntx[l];
   const int2 mine = rtot[r];   // units and pairs of the row
   const int cw = RC.cw[l], c0 = (wg - RC.wbase[l]) % RC.nch[l] * cw;
+  if (mine.x == 0 && c0 > 0) return;   // a row without units is left to its first chunk
   const int c1 = min(c0 + cw, ntx), ncol = c1 - c0;
   const int tile0 = L.tbase[l] + (r - L.rbase[l]) * ntx + c0;
   const int nt = L.tbase[L.n];
@@ -1281,7 +1282,7 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
   const int row_units = mine.x;
   const int tot = pair_count(info, cap);
   if (tot == 0) {   // no pairs (or a speculative launch past its capacity): the empty list
-    if (t < ncol) tile_starts[tile0 + t] = 0;
+    for (int j = t; j < (row_units == 0 ? ntx : ncol); j += kRowThreads) tile_starts[tile0 + j] = 0;
     if (r == 0 && c0 == 0 && t == 0) {
       tile_starts[nt] = 0;
       gid_sorted[0] = 0;
@@ -1306,6 +1307,10 @@ __global__ __launch_bounds__(kRowThreads) void k_expand_row(LevelTable L, const 
   for (int w = 0; w < kRowWaves; ++w) {
     us += s_red[0][w];
     pr += s_red[1][w];
+  }
+  if (row_units == 0) {
+    for (int j = t; j < ntx; j += kRowThreads) tile_starts[tile0 + j] = pr;
+    return;
   }
   // the row's units (at most one per pair: within the capacity the unit arrays are sized for)
   const int ue = min(us + row_units, cap);
@@ -1984,17 +1989,22 @@ int bin_pairs_launch(const int* rect, const int* offsets, const void* ws_count, 
     if (rc) return rc;
     // Level 0, and the images of a batch: chunks of at most kRowCols columns, about 8 per row of the widest level
     // (measured: 4 to 12 chunks, 256 to 1024 threads, 2 to 8 units per thread; this is the fastest at 768 x 768 and
-    // 2048 x 2048). Coarse levels hold few rows of long lists (27,000 pairs in a row of 12 tiles at 768 x 768): up to
-    // kCoarseChunks chunks per row. One workgroup per chunk and no more: taken as columns of a grid as wide as level 0's,
-    // the coarse rows' only chunks all fell on one XCD, and after level 0's (octave render at 768 x 768 with the encoder's
-    // splats: 59 us; spread 45 us, and the coarsest level first 32 us).
+    // 2048 x 2048). Coarse levels hold few rows of long lists (27,000 pairs in a row of 12 tiles at 768 x 768): as many
+    // chunks as make a workgroup per CU, up to kCoarseChunks per row, and no wider ones than level 0's. One workgroup per
+    // chunk and no more: taken as columns of a grid as wide as level 0's, the coarse rows' only chunks all fell on one XCD,
+    // and after level 0's (octave render at 768 x 768 with the encoder's splats: 59 us; spread 45 us, and the coarsest level
+    // first 32 us). 16 chunks for every coarse row took 33 us where the octaves past the first are empty (2048 x 2048, 20,000
+    // splats; 22 us so) and 33 against 26 us with the encoder's splats, whose octave 1 rows then had 4 columns for 8 waves.
     const bool batch = L.n > 1 && L.H[1] == L.H[0] && L.W[1] == L.W[0];
     RowChunks RC{};
+    const int cw0 = min(kRowCols, max(8, div_up(L.ntx[0], 8)));
     int cw = 1;
     for (int l = 0; l < L.n; ++l) {
-      RC.cw[l] = min(kRowCols, l == 0 || batch ? max(8, div_up(L.ntx[l], 8)) : div_up(L.ntx[l], kCoarseChunks));
+      const int rows = L.rbase[l + 1] - L.rbase[l];
+      const int spread = l == 0 || batch ? 1 : min(kCoarseChunks, max(1, 256 / rows));
+      RC.cw[l] = min(cw0, div_up(L.ntx[l], spread));
       RC.nch[l] = div_up(L.ntx[l], RC.cw[l]);
-      RC.wbase[l + 1] = RC.wbase[l] + RC.nch[l] * (L.rbase[l + 1] - L.rbase[l]);
+      RC.wbase[l + 1] = RC.wbase[l] + RC.nch[l] * rows;
       cw = max(cw, RC.cw[l]);
     }
     const int grid = RC.wbase[L.n];

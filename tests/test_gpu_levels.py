@@ -368,3 +368,42 @@ def test_levels_that_stay_empty_are_dropped(dev, monkeypatch):
             assert torch.equal(image(small), want[id(small)])
         assert masks[-1] == 1
         assert torch.equal(image(ls), want[id(ls)])
+
+
+@pytest.mark.parametrize("H,W,TILE,px,top,lv", [
+    (600, 5000, 8, 2.0, 0.1, octave_lv()), (600, 5000, 8, 30.0, 0.05, octave_lv()), (128, 4800, 8, 3.0, 1.0, split_lv(128, 4800, 5)),
+    (520, 520, 4, 20.0, 0.3, octave_lv()), (1024, 640, 16, 60.0, 0.2, octave_lv())])
+def test_rows_without_units(dev, H, W, TILE, px, top, lv):
+    """Splats in the top rows of their canvases only, levels without any, rows of more tiles than a workgroup has threads:
+    lists and tile starts of every level, for a first call, speculated ones and ones past the capacity."""
+    mu, ls, *_ = random_scene(3000, H, W, seed=9, dev=dev, ls_mean_px=px, ls_std=0.3)
+    mu[..., 0] *= top
+    more = ls + 1.5
+    for scales in (ls, ls, more, more, ls):
+        check_level_bins(mu, activate_scale(scales), H, W, TILE, lv)
+
+
+def test_empty_coarse_levels_take_no_longer_to_bin(dev):
+    """20,000 splats that all stay on octave 0 of 2048 x 2048, binned with the octave levels and on one canvas: the levels'
+    empty rows add less than three tenths (the least of ten measurements of 50 binnings queued back to back; 46 against 40 us)."""
+    H = W = 2048
+    mu, ls, col, op, _, th = random_scene(20000, H, W, seed=3, dev=dev, ls_mean_px=2.0, ls_std=0.2)
+    sc = activate_scale(ls)
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+
+    def us(lv):
+        run = lambda defer: RH._bin(mu, sc, col, op, th, H, W, 8, 3.0, lv=lv, defer=defer)   # noqa: E731
+        for _ in range(3):
+            run(False)
+        best = float("inf")
+        for _ in range(10):
+            a.record()
+            for _ in range(50):
+                run(True)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) / 50 * 1e3)
+        return best
+    single, levels = us(None), us(octave_lv())
+    print(f"one canvas {single:.1f} us, octave levels {levels:.1f} us", flush=True)
+    assert levels <= 1.3 * single
